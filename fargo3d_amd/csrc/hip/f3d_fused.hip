@@ -1,10 +1,12 @@
 // f3d_fused.hip -- the FP64 build of the fused step (entry points f3d_fused_*):
 // bit-for-bit the reference's arithmetic.  The kernels are in f3d_fused_body.h.
 #include <cstring>
+#include <algorithm>
 #include <type_traits>
 
 #include "f3d_internal.h"
 #include "f3d_cell.h"
+#include "f3d_ringsum.h"
 
 #define F3D_NS f3d
 #define F3D_PREC 64
@@ -86,7 +88,7 @@ extern "C" int f3d_fused_cfl_fluids_noalloc(f3d_hip_ctx* ctx, int nf, double* co
     T.ringmin[k] = sp + (size_t)k * nrings;
   }
   const int wg = (mode & 4) ? 64 : WG;
-  const size_t shmem = 16 * sizeof(double);
+  const size_t shmem = cfl_lds(pre);
   if (pre)
     FDISPATCH_T(ctx, kf_cfl_fluids, 1, dim3(nrings * nf), dim3(wg), shmem, T, nrings, vxm, ctx->f.VxMed, result, 0,
                 cfl_par_f(ctx));

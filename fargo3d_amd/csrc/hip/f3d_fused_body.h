@@ -227,53 +227,11 @@ __device__ __forceinline__ dim3 xcd_bid() {
 // The sequential sum in index order (the reduction order of
 // src/reduction_generic.c:18-20), in FP64, of a ring's weights
 // w_i = v_i (x_{i+1} - x_i) (src/compute_vmed.c:14-21), i in [0, n), by one
-// wave (all 64 lanes taking part) with the terms in registers.  The ring goes
-// in chunks of 64*S terms, lane L holding terms [c + L*S, c + (L+1)*S) of the
-// chunk at c.  The running sum
-// passes from lane to lane: every lane adds its own S terms to the sum so far
-// (one chain of dependent register additions), and lane L's result -- the
-// sequential sum through its last term -- is read out (v_readlane) as the
-// start of lane L+1's chain; the other lanes' results are discarded.  Terms
-// past the ring's end are +0.0, which leaves a sum started at +0.0 unchanged
-// (in round-to-nearest such a sum is never -0.0).  The next chunk's loads are
-// issued before the current chunk's chain.  Every lane returns the sum.
-// Measured on MI355X: a dependent FP64 addition in registers takes about
-// 4.5 ns, the same sum read from LDS about 12 ns per term.
-// The chain of wave_ring_sum over one chunk: lane L's S terms w follow the
-// terms of lanes 0 .. L-1, after acc; lanes 0 .. lanes-1 hold terms.
+// wave (f3d_ringsum.h); sh: LDS of its own, f3d_ring::lds_doubles(S) doubles.
+// Every lane returns the sum.
 template <int S>
-__device__ __forceinline__ double wave_chain(const double (&w)[S], double acc, int lanes) {
-#pragma clang fp contract(off)
-  for (int L = 0; L < lanes; L++) {
-    double t = acc;
-#pragma unroll
-    for (int s = 0; s < S; s++) t = t + w[s];
-    acc = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(t), L),
-                           __builtin_amdgcn_readlane(__double2loint(t), L));
-  }
-  return acc;
-}
-template <int S>
-__device__ __forceinline__ double wave_ring_sum(const real* __restrict__ v, const double* __restrict__ x, int n) {
-#pragma clang fp contract(off)
-  const int lane = (int)threadIdx.x & 63;
-  double a[S], x0[S + 1];
-  auto load = [&](int c) {
-#pragma unroll
-    for (int s = 0; s < S; s++) a[s] = (double)v[min(c + lane * S + s, n - 1)];
-#pragma unroll
-    for (int s = 0; s <= S; s++) x0[s] = x[min(c + lane * S + s, n)];
-  };
-  load(0);
-  double acc = 0.0;
-  for (int c = 0; c < n; c += 64 * S) {
-    double w[S];
-#pragma unroll
-    for (int s = 0; s < S; s++) w[s] = (c + lane * S + s < n) ? a[s] * (x0[s + 1] - x0[s]) : 0.0;
-    if (c + 64 * S < n) load(c + 64 * S);
-    acc = wave_chain<S>(w, acc, min(64, (n - c + S - 1) / S));
-  }
-  return acc;
+__device__ __forceinline__ double wave_ring_sum(const real* __restrict__ v, const dmesh& m, double* sh) {
+  return f3d_ring::ordered_sum<S, 1>(v, m.xmin64, f3d_ring::Straight(), m.nx, sh);
 }
 
 // VxMed of ring (j,k) from the ring mean of the stored velocity: the
@@ -295,9 +253,11 @@ __device__ __forceinline__ double vmed_full(double stored_mean, const dmesh& m, 
 // PRE: VxMed of the ring and the next from kf_vmed_rings; else summed here
 // (the in-kernel sum's registers would halve the occupancy of the PRE form,
 // hence a template parameter).
+constexpr int kCflSumLds = 16 + 2 * f3d_ring::lds_doubles(8);
+constexpr size_t cfl_lds(int pre) { return (pre ? 16 : kCflSumLds) * sizeof(double); }
 template <int G, int DZ, int PRE, int FX = 0>
 __device__ __forceinline__ void kd_cfl(int ring, const dmesh& m, const real* cs, const real* rho, const real* vx, const real* vy, const real* vz, const real* vxm, double* vxmed, unsigned long long* result, int slot, cell::CflPar cp, double* ringmin) {
-  extern __shared__ double lds[];  // 16
+  extern __shared__ double lds[];  // 16, and without PRE the two sums' staging
   double* sh = lds;
   const int j = m.nghy + ring % m.ny;
   const int k = DZ ? m.nghz + ring / m.ny : 0;
@@ -314,14 +274,14 @@ __device__ __forceinline__ void kd_cfl(int ring, const dmesh& m, const real* cs,
     // ComputeVweight + reduction_SUM (src/compute_vmed.c:14-30) of rings j and j+1
     // of vxm (the velocity whose VxMed the reference's cfl reads: with several
     // fluids, the last fluid's, src/main.c:366 then :381): the first wave sums
-    // ring j, the second ring j+1, each with its terms in registers
-    // (wave_ring_sum; this form runs with workgroups of four waves)
+    // ring j, the second ring j+1 (wave_ring_sum; this form runs with workgroups
+    // of four waves and kCflSumLds doubles of LDS)
     const int wv = (int)threadIdx.x >> 6;
     if (wv == 0) {
-      const double s0 = wave_ring_sum<4>(vxm + base, m.xmin64, m.nx);
+      const double s0 = wave_ring_sum<8>(vxm + base, m, lds + 16);
       if (threadIdx.x == 0) sh[8] = vmed_full(s0 / (m.XMAX - m.XMIN), m, j, k);
     } else if (wv == 1 && cp.fargo) {
-      const double s1 = wave_ring_sum<4>(vxm + base + m.pitch, m.xmin64, m.nx);
+      const double s1 = wave_ring_sum<8>(vxm + base + m.pitch, m, lds + 16 + f3d_ring::lds_doubles(8));
       if (threadIdx.x == 64) sh[9] = vmed_full(s1 / (m.XMAX - m.XMIN), m, j + 1, k);
     }
   }
@@ -370,7 +330,8 @@ __global__ void __launch_bounds__(64) kf_vmed_rings(dmesh m, const real* __restr
   const int j = m.nghy + (int)(blockIdx.x % nry);
   const int k = DZ ? m.nghz + (int)(blockIdx.x / nry) : 0;
   const int base = j * m.pitch + k * m.stride;
-  const double sum = wave_ring_sum<S>(v + base, m.xmin64, m.nx);
+  __shared__ double sh[f3d_ring::lds_doubles(S)];
+  const double sum = wave_ring_sum<S>(v + base, m, sh);
   if (threadIdx.x == 0) vxmed[j + k * m.sy] = vmed_full(sum / (m.XMAX - m.XMIN), m, j, k);
 }
 
@@ -1132,9 +1093,9 @@ __device__ __forceinline__ void xsweep_ring(const dmesh& m, int ring, double dt6
     vmed = vxmed_out[j + k * m.sy];
   } else {
     // ComputeVmed(Vx_temp) (src/compute_vmed.c:14-30), FP64, by the first
-    // wave with the terms in registers (wave_ring_sum)
+    // wave, staged through the start of the LDS (free until the barrier)
     if (t < 64) {
-      const double sum = wave_ring_sum<4>(vxt + base, m.xmin64, nx);
+      const double sum = wave_ring_sum<8>(vxt + base, m, lds_d);
       if (t == 0) sh[0] = vmed_full(sum / (m.XMAX - m.XMIN), m, j, k);
     }
     __syncthreads();
@@ -1429,7 +1390,7 @@ struct WRing {
 // neighbour read from a register or from the next lane.  Each quantity goes
 // through a pass on its own after the density's faces (which every update
 // reads), so only one quantity's stencil arrays are live at a time.  VxMed
-// is summed in the wave (wave_chain) from the velocities it holds.
+// is summed in the wave (f3d_ring::literal) from the velocities it holds.
 // TILE = 1: the wave holds a tile of a longer ring instead, the 64*CPT cells
 // from tile*(64*CPT - 2 kXHalo) - kXHalo on (indexes wrapped around the
 // ring), and updates the 64*CPT - 2 kXHalo cells inside the halos, the same
@@ -1486,11 +1447,11 @@ __device__ __forceinline__ void xsweep_wave(const dmesh& m, int ring, double dt6
       vmed = vxmed[j + k * m.sy];  // from kf_vmed
     } else {
       // ComputeVmed(Vx_temp) (src/compute_vmed.c:14-30): the ring's weights
-      // are in the lanes already, in the layout of wave_ring_sum's chunks
+      // are in the lanes already, consecutive ones in each
       double w[CPT];
 #pragma unroll
       for (int s = 0; s < CPT; s++) w[s] = vt[s] * (m.xmin64[ix[s] + 1] - m.xmin64[ix[s]]);
-      vmed = vmed_full(wave_chain<CPT>(w, 0.0, 64) / (m.XMAX - m.XMIN), m, j, k);
+      vmed = vmed_full(f3d_ring::literal<CPT>(w, 0.0, 0, 64) / (m.XMAX - m.XMIN), m, j, k);
     }
     const double vb = cell::vbase(m, j, k);
     double nr0 = 0.0;
@@ -1634,7 +1595,7 @@ __device__ __forceinline__ void xsweep_wave(const dmesh& m, int ring, double dt6
 // LDS bytes of xsweep_ring for n carried quantities + the density
 inline size_t xsweep_ring_lds(int nx, int ncarried) {
   const size_t P = ((size_t)(ncarried + 1) * nx + 1) & ~(size_t)1;
-  return (3 * P + nx) * sizeof(real) + 64;
+  return std::max((3 * P + nx) * sizeof(real) + 64, (f3d_ring::lds_doubles(8) + 8) * sizeof(double));
 }
 
 // ComputeVmed(Vx_temp) (src/compute_vmed.c:14-30) for the X sweeps: one wave
@@ -1649,7 +1610,8 @@ __device__ __forceinline__ void kd_vmed(const dim3 bid, const dmesh& m, const re
   const int j = m.nghy + (int)(bid.x % m.ny);
   const int k = DZ ? m.nghz + (int)(bid.x / m.ny) : 0;
   const int base = j * m.pitch + k * m.stride;
-  const double sum = wave_ring_sum<S>(vxt + base, m.xmin64, m.nx);
+  __shared__ double sh[f3d_ring::lds_doubles(S)];
+  const double sum = wave_ring_sum<S>(vxt + base, m, sh);
   if (threadIdx.x == 0) vxmed[j + k * m.sy] = vmed_full(sum / (m.XMAX - m.XMIN), m, j, k);
 }
 template <int G, int DZ, int S>
@@ -2573,20 +2535,14 @@ static int cfl_mode(const dmesh& m, int nf) {
 }
 
 // Terms per lane of the one-wave ring sums (wave_ring_sum): 4, 8 or 16; -1
-// automatic.  Measured on MI355X (whole FP64 step): 8 is fastest on rings of
-// 256 (3-D disk, 0.2503/0.2488/0.2546 ms for 4/8/16), 1024 (gas + 4 dust,
-// 0.4682/0.4573/0.4616 ms) and 4096 cells (adiabatic disk, 0.6811/0.6639/
-// 0.6756 ms), against 0.2515 and 0.680 ms with the sums read from LDS.
+// automatic: 16 from 2048 cells on (1024 rings of 4096 cells 11.6 us against
+// 13.6 with 8), else 8 (7150 rings of 500 cells 10.3 us against 13.7 with 16
+// and 11.9 with 4).
 static int g_vmed_terms = -1;
-static int vmed_terms(int nx) {
-  (void)nx;
-  return g_vmed_terms > 0 ? g_vmed_terms : 8;
-}
+static int vmed_terms(int nx) { return g_vmed_terms > 0 ? g_vmed_terms : nx >= 2048 ? 16 : 8; }
 
 // VxMed of every active ring and of the ring above the last (the shear limit
-// reads ring j+1), for the CFL kernel's pre-pass form: one wave per ring, four
-// for rings of 1024 cells or more (measured on MI355X: their loads, issued
-// by one wave, would take longer than the sum)
+// reads ring j+1), for the CFL kernel's pre-pass form: one wave per ring
 static int vmed_prepass_m(f3d_hip_ctx* ctx, const dmesh& m, const real* v) {
   const int nry = m.ny + (ctx->ph.fargo ? 1 : 0);
   const int nr = nry * (m.dimz ? m.nz : 1);
@@ -3113,7 +3069,7 @@ static int transport_fluids(f3d_hip_ctx* ctx, double dt, int nf, const f3d_field
   // the one-wave sweep sums VxMed itself; the tiled ones take it from the pass
   const int vpre = (ctx->ph.fargo && !wave) ? x_vmed_form(S->m, nf, tiles || wtiles) : 0;
   // 2-D: the pass in the Y sweep's launch instead of on the second stream
-  const bool vin = vpre == 1 && !S->m.dimz && g_y2v != 0 && vmed_terms(S->m.nx) == 8 &&
+  const bool vin = vpre == 1 && !S->m.dimz && g_y2v != 0 && (g_vmed_terms < 0 || g_vmed_terms == 8) &&
                    (size_t)S->m.nx * sizeof(double) <= 64 * 1024;
   VmTab VT;
   memset(&VT, 0, sizeof(VT));
@@ -3235,7 +3191,7 @@ int F3D_API(fused_cfl_vm)(f3d_hip_ctx* ctx, const double* vxm_in, double* fluid_
   if (pre && vmed_prepass(ctx, S, vxm ? vxm : f.Vx)) return -1;
   const int wg = (mode & 4) ? 64 : WG;
 #define CFL1(P_)                                                                                                 \
-  FDISPATCH_T(ctx, kf_cfl, P_, dim3(nrings), dim3(wg), 16 * sizeof(double), f.Energy, f.Density,            \
+  FDISPATCH_T(ctx, kf_cfl, P_, dim3(nrings), dim3(wg), cfl_lds(P_), f.Energy, f.Density,            \
               f.Vx, f.Vy, f.Vz, vxm ? vxm : f.Vx, f.VxMed, S->result, slot, cfl_par_f(ctx), rm)
   if (pre) CFL1(1);
   else CFL1(0);
@@ -3296,7 +3252,7 @@ int F3D_API(fused_cfl_fluids_async)(f3d_hip_ctx* ctx, int nf, double* const* cs,
   }
   const int wg = (mode & 4) ? 64 : WG;
 #define CFLF(P_)                                                                                             \
-  FDISPATCH_T(ctx, kf_cfl_fluids, P_, dim3(nrings * nf), dim3(wg), 16 * sizeof(double), T,                  \
+  FDISPATCH_T(ctx, kf_cfl_fluids, P_, dim3(nrings * nf), dim3(wg), cfl_lds(pre), T,                  \
               nrings, vxm, f.VxMed, S->result, slot, cfl_par_f(ctx))
   // the flag set of the common configurations at compile time (FARGO:
   // isothermal with constant nu or alpha, adiabatic with constant nu)

@@ -10,6 +10,7 @@
 // path live in f3d_fused.hip and reuse the per-cell arithmetic written here.
 #include "f3d_internal.h"
 #include "f3d_cell.h"
+#include "f3d_ringsum.h"
 #include "../host/f3d_host.h"
 
 using namespace f3d;
@@ -495,55 +496,102 @@ __global__ void k_cfl(dmesh m, Range r, const double* cs, const double* rho, con
 }
 
 // ---- reductions (src/reduction_generic.c:5-23, sequential i order per ring)
-__global__ void k_ring_sum(dmesh m, const double* f, double* red2d, int jb, int je, int kb, int ke, int is_min) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  int nj = je - jb;
-  if (t >= nj * (ke - kb)) return;
-  int j = jb + t % nj, k = kb + t / nj;
-  const double* row = f + (size_t)j * m.pitch + (size_t)k * m.stride;
-  double acc = is_min ? 1e20 : 0.0;
-  if (is_min) {
+// SUM: one wave per ring (f3d_ring::ordered_sum).  On the 384x128 disk's 134
+// rings one thread per ring took 41 us: two waves of uncoalesced dependent
+// loads and additions.
+__global__ void __launch_bounds__(64) k_ring_sum(dmesh m, const double* f, double* red2d, int jb, int je, int kb) {
+  const int nj = je - jb, j = jb + (int)blockIdx.x % nj, k = kb + (int)blockIdx.x / nj;
+  const double* __restrict__ row = f + (size_t)j * m.pitch + (size_t)k * m.stride;
+  __shared__ double sh[f3d_ring::lds_doubles(8)];
+  const double sum = f3d_ring::ordered_sum<8, 0>(row, row, f3d_ring::Straight(), m.nx, sh);
+  if (threadIdx.x == 0) red2d[j + k * m.sy] = sum;
+}
+// MIN of a ring by one wave.  The reference's running (acc < b) ? acc : b
+// starts again after a NaN and takes the later of two zeros of either sign;
+// where a NaN or a zero minimum makes the order matter, one lane walks the ring.
+__global__ void __launch_bounds__(64) k_ring_min(dmesh m, const double* f, double* red2d, int jb, int je, int kb) {
+  const int nj = je - jb, j = jb + (int)blockIdx.x % nj, k = kb + (int)blockIdx.x / nj;
+  const double* __restrict__ row = f + (size_t)j * m.pitch + (size_t)k * m.stride;
+  double acc = 1e20;
+  bool nan = false;
+  for (int i = threadIdx.x; i < m.nx; i += 64) {
+    const double b = row[i];
+    nan |= b != b;
+    acc = (acc < b) ? acc : b;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    const double b = __shfl_xor(acc, o, 64);
+    acc = (acc < b) ? acc : b;
+  }
+  if (__ballot(nan) || acc == 0.0) {
+    acc = 1e20;
     for (int i = 0; i < m.nx; i++) {
-      double b = row[i];
+      const double b = row[i];
       acc = (acc < b) ? acc : b;
     }
-  } else {
-    for (int i = 0; i < m.nx; i++) acc = acc + row[i];
   }
-  red2d[j + k * m.sy] = acc;
+  if (threadIdx.x == 0) red2d[j + k * m.sy] = acc;
 }
 
-// final (j,k) pass of reduction_full (src/reduction_full_generic.c:11-16), one thread
-__global__ void k_full_finish(dmesh m, const double* red2d, double* out, int jb, int je, int kb, int ke, int is_min) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  double result = is_min ? 1e20 : 0.0;
-  for (int k = kb; k < ke; k++)
-    for (int j = jb; j < je; j++) {
-      double a = red2d[j + k * m.sy];
-      result = is_min ? ((a < result) ? a : result) : a + result;
+// final (j,k) pass of reduction_full (src/reduction_full_generic.c:11-16), one
+// wave: the rings' sums in the reference's order, or their MIN, which skips
+// NaN and keeps the first of equal values (order matters for zeros alone)
+__global__ void __launch_bounds__(64) k_full_finish(dmesh m, const double* red2d, double* out, int jb, int je, int kb,
+                                                    int ke, int is_min) {
+  const int nj = je - jb, n = nj > 0 && ke > kb ? nj * (ke - kb) : 0;
+  __shared__ double sh[f3d_ring::lds_doubles(8)];
+  auto at = [&](int t) { return jb + t % nj + (kb + t / nj) * m.sy; };
+  double result;
+  if (is_min) {
+    result = 1e20;
+    for (int t = threadIdx.x; t < n; t += 64) {
+      const double a = red2d[at(t)];
+      result = (a < result) ? a : result;
     }
-  *out = result;
+    for (int o = 32; o > 0; o >>= 1) {
+      const double a = __shfl_xor(result, o, 64);
+      result = (a < result) ? a : result;
+    }
+    if (result == 0.0) {
+      result = 1e20;
+      for (int t = 0; t < n; t++) {
+        const double a = red2d[at(t)];
+        result = (a < result) ? a : result;
+      }
+    }
+  } else {
+    result = f3d_ring::ordered_sum<8, 0>(red2d, red2d, at, n, sh);
+  }
+  if (threadIdx.x == 0) *out = result;
 }
 
 // cfl_b shear limit (src/cfl_b.c:14-37) folded into the MIN of the per-ring minima
-__global__ void k_cfl_finish(dmesh m, const double* red2d, const double* vxmed, double* out, int fargo, double cfl) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  const int kb = m.dimz ? m.nghz : 0, ke = m.dimz ? m.nz + m.nghz : 1;
+// (one workgroup; every comparison skips NaN, and no minimum is a zero, so the
+// order does not matter; one thread took 33 us on 128 rings)
+__global__ void __launch_bounds__(256) k_cfl_finish(dmesh m, const double* red2d, const double* vxmed, double* out,
+                                                    int fargo, double cfl) {
+  __shared__ double sh[4];
+  const int kb = m.dimz ? m.nghz : 0, nk = m.dimz ? m.nz : 1;
   double result = 1e20;
-  for (int k = kb; k < ke; k++)
-    for (int j = m.nghy; j < m.ny + m.nghy; j++) {
-      double a = red2d[j + k * m.sy];
-      result = (a < result) ? a : result;
+  for (int t = threadIdx.x; t < m.ny * nk; t += 256) {
+    const int j = m.nghy + t % m.ny, l2 = j + (kb + t / m.ny) * m.sy;
+    const double a = red2d[l2];
+    result = (a < result) ? a : result;
+    if (fargo) {
+      const double shearlimit = cfl * m.mindx / fabs(vxmed[l2] / m.ymed[j] - vxmed[l2 + 1] / m.ymed[j + 1]);
+      if (shearlimit < result) result = shearlimit;
     }
-  if (fargo) {
-    for (int k = kb; k < ke; k++)
-      for (int j = m.nghy; j < m.ny + m.nghy; j++) {
-        int l2 = j + k * m.sy;
-        double shearlimit = cfl * m.mindx / fabs(vxmed[l2] / m.ymed[j] - vxmed[l2 + 1] / m.ymed[j + 1]);
-        if (shearlimit < result) result = shearlimit;
-      }
   }
-  *out = result;
+  for (int o = 32; o > 0; o >>= 1) {
+    const double a = __shfl_xor(result, o, 64);
+    result = (a < result) ? a : result;
+  }
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = result;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 4; w++) result = (sh[w] < result) ? sh[w] : result;
+    *out = result;
+  }
 }
 
 __global__ void k_vmed_div(dmesh m, const double* red2d, double* vxmed, int n2) {
@@ -1113,8 +1161,8 @@ int f3d_ComputeVweight(f3d_hip_ctx* ctx, const double* V, double* Q) {
 static int ring_reduce(f3d_hip_ctx* ctx, const double* F, double* red2d, int jb, int je, int kb, int ke, int is_min) {
   int n = (je - jb) * (ke - kb);
   if (n <= 0) return 0;
-  hipLaunchKernelGGL(k_ring_sum, dim3((n + 63) / 64), dim3(64), 0, ctx->stream, ctx->m, F, red2d, jb, je, kb, ke,
-                     is_min);
+  if (is_min) hipLaunchKernelGGL(k_ring_min, dim3(n), dim3(64), 0, ctx->stream, ctx->m, F, red2d, jb, je, kb);
+  else hipLaunchKernelGGL(k_ring_sum, dim3(n), dim3(64), 0, ctx->stream, ctx->m, F, red2d, jb, je, kb);
   F3D_LAUNCH_CHECK(ctx);
   return 0;
 }
@@ -1233,7 +1281,7 @@ int f3d_cfl(f3d_hip_ctx* ctx, double* fluid_min) {
            ctx->f.DensStar, cfl_par(ctx));
   int kb = m.dimz ? m.nghz : 0, ke = m.dimz ? m.nz + m.nghz : 1;
   if (ring_reduce(ctx, ctx->f.DensStar, ctx->f.Reduction2D, m.nghy, m.ny + m.nghy, kb, ke, 1)) return -1;
-  hipLaunchKernelGGL(k_cfl_finish, dim3(1), dim3(64), 0, ctx->stream, m, ctx->f.Reduction2D, ctx->f.VxMed, ctx->dred,
+  hipLaunchKernelGGL(k_cfl_finish, dim3(1), dim3(256), 0, ctx->stream, m, ctx->f.Reduction2D, ctx->f.VxMed, ctx->dred,
                      ctx->ph.fargo, ctx->ph.cfl);
   F3D_LAUNCH_CHECK(ctx);
   F3D_CHECK(ctx, hipMemcpyAsync(ctx->hres, ctx->dred, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
