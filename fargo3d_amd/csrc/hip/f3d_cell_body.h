@@ -82,7 +82,7 @@ __device__ __forceinline__ real substep1_x(const dmesh& m, int i, int j, int k, 
                                              LPOT pot, LV vx, int dust, int potential) {
   const int im = ixm_of(i, m.nx);
   real dxmed = real(0.5) * (m.sxi[i] + m.sxi[im]);
-  real dtOVERrhom = real(2.) * dt / (rho(0, 0, 0) * m.sxi[i] + rho(-1, 0, 0) * m.sxi[im]) * dxmed;
+  real dtOVERrhom = qdiv(real(2.) * dt, rho(0, 0, 0) * m.sxi[i] + rho(-1, 0, 0) * m.sxi[im]) * dxmed;
   real v = vx(0, 0, 0);
   const real izs = inv_zone_size_xmed<G>(m, i, j, k);
   if (!dust) v -= dtOVERrhom * (p(0, 0, 0) - p(-1, 0, 0)) * izs;
@@ -95,10 +95,10 @@ template <int G, int DZ, class LR, class LP, class LPOT, class LVX, class LVY, c
 __device__ __forceinline__ real substep1_y(const dmesh& m, int i, int j, int k, real dt, LR rho, LP p,
                                              LPOT pot, LVX vx, LVY vy, LVZ vz, int dust, int potential,
                                              double omegaframe) {
-  real dtOVERrhom = real(2.0) * dt / (rho(0, 0, 0) * (m.ymin[j + 1] - m.ymin[j]) + rho(0, -1, 0) * (m.ymin[j] - m.ymin[j - 1])) *
+  real dtOVERrhom = qdiv(real(2.0) * dt, rho(0, 0, 0) * (m.ymin[j + 1] - m.ymin[j]) + rho(0, -1, 0) * (m.ymin[j] - m.ymin[j - 1])) *
                       (m.ymed[j] - m.ymed[j - 1]);
   real v = vy(0, 0, 0);
-  if (!dust) v -= dtOVERrhom * (p(0, 0, 0) - p(0, -1, 0)) / (m.ymed[j] - m.ymed[j - 1]);
+  if (!dust) v -= qdiv(dtOVERrhom * (p(0, 0, 0) - p(0, -1, 0)), m.ymed[j] - m.ymed[j - 1]);
   if constexpr (kFix64) {
     double vphi = 0.25 * ((double)vx(0, 0, 0) + (double)vx(1, 0, 0) + (double)vx(0, -1, 0) + (double)vx(1, -1, 0)) +
                   0.5 * (vbase(m, j, k) + vbase(m, j - 1, k));
@@ -108,24 +108,24 @@ __device__ __forceinline__ real substep1_y(const dmesh& m, int i, int j, int k, 
       const double vzz = DZ ? 0.25 * ((double)vz(0, 0, 0) + (double)vz(0, 0, 1) + (double)vz(0, -1, 0) +
                                       (double)vz(0, -1, 1))
                             : 0.0;
-      acc = (vphi * vphi + vzz * vzz) / m.ymin64[j];
+      acc = qdivd(vphi * vphi + vzz * vzz, m.ymin64[j]);
     } else {
       vphi += m.ymin64[j] * (double)omegaframe;
-      acc = vphi * vphi / m.ymin64[j];
+      acc = qdivd(vphi * vphi, m.ymin64[j]);
     }
-    if (potential) acc -= ((double)pot(0, 0, 0) - (double)pot(0, -1, 0)) / (m.ymed64[j] - m.ymed64[j - 1]);
+    if (potential) acc -= qdivd((double)pot(0, 0, 0) - (double)pot(0, -1, 0), m.ymed64[j] - m.ymed64[j - 1]);
     return v + (real)(acc * (double)dt);
   } else {
     real vphi = real(.25) * (vx(0, 0, 0) + vx(1, 0, 0) + vx(0, -1, 0) + vx(1, -1, 0));
     if (G == SPH) {
       vphi += m.ymin[j] * m.sinzmed[k] * omegaframe;
       real vzz = DZ ? real(.25) * (vz(0, 0, 0) + vz(0, 0, 1) + vz(0, -1, 0) + vz(0, -1, 1)) : real(0.0);
-      v += (vphi * vphi + vzz * vzz) / m.ymin[j] * dt;
+      v += qdiv(vphi * vphi + vzz * vzz, m.ymin[j]) * dt;
     } else {
       vphi += m.ymin[j] * omegaframe;
-      v += vphi * vphi / m.ymin[j] * dt;
+      v += qdiv(vphi * vphi, m.ymin[j]) * dt;
     }
-    if (potential) v -= (pot(0, 0, 0) - pot(0, -1, 0)) * dt / (m.ymed[j] - m.ymed[j - 1]);
+    if (potential) v -= qdiv((pot(0, 0, 0) - pot(0, -1, 0)) * dt, m.ymed[j] - m.ymed[j - 1]);
     return v;
   }
 }
@@ -135,7 +135,7 @@ template <int G, class LR, class LP, class LPOT, class LVX, class LVZ>
 __device__ __forceinline__ real substep1_z(const dmesh& m, int i, int j, int k, real dt, LR rho, LP p,
                                              LPOT pot, LVX vx, LVZ vz, int dust, int potential,
                                              double omegaframe) {
-  real dtOVERrhom = real(2.0) * dt / (rho(0, 0, 0) * (m.zmin[k + 1] - m.zmin[k]) + rho(0, 0, -1) * (m.zmin[k] - m.zmin[k - 1])) *
+  real dtOVERrhom = qdiv(real(2.0) * dt, rho(0, 0, 0) * (m.zmin[k + 1] - m.zmin[k]) + rho(0, 0, -1) * (m.zmin[k] - m.zmin[k - 1])) *
                       (m.zmed[k] - m.zmed[k - 1]);
   real v;
   if (G == SPH && kFix64) {
@@ -144,21 +144,21 @@ __device__ __forceinline__ real substep1_z(const dmesh& m, int i, int j, int k, 
     const double smin = m.sinzmin64[k], r = m.ymed64[j];
     vphi += r * smin * (double)omegaframe;
     v = vz(0, 0, 0);
-    if (!dust) v -= dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)) / (m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
-    double acc = vphi * vphi * m.coszmin64[k] / (smin * r);
-    if (potential) acc -= ((double)pot(0, 0, 0) - (double)pot(0, 0, -1)) / (r * (m.zmed64[k] - m.zmed64[k - 1]));
+    if (!dust) v -= qdiv(dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)), m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
+    double acc = qdivd(vphi * vphi * m.coszmin64[k], smin * r);
+    if (potential) acc -= qdivd((double)pot(0, 0, 0) - (double)pot(0, 0, -1), r * (m.zmed64[k] - m.zmed64[k - 1]));
     v += (real)(acc * (double)dt);
   } else if (G == SPH) {
     real vphi = real(.25) * (vx(0, 0, 0) + vx(1, 0, 0) + vx(0, 0, -1) + vx(1, 0, -1));
     vphi += m.ymed[j] * m.sinzmin[k] * omegaframe;
     v = vz(0, 0, 0);
-    if (!dust) v -= dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)) / (m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
-    v += vphi * vphi * m.coszmin[k] / (m.sinzmin[k] * m.ymed[j]) * dt;
-    if (potential) v -= (pot(0, 0, 0) - pot(0, 0, -1)) * dt / (m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
+    if (!dust) v -= qdiv(dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)), m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
+    v += qdiv(vphi * vphi * m.coszmin[k], m.sinzmin[k] * m.ymed[j]) * dt;
+    if (potential) v -= qdiv((pot(0, 0, 0) - pot(0, 0, -1)) * dt, m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
   } else {
     v = vz(0, 0, 0);
-    if (!dust) v -= dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)) / (m.zmed[k] - m.zmed[k - 1]);
-    if (potential) v -= (pot(0, 0, 0) - pot(0, 0, -1)) * dt / (m.zmed[k] - m.zmed[k - 1]);
+    if (!dust) v -= qdiv(dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)), m.zmed[k] - m.zmed[k - 1]);
+    if (potential) v -= qdiv((pot(0, 0, 0) - pot(0, 0, -1)) * dt, m.zmed[k] - m.zmed[k - 1]);
   }
   return v;
 }
@@ -180,23 +180,23 @@ __device__ __forceinline__ void substep2_b(const dmesh& m, int i, int j, int k, 
   real dxrho1 = m.sxi[i];
   real dxrho2 = m.sxi[im];
   real dxmed = real(0.5) * (m.sxi[i] + m.sxi[im]);
-  vxt += -real(2.0) * dt * dxmed * (px(0, 0, 0) - px(-1, 0, 0)) / (rho(0, 0, 0) * dxrho1 + rho(-1, 0, 0) * dxrho2) *
+  vxt += qdiv(-real(2.0) * dt * dxmed * (px(0, 0, 0) - px(-1, 0, 0)), rho(0, 0, 0) * dxrho1 + rho(-1, 0, 0) * dxrho2) *
          inv_zone_size_xmed<G>(m, i, j, k);
-  if (adiabatic) e += -dt * (px(0, 0, 0) * (vx(1, 0, 0) - vx(0, 0, 0)) / zone_size_x<G>(m, i, j, k));
+  if (adiabatic) e += -dt * qdiv(px(0, 0, 0) * (vx(1, 0, 0) - vx(0, 0, 0)), zone_size_x<G>(m, i, j, k));
   real dyrho1 = m.ymin[j + 1] - m.ymin[j];
   real dyrho2 = m.ymin[j] - m.ymin[j - 1];
-  vyt += -real(2.0) * (py(0, 0, 0) - py(0, -1, 0)) / (rho(0, 0, 0) * dyrho1 + rho(0, -1, 0) * dyrho2) * dt;
-  if (adiabatic) e += -dt * (py(0, 0, 0) * (vy(0, 1, 0) - vy(0, 0, 0)) / zone_size_y(m, j));
+  vyt += qdiv(-real(2.0) * (py(0, 0, 0) - py(0, -1, 0)), rho(0, 0, 0) * dyrho1 + rho(0, -1, 0) * dyrho2) * dt;
+  if (adiabatic) e += -dt * qdiv(py(0, 0, 0) * (vy(0, 1, 0) - vy(0, 0, 0)), zone_size_y(m, j));
   if (DZ) {
     real dzmed = m.zmed[k] - m.zmed[k - 1];
     real dzrho1 = m.zmin[k + 1] - m.zmin[k];
     real dzrho2 = m.zmin[k] - m.zmin[k - 1];
     if (G == SPH)
-      vzt += -real(2.0) * dzmed * (pz(0, 0, 0) - pz(0, 0, -1)) / (rho(0, 0, 0) * dzrho1 + rho(0, 0, -1) * dzrho2) * dt /
-             (m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
+      vzt += qdiv(qdiv(-real(2.0) * dzmed * (pz(0, 0, 0) - pz(0, 0, -1)), rho(0, 0, 0) * dzrho1 + rho(0, 0, -1) * dzrho2) * dt,
+                  m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
     else
-      vzt += -real(2.0) * (pz(0, 0, 0) - pz(0, 0, -1)) / (rho(0, 0, 0) * dzrho1 + rho(0, 0, -1) * dzrho2) * dt;
-    if (adiabatic) e += -dt * (pz(0, 0, 0) * (vz(0, 0, 1) - vz(0, 0, 0)) / zone_size_z<G>(m, j, k));
+      vzt += qdiv(-real(2.0) * (pz(0, 0, 0) - pz(0, 0, -1)), rho(0, 0, 0) * dzrho1 + rho(0, 0, -1) * dzrho2) * dt;
+    if (adiabatic) e += -dt * qdiv(pz(0, 0, 0) * (vz(0, 0, 1) - vz(0, 0, 0)), zone_size_z<G>(m, j, k));
   }
   oxt = vxt;
   oyt = vyt;
@@ -225,10 +225,10 @@ __device__ __forceinline__ real substep3(const dmesh& m, int i, int j, int k, re
     // In FP32 the rounding of 1 - t is the same for every cell of a ring
     // with the same t and would heat or cool the ring by a fixed amount
     // each step; here it is relative to the change only.
-    e -= e * (real(2.0) * term / (real(1.0) + term));
+    e -= e * qdiv(real(2.0) * term, real(1.0) + term);
     return e;
   }
-  e *= (real(1.0) - term) / (real(1.0) + term);
+  e *= qdiv(real(1.0) - term, real(1.0) + term);
   return e;
 }
 
@@ -264,14 +264,14 @@ __device__ __forceinline__ Taus visctensor(const dmesh& m, int i, int j, int k, 
       }
     } else {
       const real gg = vp.alpha * vp.gamma * (vp.gamma - real(1.0));
-      visc = gg * energy(0, 0, 0) / rho(0, 0, 0) * sq_med;
-      viscm = gg * (energy(0, 0, 0) + energy(-1, 0, 0) + energy(0, -1, 0) + energy(-1, -1, 0)) /
-              (rho(0, 0, 0) + rho(-1, 0, 0) + rho(0, -1, 0) + rho(-1, -1, 0)) * sq_min;
+      visc = qdiv(gg * energy(0, 0, 0), rho(0, 0, 0)) * sq_med;
+      viscm = qdiv(gg * (energy(0, 0, 0) + energy(-1, 0, 0) + energy(0, -1, 0) + energy(-1, -1, 0)),
+                   rho(0, 0, 0) + rho(-1, 0, 0) + rho(0, -1, 0) + rho(-1, -1, 0)) * sq_min;
       if (DZ) {
-        visczm = gg * (energy(0, 0, 0) + energy(0, 0, -1) + energy(-1, 0, 0) + energy(-1, 0, -1)) /
-                 (rho(0, 0, 0) + rho(0, 0, -1) + rho(-1, 0, 0) + rho(-1, 0, -1)) * sq_med;
-        visczmym = gg * (energy(0, 0, 0) + energy(0, -1, 0) + energy(0, 0, -1) + energy(0, -1, -1)) /
-                   (rho(0, 0, 0) + rho(0, -1, 0) + rho(0, 0, -1) + rho(0, -1, -1)) * sq_min;
+        visczm = qdiv(gg * (energy(0, 0, 0) + energy(0, 0, -1) + energy(-1, 0, 0) + energy(-1, 0, -1)),
+                      rho(0, 0, 0) + rho(0, 0, -1) + rho(-1, 0, 0) + rho(-1, 0, -1)) * sq_med;
+        visczmym = qdiv(gg * (energy(0, 0, 0) + energy(0, -1, 0) + energy(0, 0, -1) + energy(0, -1, -1)),
+                        rho(0, 0, 0) + rho(0, -1, 0) + rho(0, 0, -1) + rho(0, -1, -1)) * sq_min;
       }
     }
   } else {
@@ -281,43 +281,43 @@ __device__ __forceinline__ Taus visctensor(const dmesh& m, int i, int j, int k, 
   dv *= mul_invvol(m, real(2.0) / real(3.0), i, j, k);
   const real r0 = rho(0, 0, 0);
   Taus t;
-  t.xx = visc * r0 * (real(2.0) * (vx(1, 0, 0) - vx(0, 0, 0)) / zone_size_x<G>(m, i, j, k) - dv);
-  t.xx += visc * r0 * (vy(0, 1, 0) + vy(0, 0, 0)) / m.ymed[j];
-  if (G == SPH && DZ) t.xx += visc * r0 * (vz(0, 0, 1) + vz(0, 0, 0)) * m.coszmed[k] / (m.sinzmed[k] * m.ymed[j]);
-  t.yy = visc * r0 * (real(2.0) * (vy(0, 1, 0) - vy(0, 0, 0)) / (m.ymin[j + 1] - m.ymin[j]) - dv);
+  t.xx = visc * r0 * (qdiv(real(2.0) * (vx(1, 0, 0) - vx(0, 0, 0)), zone_size_x<G>(m, i, j, k)) - dv);
+  t.xx += qdiv(visc * r0 * (vy(0, 1, 0) + vy(0, 0, 0)), m.ymed[j]);
+  if (G == SPH && DZ) t.xx += qdiv(visc * r0 * (vz(0, 0, 1) + vz(0, 0, 0)) * m.coszmed[k], m.sinzmed[k] * m.ymed[j]);
+  t.yy = visc * r0 * (qdiv(real(2.0) * (vy(0, 1, 0) - vy(0, 0, 0)), m.ymin[j + 1] - m.ymin[j]) - dv);
   t.zz = t.xz = t.zy = real(0.0);
   if (DZ) {
     if (G == SPH) {
-      t.zz = visc * r0 * (real(2.0) * (vz(0, 0, 1) - vz(0, 0, 0)) / (m.ymed[j] * (m.zmin[k + 1] - m.zmin[k])) - dv);
-      t.zz += visc * r0 * (vy(0, 0, 0) + vy(0, 1, 0)) / m.ymed[j];
+      t.zz = visc * r0 * (qdiv(real(2.0) * (vz(0, 0, 1) - vz(0, 0, 0)), m.ymed[j] * (m.zmin[k + 1] - m.zmin[k])) - dv);
+      t.zz += qdiv(visc * r0 * (vy(0, 0, 0) + vy(0, 1, 0)), m.ymed[j]);
       t.xz = visczm * real(.25) * (r0 + rho(0, 0, -1) + rho(-1, 0, 0) + rho(-1, 0, -1)) *
-             ((vx(0, 0, 0) / m.sinzmed[k] - vx(0, 0, -1) / m.sinzmed[k - 1]) * m.sinzmin[k] /
-                  (m.ymed[j] * (m.zmed[k] - m.zmed[k - 1])) +
-              ((vz(0, 0, 0) - vz(-1, 0, 0)) * m.invdiffxmed[i] / (m.sinzmin[k] * m.ymed[j])));
+             (qdiv((qdiv(vx(0, 0, 0), m.sinzmed[k]) - qdiv(vx(0, 0, -1), m.sinzmed[k - 1])) * m.sinzmin[k],
+                   m.ymed[j] * (m.zmed[k] - m.zmed[k - 1])) +
+              qdiv((vz(0, 0, 0) - vz(-1, 0, 0)) * m.invdiffxmed[i], m.sinzmin[k] * m.ymed[j]));
     } else {
-      t.zz = visc * r0 * (real(2.0) * (vz(0, 0, 1) - vz(0, 0, 0)) / (m.zmin[k + 1] - m.zmin[k]) - dv);
+      t.zz = visc * r0 * (qdiv(real(2.0) * (vz(0, 0, 1) - vz(0, 0, 0)), m.zmin[k + 1] - m.zmin[k]) - dv);
       t.xz = visczm * real(.25) * (r0 + rho(0, 0, -1) + rho(-1, 0, 0) + rho(-1, 0, -1)) *
-             ((vx(0, 0, 0) - vx(0, 0, -1)) / (m.zmed[k] - m.zmed[k - 1]) +
-              (vz(0, 0, 0) - vz(-1, 0, 0)) * m.invdiffxmed[i] / m.ymed[j]);
+             (qdiv(vx(0, 0, 0) - vx(0, 0, -1), m.zmed[k] - m.zmed[k - 1]) +
+              qdiv((vz(0, 0, 0) - vz(-1, 0, 0)) * m.invdiffxmed[i], m.ymed[j]));
     }
   }
   if (G == SPH)
     t.yx = viscm * real(.25) * (r0 + rho(-1, 0, 0) + rho(0, -1, 0) + rho(-1, -1, 0)) *
-           ((vy(0, 0, 0) - vy(-1, 0, 0)) * m.invdiffxmed[i] / (m.ymin[j] * m.sinzmed[k]) +
-            (vx(0, 0, 0) - vx(0, -1, 0)) / (m.ymed[j] - m.ymed[j - 1]) - real(.5) * (vx(0, 0, 0) + vx(0, -1, 0)) / m.ymin[j]);
+           (qdiv((vy(0, 0, 0) - vy(-1, 0, 0)) * m.invdiffxmed[i], m.ymin[j] * m.sinzmed[k]) +
+            qdiv(vx(0, 0, 0) - vx(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) - qdiv(real(.5) * (vx(0, 0, 0) + vx(0, -1, 0)), m.ymin[j]));
   else
     t.yx = viscm * real(.25) * (r0 + rho(-1, 0, 0) + rho(0, -1, 0) + rho(-1, -1, 0)) *
-           ((vy(0, 0, 0) - vy(-1, 0, 0)) * m.invdiffxmed[i] / m.ymin[j] +
-            (vx(0, 0, 0) - vx(0, -1, 0)) / (m.ymed[j] - m.ymed[j - 1]) - real(.5) * (vx(0, 0, 0) + vx(0, -1, 0)) / m.ymin[j]);
+           (qdiv((vy(0, 0, 0) - vy(-1, 0, 0)) * m.invdiffxmed[i], m.ymin[j]) +
+            qdiv(vx(0, 0, 0) - vx(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) - qdiv(real(.5) * (vx(0, 0, 0) + vx(0, -1, 0)), m.ymin[j]));
   if (DZ) {
     if (G == SPH)
       t.zy = visczmym * real(.25) * (r0 + rho(0, -1, 0) + rho(0, 0, -1) + rho(0, -1, -1)) *
-             ((vz(0, 0, 0) - vz(0, -1, 0)) / (m.ymed[j] - m.ymed[j - 1]) - real(.5) * (vz(0, 0, 0) + vz(0, -1, 0)) / m.ymin[j] +
-              (vy(0, 0, 0) - vy(0, 0, -1)) / (m.ymin[j] * (m.zmed[k] - m.zmed[k - 1])));
+             (qdiv(vz(0, 0, 0) - vz(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) - qdiv(real(.5) * (vz(0, 0, 0) + vz(0, -1, 0)), m.ymin[j]) +
+              qdiv(vy(0, 0, 0) - vy(0, 0, -1), m.ymin[j] * (m.zmed[k] - m.zmed[k - 1])));
     else
       t.zy = visczmym * real(.25) * (r0 + rho(0, -1, 0) + rho(0, 0, -1) + rho(0, -1, -1)) *
-             ((vz(0, 0, 0) - vz(0, -1, 0)) / (m.ymed[j] - m.ymed[j - 1]) +
-              (vy(0, 0, 0) - vy(0, 0, -1)) / (m.zmed[k] - m.zmed[k - 1]));
+             (qdiv(vz(0, 0, 0) - vz(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) +
+              qdiv(vy(0, 0, 0) - vy(0, 0, -1), m.zmed[k] - m.zmed[k - 1]));
   }
   return t;
 }
@@ -329,40 +329,41 @@ __device__ __forceinline__ void addviscosity(const dmesh& m, int i, int j, int k
                                              real vz, real& ox, real& oy, real& oz) {
   const real r0 = rho(0, 0, 0), rxm = rho(-1, 0, 0), rym = rho(0, -1, 0);
   const real ymn = m.ymin[j], ymp = m.ymin[j + 1], yd = m.ymed[j], ydm = m.ymed[j - 1];
-  vx += real(2.0) * (txx(0, 0, 0) - txx(-1, 0, 0)) * inv_zone_size_xmed<G>(m, i, j, k) / ((r0 + rxm)) * dt;
-  vx += real(2.0) * (ymp * ymp * tyx(0, 1, 0) - ymn * ymn * tyx(0, 0, 0)) / ((ymp - ymn) * yd * yd * (rxm + r0)) * dt;
+  vx += qdiv(real(2.0) * (txx(0, 0, 0) - txx(-1, 0, 0)) * inv_zone_size_xmed<G>(m, i, j, k), r0 + rxm) * dt;
+  vx += qdiv(real(2.0) * (ymp * ymp * tyx(0, 1, 0) - ymn * ymn * tyx(0, 0, 0)), (ymp - ymn) * yd * yd * (rxm + r0)) * dt;
   if (G == SPH) {
-    vx += (tyx(0, 1, 0) + tyx(0, 0, 0)) / ((rxm + r0) * yd) * dt;
+    vx += qdiv(tyx(0, 1, 0) + tyx(0, 0, 0), (rxm + r0) * yd) * dt;
     if (DZ) {
-      vx += real(2.0) * (txz(0, 0, 1) - txz(0, 0, 0)) / (zone_size_z<G>(m, j, k) * (rxm + r0)) * dt;
-      vx += real(2.0) * (txz(0, 0, 1) + txz(0, 0, 0)) * m.coszmed[k] / (m.sinzmed[k] * yd * (rxm + r0)) * dt;
+      vx += qdiv(real(2.0) * (txz(0, 0, 1) - txz(0, 0, 0)), zone_size_z<G>(m, j, k) * (rxm + r0)) * dt;
+      vx += qdiv(real(2.0) * (txz(0, 0, 1) + txz(0, 0, 0)) * m.coszmed[k], m.sinzmed[k] * yd * (rxm + r0)) * dt;
     }
-    vy += real(2.0) * (yd * yd * tyy(0, 0, 0) - ydm * ydm * tyy(0, -1, 0)) / ((yd - ydm) * (r0 + rym) * ymn * ymn) * dt;
-    vy += real(2.0) * (tyx(1, 0, 0) - tyx(0, 0, 0)) / ((m.xmin[i + 1] - m.xmin[i]) * ymn * m.sinzmed[k] * (r0 + rym)) * dt;
-    vy -= (txx(0, 0, 0) + txx(0, -1, 0)) / (ymn * (r0 + rym)) * dt;
+    vy += qdiv(real(2.0) * (yd * yd * tyy(0, 0, 0) - ydm * ydm * tyy(0, -1, 0)), (yd - ydm) * (r0 + rym) * ymn * ymn) * dt;
+    vy += qdiv(real(2.0) * (tyx(1, 0, 0) - tyx(0, 0, 0)),
+               (m.xmin[i + 1] - m.xmin[i]) * ymn * m.sinzmed[k] * (r0 + rym)) * dt;
+    vy -= qdiv(txx(0, 0, 0) + txx(0, -1, 0), ymn * (r0 + rym)) * dt;
     if (DZ) {
       const real rzm = rho(0, 0, -1);
-      vy -= (tzz(0, 0, 0) + tzz(0, -1, 0)) / (ymn * (r0 + rym)) * dt;
-      vy += real(2.0) * (tzy(0, 0, 1) * m.sinzmin[k + 1] - tzy(0, 0, 0) * m.sinzmin[k]) /
-            ((m.zmin[k + 1] - m.zmin[k]) * ymn * m.sinzmed[k] * (r0 + rym)) * dt;
-      vz += real(2.0) * (tzz(0, 0, 0) * m.sinzmed[k] - tzz(0, 0, -1) * m.sinzmed[k - 1]) /
-            ((m.zmed[k] - m.zmed[k - 1]) * yd * m.sinzmin[k] * (r0 + rzm)) * dt;
-      vz += real(2.0) * (txz(1, 0, 0) - txz(0, 0, 0)) / ((m.sxi[i] * yd * m.sinzmin[k]) * (r0 + rzm)) * dt;
-      vz += real(2.0) * (ymp * ymp * ymp * tzy(0, 1, 0) - ymn * ymn * ymn * tzy(0, 0, 0)) /
-            ((ymp - ymn) * yd * yd * yd * (r0 + rzm)) * dt;
-      vz -= (txx(0, 0, 0) + txx(0, 0, -1)) * m.coszmin[k] / (yd * m.sinzmin[k] * (r0 + rzm)) * dt;
+      vy -= qdiv(tzz(0, 0, 0) + tzz(0, -1, 0), ymn * (r0 + rym)) * dt;
+      vy += qdiv(real(2.0) * (tzy(0, 0, 1) * m.sinzmin[k + 1] - tzy(0, 0, 0) * m.sinzmin[k]),
+                 (m.zmin[k + 1] - m.zmin[k]) * ymn * m.sinzmed[k] * (r0 + rym)) * dt;
+      vz += qdiv(real(2.0) * (tzz(0, 0, 0) * m.sinzmed[k] - tzz(0, 0, -1) * m.sinzmed[k - 1]),
+                 (m.zmed[k] - m.zmed[k - 1]) * yd * m.sinzmin[k] * (r0 + rzm)) * dt;
+      vz += qdiv(real(2.0) * (txz(1, 0, 0) - txz(0, 0, 0)), (m.sxi[i] * yd * m.sinzmin[k]) * (r0 + rzm)) * dt;
+      vz += qdiv(real(2.0) * (ymp * ymp * ymp * tzy(0, 1, 0) - ymn * ymn * ymn * tzy(0, 0, 0)),
+                 (ymp - ymn) * yd * yd * yd * (r0 + rzm)) * dt;
+      vz -= qdiv((txx(0, 0, 0) + txx(0, 0, -1)) * m.coszmin[k], yd * m.sinzmin[k] * (r0 + rzm)) * dt;
     }
   } else {
-    if (DZ) vx += real(2.0) * (txz(0, 0, 1) - txz(0, 0, 0)) / ((m.zmin[k + 1] - m.zmin[k]) * (rxm + r0)) * dt;
-    vy += real(2.0) * (yd * tyy(0, 0, 0) - ydm * tyy(0, -1, 0)) / ((yd - ydm) * (r0 + rym) * ymn) * dt;
-    vy += real(2.0) * (tyx(1, 0, 0) - tyx(0, 0, 0)) / ((m.xmin[i + 1] - m.xmin[i]) * ymn * (r0 + rym)) * dt;
-    vy -= (txx(0, 0, 0) + txx(0, -1, 0)) / (ymn * (r0 + rym)) * dt;
+    if (DZ) vx += qdiv(real(2.0) * (txz(0, 0, 1) - txz(0, 0, 0)), (m.zmin[k + 1] - m.zmin[k]) * (rxm + r0)) * dt;
+    vy += qdiv(real(2.0) * (yd * tyy(0, 0, 0) - ydm * tyy(0, -1, 0)), (yd - ydm) * (r0 + rym) * ymn) * dt;
+    vy += qdiv(real(2.0) * (tyx(1, 0, 0) - tyx(0, 0, 0)), (m.xmin[i + 1] - m.xmin[i]) * ymn * (r0 + rym)) * dt;
+    vy -= qdiv(txx(0, 0, 0) + txx(0, -1, 0), ymn * (r0 + rym)) * dt;
     if (DZ) {
       const real rzm = rho(0, 0, -1);
-      vy += real(2.0) * (tzy(0, 0, 1) - tzy(0, 0, 0)) / ((m.zmin[k + 1] - m.zmin[k]) * (r0 + rym)) * dt;
-      vz += real(2.0) * (tzz(0, 0, 0) - tzz(0, 0, -1)) / ((m.zmed[k] - m.zmed[k - 1]) * (r0 + rzm)) * dt;
-      vz += real(2.0) * (txz(1, 0, 0) - txz(0, 0, 0)) / (zone_size_x<G>(m, i, j, k) * (r0 + rzm)) * dt;
-      vz += real(2.0) * (ymp * tzy(0, 1, 0) - ymn * tzy(0, 0, 0)) / ((ymp - ymn) * yd * (r0 + rzm)) * dt;
+      vy += qdiv(real(2.0) * (tzy(0, 0, 1) - tzy(0, 0, 0)), (m.zmin[k + 1] - m.zmin[k]) * (r0 + rym)) * dt;
+      vz += qdiv(real(2.0) * (tzz(0, 0, 0) - tzz(0, 0, -1)), (m.zmed[k] - m.zmed[k - 1]) * (r0 + rzm)) * dt;
+      vz += qdiv(real(2.0) * (txz(1, 0, 0) - txz(0, 0, 0)), zone_size_x<G>(m, i, j, k) * (r0 + rzm)) * dt;
+      vz += qdiv(real(2.0) * (ymp * tzy(0, 1, 0) - ymn * tzy(0, 0, 0)), (ymp - ymn) * yd * (r0 + rzm)) * dt;
     }
   }
   ox = vx;
@@ -481,20 +482,20 @@ __device__ __forceinline__ real newvel_x(const dmesh& m, int i, int j, int k, re
     // from the momenta's deviations: l0/r - Omega_f r = V0 drops out, and the
     // result is the deviation vx'
     const double r = rcyl64<G>(m, j, k);
-    return (real)(((double)mul_vol(m, mmx, i, j, k) + (double)mul_vol(m, mpxm, im, j, k)) /
-                  (((double)mul_vol(m, rho, i, j, k) + (double)mul_vol(m, rhoxm, im, j, k)) * r));
+    return (real)qdivd((double)mul_vol(m, mmx, i, j, k) + (double)mul_vol(m, mpxm, im, j, k),
+                       ((double)mul_vol(m, rho, i, j, k) + (double)mul_vol(m, rhoxm, im, j, k)) * r);
   }
   real r = (G == SPH) ? m.ymed[j] * m.sinzmed[k] : m.ymed[j];
-  return (mul_vol(m, mmx, i, j, k) + mul_vol(m, mpxm, im, j, k)) /
-             ((mul_vol(m, rho, i, j, k) + mul_vol(m, rhoxm, im, j, k)) * r) -
+  return qdiv(mul_vol(m, mmx, i, j, k) + mul_vol(m, mpxm, im, j, k),
+              (mul_vol(m, rho, i, j, k) + mul_vol(m, rhoxm, im, j, k)) * r) -
          omegaframe * r;
 }
 
 // src/newvel_y.c:67
 __device__ __forceinline__ real newvel_y(const dmesh& m, int i, int j, int k, real rho, real rhoym, real mmy,
                                            real mpym) {
-  return (mul_vol(m, mmy, i, j, k) + mul_vol(m, mpym, i, j - 1, k)) /
-         (mul_vol(m, rho, i, j, k) + mul_vol(m, rhoym, i, j - 1, k));
+  return qdiv(mul_vol(m, mmy, i, j, k) + mul_vol(m, mpym, i, j - 1, k),
+              mul_vol(m, rho, i, j, k) + mul_vol(m, rhoym, i, j - 1, k));
 }
 
 // ---------------------------------------------------------------- PPA (src/fargo_ppa_*.c)
@@ -526,7 +527,7 @@ __device__ __forceinline__ void ppa_limit(real q, real& qL, real& qR) {
 }
 // the swept fraction ksi of ppa_flux_value, the same for every quantity of a cell
 __device__ __forceinline__ real ppa_ksi(real v, real dt, real zsx) {
-  return (v > real(0.0)) ? v * dt / zsx : -v * dt / zsx;
+  return qdiv(fabs(v * dt), zsx);  // v dt / zsx where v > 0, else -v dt / zsx
 }
 __device__ __forceinline__ real ppa_flux_ksi(real v, real ksi, real qm, real qLm, real qRm, real q, real qL, real qR) {
   real qs;
@@ -544,11 +545,11 @@ __device__ __forceinline__ real ppa_flux_value(real v, real dt, real zsx, real q
                                                  real q, real qL, real qR) {
   real qs;
   if (v > real(0.0)) {
-    real ksi = v * dt / zsx;
+    real ksi = qdiv(v * dt, zsx);
     qs = qRm + ksi * (qm - qRm);
     qs += ksi * (real(1.0) - ksi) * (real(2.0) * qm - qRm - qLm);
   } else {
-    real ksi = -v * dt / zsx;
+    real ksi = qdiv(-v * dt, zsx);
     qs = qL + ksi * (q - qL);
     qs += ksi * (real(1.0) - ksi) * (real(2.0) * q - qR - qL);
   }
@@ -636,12 +637,12 @@ __device__ __forceinline__ double cfl_sumsq(const dmesh& m, int i, int j, int k,
   const double c0 = cs[l];
   double soundspeed2, viscosity;
   if (cp.iso) soundspeed2 = c0 * c0;
-  else soundspeed2 = cp.gamma * (cp.gamma - 1) * c0 / (double)rho[l];
+  else soundspeed2 = qdivd(cp.gamma * (cp.gamma - 1) * c0, (double)rho[l]);
   if (cp.alpha_visc) {
     const double y = m.ymed64[j];
     const double sq = sqrt(y * y * y / (1.0 * 1.0));
     if (cp.iso) viscosity = cp.alpha * c0 * c0 * sq;
-    else viscosity = cp.alpha * cp.gamma * (cp.gamma - 1.0) * c0 / (double)rho[l] * sq;
+    else viscosity = qdivd(cp.alpha * cp.gamma * (cp.gamma - 1.0) * c0, (double)rho[l]) * sq;
   } else {
     viscosity = cp.nu;
   }
@@ -671,7 +672,7 @@ __device__ __forceinline__ double cfl_sumsq(const dmesh& m, int i, int j, int k,
   const double cfl5_b = rdivd(fabs(vy1 - vy0), Zy);
   const double t5 = cfl5_a > cfl5_b ? cfl5_a : cfl5_b;
   const double cfl5 = (t5 > cfl5_c ? t5 : cfl5_c) * 4.0 * 1.41;  // 4 CVNR
-  const double m7 = Zmin.r;  // 1.0 / zmin
+  const double m7 = rdivd(1.0, Zmin);  // 1.0 / zmin
   const double cfl7 = 4.0 * viscosity * (m7 * m7);
   // the reference sums ten squares; the MHD/strong-shock terms (cfl6, cfl8-10)
   // are exact zeros here and adding +0.0 does not change the sum
@@ -725,18 +726,18 @@ template <int G>
 __device__ __forceinline__ void stockholm_rxy(const dmesh& m, int j, int k, real dt, const Ramps& R, real& rho,
                                               real& vx, real& vy, real rho0, real vx0, real vy0, const DampPar& d) {
   real taud = R.tau / R.ramp;
-  rho = (rho * taud + rho0 * dt) / (dt + taud);
+  rho = qdiv(rho * taud + rho0 * dt, dt + taud);
   real vx0_target = vx0;
   real radius = m.ymed[j];
   if (G == SPH) radius *= m.sinzmed[k];
   vx0_target -= (real)((d.of - d.of0) * radius);
-  vx = (vx * taud + vx0_target * dt) / (dt + taud);
-  vy = (vy * taud + vy0 * dt) / (dt + taud);
+  vx = qdiv(vx * taud + vx0_target * dt, dt + taud);
+  vy = qdiv(vy * taud + vy0 * dt, dt + taud);
 }
 // vz of a cell where R.rampi > 0
 __device__ __forceinline__ real stockholm_z(real dt, const Ramps& R, real vz, real vz0) {
   real taud = R.tau / R.rampi;
-  return (vz * taud + vz0 * dt) / (dt + taud);
+  return qdiv(vz * taud + vz0 * dt, dt + taud);
 }
 // the same on the arrays (cell l of ring (j,k))
 template <int G, int DZ>

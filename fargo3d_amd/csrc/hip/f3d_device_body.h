@@ -48,46 +48,66 @@ __device__ __forceinline__ int lxm_of(int l, int i, int nx) { return (i > 0) ? l
 __device__ __forceinline__ int ixm_of(int i, int nx) { return i > 0 ? i - 1 : nx - 1; }
 __device__ __forceinline__ int ixp_of(int i, int nx) { return i < nx - 1 ? i + 1 : 0; }
 
-// Division by a divisor that several quotients share, correctly rounded: with
-// r = RN(1/d) and q0 = RN(a r), the remainder a - q0 d is exact (one FMA)
-// and q0 + r (a - q0 d), rounded once (a second FMA), is RN(a/d) -- the
+// Division by a divisor d > 0 that several quotients share: r = recip(d), then
+// per quotient q0 = RN(a r), rem = q0 d - a (exact: one FMA) and
+// q = RN(q0 - rem r) (a second FMA).  With r = RN(1/d) that is RN(a/d), the
 // correction step of Markstein's division (round to nearest, d finite and
-// nonzero, no overflow or underflow).  Checked with exact integer arithmetic
-// for every pair of significands of the binary formats of precision 4 to 16
-// (1.4e9 pairs; q0 alone is wrong in 27% of them) and against IEEE division
-// on 6e8 random and near-midpoint binary64 pairs.  An exact quotient
-// (remainder 0, also a = -0) keeps q0.  So each quotient costs a multiply and
-// two FMAs instead of the full division sequence, and equals a/d bit for bit.
+// nonzero, no overflow or underflow), checked with exact integer arithmetic for
+// every pair of significands of the binary formats of precision 4 to 16 (1.4e9
+// pairs; q0 alone is wrong in 27% of them) and against IEEE division on 6e8
+// random and near-midpoint binary64 pairs.  The remainder is formed as q0 d - a:
+// where it vanishes it is then +0, and q0 - (+0) r keeps q0, a zero of either
+// sign included, without the comparison and the two selects that the remainder
+// a - q0 d needs.  recip() refines the hardware's estimate of 1/d by two Newton
+// steps r += r (1 - d r), and q is then, operation for operation, what the
+// full division computes for operands that it does not have to scale
+// (magnitudes far from the ends of the exponent range, as every density, zone
+// size and volume here), without its scaling and special-case instructions: 5
+// for the reciprocal and 3 per quotient against 11 per division.  A quotient
+// by 0 is NaN.
 struct Recip {
   real d, r;
 };
-__device__ __forceinline__ Recip recip(real d) { return Recip{d, real(1.0) / d}; }
+__device__ __forceinline__ double rcp_estimate(double d) { return __builtin_amdgcn_rcp(d); }
+__device__ __forceinline__ float rcp_estimate(float d) { return __builtin_amdgcn_rcpf(d); }
+__device__ __forceinline__ Recip recip(real d) {
+  real r = rcp_estimate(d);
+  r = fma(fma(-d, r, real(1.0)), r, r);
+  r = fma(fma(-d, r, real(1.0)), r, r);
+  return Recip{d, r};
+}
 __device__ __forceinline__ real rdiv(real a, const Recip& R) {
   const real q0 = a * R.r;
-  const real rem = fma(-q0, R.d, a);
-  return rem == real(0.0) ? q0 : fma(rem, R.r, q0);
+  return fma(-fma(q0, R.d, -a), R.r, q0);
 }
+// a / d for one quotient (the compiler shares recip() between equal divisors)
+__device__ __forceinline__ real qdiv(real a, real d) { return rdiv(a, recip(d)); }
 // the same in FP64 in every build (the CFL time step)
 struct RecipD {
   double d, r;
 };
-__device__ __forceinline__ RecipD recipd(double d) { return RecipD{d, 1.0 / d}; }
+__device__ __forceinline__ RecipD recipd(double d) {
+  double r = rcp_estimate(d);
+  r = fma(fma(-d, r, 1.0), r, r);
+  r = fma(fma(-d, r, 1.0), r, r);
+  return RecipD{d, r};
+}
 __device__ __forceinline__ double rdivd(double a, const RecipD& R) {
   const double q0 = a * R.r;
-  const double rem = fma(-q0, R.d, a);
-  return rem == 0.0 ? q0 : fma(rem, R.r, q0);
+  return fma(-fma(q0, R.d, -a), R.r, q0);
 }
+__device__ __forceinline__ double qdivd(double a, double d) { return rdivd(a, recipd(d)); }
 
 // x * InvVol(i,j,k)  ->  (x*InvVj[j]) / (Syk[k]*Sxi[i])
 __device__ __forceinline__ real mul_invvol(const dmesh& m, real x, int i, int j, int k) {
-  return (x * m.invvj[j]) / (m.syk[k] * m.sxi[i]);
+  return qdiv(x * m.invvj[j], m.syk[k] * m.sxi[i]);
 }
 // its divisor, for rdiv(): several quantities of one cell share it
 __device__ __forceinline__ Recip invvol_recip(const dmesh& m, int i, int k) { return recip(m.syk[k] * m.sxi[i]); }
 __device__ __forceinline__ real mul_invvol(const dmesh& m, real x, int j, const Recip& V) { return rdiv(x * m.invvj[j], V); }
 // x * Vol(i,j,k)  ->  ((x*Syk[k])*Sxi[i]) / InvVj[j]
 __device__ __forceinline__ real mul_vol(const dmesh& m, real x, int i, int j, int k) {
-  return ((x * m.syk[k]) * m.sxi[i]) / m.invvj[j];
+  return qdiv((x * m.syk[k]) * m.sxi[i], m.invvj[j]);
 }
 // the same with the ring's divisor InvVj[j] shared (rdiv())
 __device__ __forceinline__ real mul_vol(const dmesh& m, real x, int i, int k, const Recip& IV) {
@@ -95,7 +115,7 @@ __device__ __forceinline__ real mul_vol(const dmesh& m, real x, int i, int k, co
 }
 // Vol(i,j,k) standing alone  ->  (Syk[k]*Sxi[i]) / InvVj[j]
 __device__ __forceinline__ real vol(const dmesh& m, int i, int j, int k) {
-  return (m.syk[k] * m.sxi[i]) / m.invvj[j];
+  return qdiv(m.syk[k] * m.sxi[i], m.invvj[j]);
 }
 // x * SurfX(j,k)
 __device__ __forceinline__ real mul_surfx(const dmesh& m, real x, int j, int k) {
@@ -116,8 +136,8 @@ __device__ __forceinline__ real zone_size_x(const dmesh& m, int i, int j, int k)
 }
 template <int G>
 __device__ __forceinline__ real inv_zone_size_xmed(const dmesh& m, int i, int j, int k) {
-  if (G == SPH) return (m.invdiffxmed[i] / m.ymed[j]) / m.sinzmed[k];
-  return m.invdiffxmed[i] / m.ymed[j];
+  if (G == SPH) return qdiv(qdiv(m.invdiffxmed[i], m.ymed[j]), m.sinzmed[k]);
+  return qdiv(m.invdiffxmed[i], m.ymed[j]);
 }
 __device__ __forceinline__ real zone_size_y(const dmesh& m, int j) { return m.ymin[j + 1] - m.ymin[j]; }
 template <int G>
@@ -180,7 +200,7 @@ __device__ inline void cfl_min_publish(const double* ringmin, int n, unsigned lo
 // across.
 __device__ __forceinline__ real vanleer_slope(real dqm, real dqp) {
   const real p = dqp * dqm;
-  const real s = real(2.) * dqp * dqm / (dqm + dqp);
+  const real s = qdiv(p + p, dqm + dqp);  // 2 dqp dqm / (dqm + dqp); p > 0 bounds the divisor away from 0
   return (p <= real(0.0)) ? real(0.0) : s;
 }
 // upwind interface value (src/vanleer_y_b.c:60-65)

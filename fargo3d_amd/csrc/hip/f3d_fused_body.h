@@ -1111,12 +1111,12 @@ __device__ __forceinline__ void xsweep_ring(const dmesh& m, int ring, double dt6
     if (i < nx) {
       if (fargo) {
         const double zs = zone_size_x64<G>(m, i, j, k);
-        const double ntilde = vmed * dt64 / zs;
+        const double ntilde = qdivd(vmed * dt64, zs);
         const double nround = floor(ntilde + 0.5);
         if (i == 0) sh[1] = nround;
         if constexpr (cell::kFix64) V[i] = (real)(vt[s] - (vmed - vb));
         else V[i] = (real)(vt[s] - vmed);
-        vu[s] = (real)((ntilde - nround) * zs / dt64);
+        vu[s] = (real)qdivd((ntilde - nround) * zs, dt64);
       } else {
         if constexpr (cell::kFix64) V[i] = (real)(vt[s] + vb);
         else V[i] = (real)vt[s];
@@ -1458,16 +1458,16 @@ __device__ __forceinline__ void xsweep_wave(const dmesh& m, int ring, double dt6
 #pragma unroll
     for (int s = 0; s < CPT; s++) {
       const double zs = zone_size_x64<G>(m, ix[s], j, k);
-      const double ntilde = vmed * dt64 / zs;
+      const double ntilde = qdivd(vmed * dt64, zs);
       const double nround = floor(ntilde + 0.5);
       if (s == 0) nr0 = nround;
       if constexpr (cell::kFix64) vel[s] = (real)(vt[s] - (vmed - vb));
       else vel[s] = (real)(vt[s] - vmed);
-      vu[s] = (real)((ntilde - nround) * zs / dt64);
+      vu[s] = (real)qdivd((ntilde - nround) * zs, dt64);
     }
     // the shift of the ring is that of its cell 0: lane 0's, or for a tile
     // the same expression at i = 0
-    if constexpr (TILE) ns = (int)floor(vmed * dt64 / zone_size_x64<G>(m, 0, j, k) + 0.5);
+    if constexpr (TILE) ns = (int)floor(qdivd(vmed * dt64, zone_size_x64<G>(m, 0, j, k)) + 0.5);
     else
       ns = (int)__hiloint2double(__builtin_amdgcn_readlane(__double2hiint(nr0), 0),
                                  __builtin_amdgcn_readlane(__double2loint(nr0), 0));
@@ -1680,7 +1680,7 @@ __device__ __forceinline__ void kd_sweep_x_tile(const dim3 bid, const dmesh& m, 
     return g < 0 ? g + nx : g;
   };
   // the integer shift of the ring: ComputeResidual at i = 0 (src/compute_residual.c:68-71)
-  const int ns = fargo ? (int)floor(vmed * dt64 / zone_size_x64<G>(m, 0, j, k) + 0.5) : 0;
+  const int ns = fargo ? (int)floor(qdivd(vmed * dt64, zone_size_x64<G>(m, 0, j, k)) + 0.5) : 0;
   if (fargo && bid.x == 0 && p == 0) nshift_out[j + k * m.sy] = ns;
   const int g = gidx(p);
   real st[N];
@@ -1696,11 +1696,11 @@ __device__ __forceinline__ void kd_sweep_x_tile(const dim3 bid, const dmesh& m, 
     if (fargo) {
       // the residual split in FP64 (src/compute_residual.c:68-73)
       const double zs64 = zone_size_x64<G>(m, g, j, k);
-      const double ntilde = vmed * dt64 / zs64;
+      const double ntilde = qdivd(vmed * dt64, zs64);
       const double nround = floor(ntilde + 0.5);
       if constexpr (cell::kFix64) vp = (real)(v - (vmed - cell::vbase(m, j, k)));
       else vp = (real)(v - vmed);
-      vu = (real)((ntilde - nround) * zs64 / dt64);
+      vu = (real)qdivd((ntilde - nround) * zs64, dt64);
     } else {
       if constexpr (cell::kFix64) vp = (real)(v + cell::vbase(m, j, k));
       else vp = (real)v;
@@ -1877,9 +1877,9 @@ __device__ __forceinline__ void kd_finish(const dim3 bid, const dmesh& m, real d
   real y = (j > m.nghy) ? cell::newvel_y(m, i, j, k, r, rho_x[l - m.pitch], mmy[l], mpy[l - m.pitch]) : real(0.0);
   real z = real(0.0);
   if (DZ && k > m.nghz) {
-    z = (mul_vol(m, mmz[l], i, j, k) + mul_vol(m, mpz[l - m.stride], i, j, k - 1)) /
-        (mul_vol(m, r, i, j, k) + mul_vol(m, rho_x[l - m.stride], i, j, k - 1));
-    if (G == SPH) z /= m.ymed[j];
+    z = qdiv(mul_vol(m, mmz[l], i, j, k) + mul_vol(m, mpz[l - m.stride], i, j, k - 1),
+             mul_vol(m, r, i, j, k) + mul_vol(m, rho_x[l - m.stride], i, j, k - 1));
+    if (G == SPH) z = qdiv(z, m.ymed[j]);
   }
   if (stockholm) {
     // StockholmBoundary (src/stockholm.c:129-184) after NewVelocity_y/z; the
@@ -2115,7 +2115,7 @@ __device__ __forceinline__ void drag_solve(const FluidSet& F, real* const* v, in
   // the precision form solves in FP64: the stiff drag of small grains
   // couples the fluids' velocities so strongly that an FP32 solve rounds
   // every ring's cells alike, a torque that accumulates step after step
-  using dreal = std::conditional_t<cell::kFix64, double, real>;
+  using dreal = double;  // in both builds
   dreal m[NF * NF], b[NF];
 #pragma unroll
   for (int o = 0; o < NF; o++) {
@@ -2124,7 +2124,7 @@ __device__ __forceinline__ void drag_solve(const FluidSet& F, real* const* v, in
       const dreal rho_p = dreal(0.5) * ((dreal)F.rho[p][l] + (dreal)F.rho[p][idm]);
       if (p != o) {
         const dreal rho_o = dreal(0.5) * ((dreal)F.rho[o][l] + (dreal)F.rho[o][idm]);
-        if (p > o) m[p + o * NF] = -(dreal)dt * (dreal)omega * (dreal)F.alpha[p + o * NF] * rho_p / rho_o;
+        if (p > o) m[p + o * NF] = qdivd(-(dreal)dt * (dreal)omega * (dreal)F.alpha[p + o * NF] * rho_p, rho_o);
         else m[p + o * NF] = -(dreal)dt * (dreal)omega * (dreal)F.alpha[p + o * NF];
       } else {
         dreal sum = dreal(0.0);
@@ -2132,7 +2132,7 @@ __device__ __forceinline__ void drag_solve(const FluidSet& F, real* const* v, in
         for (int q = 0; q < NF; q++) {
           if (q != p) {
             const dreal rho_q = dreal(0.5) * ((dreal)F.rho[q][l] + (dreal)F.rho[q][idm]);
-            if (q > p) sum += (dreal)F.alpha[q + p * NF] * rho_q / rho_p;
+            if (q > p) sum += qdivd((dreal)F.alpha[q + p * NF] * rho_q, rho_p);
             else sum += (dreal)F.alpha[q + p * NF];
           }
         }
@@ -2170,7 +2170,7 @@ __device__ __forceinline__ void drag_solve(const FluidSet& F, real* const* v, in
     }
 #pragma unroll
     for (int ir2 = ir + 1; ir2 < NF; ir2++) {
-      const dreal factor = m[ir + ir2 * NF] / m[ir + ir * NF];
+      const dreal factor = qdivd(m[ir + ir2 * NF], m[ir + ir * NF]);
 #pragma unroll
       for (int ic = 0; ic < NF; ic++) m[ic + ir2 * NF] -= m[ic + ir * NF] * factor;
       b[ir2] -= b[ir] * factor;
@@ -2180,7 +2180,7 @@ __device__ __forceinline__ void drag_solve(const FluidSet& F, real* const* v, in
   for (int ir = NF - 1; ir > -1; ir--) {
 #pragma unroll
     for (int ic = NF - 1; ic > ir; ic--) b[ir] -= m[ic + ir * NF] * b[ic];
-    b[ir] /= m[ir + ir * NF];
+    b[ir] = qdivd(b[ir], m[ir + ir * NF]);
   }
 #pragma unroll
   for (int o = 0; o < NF; o++) v[o][l] = (real)b[o];
@@ -2241,23 +2241,23 @@ __device__ __forceinline__ void ddiff_core_cell(const dmesh& m, real dt, int bx,
   const int ll = i + j * m.pitch;
   const int llxm = lxm_of(ll, i, m.nx), llxp = lxp_of(ll, i, m.nx), llyp = ll + m.pitch, llym = ll - m.pitch;
   real update = real(0.0);
-  const real c = rhod[ll] / (rhod[ll] + rhog[ll]);
+  const real c = qdiv(rhod[ll], rhod[ll] + rhog[ll]);
   const real dxmin = m.xmin[i + 1] - m.xmin[i];
-  const real dxmedp = real(1.0) / m.invdiffxmed[ixp_of(i, m.nx)];
-  const real dxmedm = real(1.0) / m.invdiffxmed[i];
+  const real dxmedp = qdiv(real(1.0), m.invdiffxmed[ixp_of(i, m.nx)]);
+  const real dxmedm = qdiv(real(1.0), m.invdiffxmed[i]);
   const real d1 = real(0.25) * (rhod[ll] + rhog[ll] + rhod[llxp] + rhog[llxp]) * (yczc[llxp] + yczc[ll]);
   const real d2 = real(0.25) * (rhod[ll] + rhog[ll] + rhod[llxm] + rhog[llxm]) * (yczc[llxm] + yczc[ll]);
-  const real cxp = rhod[llxp] / (rhod[llxp] + rhog[llxp]);
-  const real cxm = rhod[llxm] / (rhod[llxm] + rhog[llxm]);
+  const real cxp = qdiv(rhod[llxp], rhod[llxp] + rhog[llxp]);
+  const real cxm = qdiv(rhod[llxm], rhod[llxm] + rhog[llxm]);
   const real ym = m.ymed[j];
-  update += real(1.0) / ym / ym / (dxmin) * (d1 * (cxp - c) / (dxmedp) - (d2 * (c - cxm)) / (dxmedm));
+  update += qdiv(qdiv(qdiv(real(1.0), ym), ym), dxmin) * (qdiv(d1 * (cxp - c), dxmedp) - qdiv(d2 * (c - cxm), dxmedm));
   const real d3 = real(0.5) * (rhod[ll] + rhog[ll] + rhod[llyp] + rhog[llyp]) * yfzc[llyp];
   const real d4 = real(0.5) * (rhod[ll] + rhog[ll] + rhod[llym] + rhog[llym]) * yfzc[ll];
-  const real cyp = rhod[llyp] / (rhod[llyp] + rhog[llyp]);
-  const real cym = rhod[llym] / (rhod[llym] + rhog[llym]);
-  update += real(1.0) / ym / (m.ymin[j + 1] - m.ymin[j]) *
-            (m.ymin[j + 1] * d3 * (cyp - c) / (m.ymed[j + 1] - ym) -
-             (m.ymin[j] * d4 * (c - cym)) / (ym - m.ymed[j - 1]));
+  const real cyp = qdiv(rhod[llyp], rhod[llyp] + rhog[llyp]);
+  const real cym = qdiv(rhod[llym], rhod[llym] + rhog[llym]);
+  update += qdiv(qdiv(real(1.0), ym), m.ymin[j + 1] - m.ymin[j]) *
+            (qdiv(m.ymin[j + 1] * d3 * (cyp - c), m.ymed[j + 1] - ym) -
+             qdiv(m.ymin[j] * d4 * (c - cym), ym - m.ymed[j - 1]));
   temp[ll] = rhod[ll] + dt * update;
 }
 
