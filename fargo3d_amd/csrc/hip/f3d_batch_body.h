@@ -37,6 +37,7 @@ struct BInst {
   real *rhoy, *rhox, *e2, *ey, *xm0, *xm1, *xm2, *xm3;
   double* vxmed;
   int* nshift;
+  XFluid xf;                // the X sweep's arrays
   const real *ydexp0, *ydexp1;
   cell::CflPar cp;
   cell::ViscPar vp;
@@ -339,14 +340,13 @@ __global__ void __launch_bounds__(64) kb_vmed(const BInst* I, const int* off, in
   kd_vmed<CYL, 0, 8>(dim3(blockIdx.x - off[ii]), in.m, in.vxt, in.vxmed);
 }
 
-template <int T>
-__global__ void __launch_bounds__(T) kb_sweep_x(const BInst* I, const int* off, int n) {
+// tiles of 64*CPT cells, one wave each
+template <int CPT>
+__global__ void __launch_bounds__(64) kb_sweep_x(const BInst* I, const int* off, int n) {
   const int ii = find_inst(off, n, blockIdx.x);
   const BInst& in = I[ii];
-  const int tx = (in.m.nx + x_tile_cells(T) - 1) / x_tile_cells(T);
-  kd_sweep_x_tile<CYL, 0, 0, T>(local2(blockIdx.x - off[ii], tx), in.m, in.clk[0], in.rhoy, in.vxt, in.mpx, in.mmx,
-                                in.mpy, in.mmy, nullptr, nullptr, in.ey, in.e2, in.rhox, in.vx, in.xm0, in.xm1,
-                                in.xm2, in.xm3, in.vxmed, in.nshift, in.of, in.fargo);
+  const int tx = (in.m.nx + x_tile_out(CPT) - 1) / x_tile_out(CPT), b = blockIdx.x - off[ii];
+  xsweep<CYL, 0, CPT, 0>(in.m, b / tx, b % tx, 0, 1, in.clk[0], in.xf, 4, in.of, in.fargo);
 }
 
 __global__ void __launch_bounds__(BXF) kb_finish(const BInst* I, const int* off, int n) {
@@ -422,7 +422,7 @@ static int batch_layout(f3d_batch* B) {
     c[BK_FIN][i] = gx * m.ny;
     c[BK_POT][i] = B->has_ps[i] ? gx * m.sy : 0;
     swy[i] = gx * ((m.ny + B->rows_y - 1) / B->rows_y);
-    xt[i] = ((m.nx + x_tile_cells(B->tile) - 1) / x_tile_cells(B->tile)) * m.ny;
+    xt[i] = ((m.nx + x_tile_out(B->tile / 64) - 1) / x_tile_out(B->tile / 64)) * m.ny;
   }
   for (int k = 0; k < BK_N; k++)
     if (k != BK_SWY && k != BK_XT && batch_offsets(B, c[k], &B->doff[k], &B->total[k])) return -1;
@@ -448,9 +448,9 @@ static void batch_launch(f3d_batch* B) {
   hipLaunchKernelGGL(kb_sweep_y, dim3(B->swy_total), dim3(BXF), 0, s, B->dI, B->dswy, n, B->rows_y);
   hipLaunchKernelGGL(kb_vmed, dim3(B->total[BK_VMED]), dim3(64), 0, s, B->dI,
                      B->doff[BK_VMED], n);
-  if (B->tile == 64) hipLaunchKernelGGL(kb_sweep_x<64>, dim3(B->xt_total), dim3(64), 0, s, B->dI, B->dxt, n);
-  else if (B->tile == 256) hipLaunchKernelGGL(kb_sweep_x<256>, dim3(B->xt_total), dim3(256), 0, s, B->dI, B->dxt, n);
-  else hipLaunchKernelGGL(kb_sweep_x<128>, dim3(B->xt_total), dim3(128), 0, s, B->dI, B->dxt, n);
+  if (B->tile == 64) hipLaunchKernelGGL(kb_sweep_x<1>, dim3(B->xt_total), dim3(64), 0, s, B->dI, B->dxt, n);
+  else if (B->tile == 256) hipLaunchKernelGGL(kb_sweep_x<4>, dim3(B->xt_total), dim3(64), 0, s, B->dI, B->dxt, n);
+  else hipLaunchKernelGGL(kb_sweep_x<2>, dim3(B->xt_total), dim3(64), 0, s, B->dI, B->dxt, n);
   hipLaunchKernelGGL(kb_finish, dim3(B->total[BK_FIN]), dim3(BXF), 0, s, B->dI, B->doff[BK_FIN], n);
   hipLaunchKernelGGL(kb_bound, dim3(B->total[BK_BND]), dim3(BXF), 0, s, B->dI, B->doff[BK_BND], n, 0);
 }
@@ -569,6 +569,11 @@ f3d_batch* f3d_batch_create(int n, const char* const* parfiles, const char* cons
     b.e2 = S->f[FS_E2]; b.ey = S->f[FS_EY];
     b.xm0 = S->f[FS_XM0]; b.xm1 = S->f[FS_XM0 + 1]; b.xm2 = S->f[FS_XM0 + 2]; b.xm3 = S->f[FS_XM0 + 3];
     b.vxmed = f.VxMed; b.nshift = f.Nshift;
+    memset(&b.xf, 0, sizeof(b.xf));
+    b.xf.rho_in = b.rhoy; b.xf.vxt = b.vxt; b.xf.rho_out = b.rhox; b.xf.vx_out = b.vx;
+    b.xf.vxmed = b.vxmed; b.xf.nshift = b.nshift;
+    b.xf.in[0] = b.mpx; b.xf.in[1] = b.mmx; b.xf.in[2] = b.mpy; b.xf.in[3] = b.mmy;
+    b.xf.out[2] = b.xm0; b.xf.out[3] = b.xm1;
     b.ydexp0 = S->ymin_dexp; b.ydexp1 = S->ymax_dexp;
     b.cp = cfl_par_f(c);
     b.vp.model = c->ph.visc; b.vp.nu = (real)c->ph.nu; b.vp.alpha = (real)c->ph.alpha;

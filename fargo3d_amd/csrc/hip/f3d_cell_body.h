@@ -499,61 +499,56 @@ __device__ __forceinline__ real newvel_y(const dmesh& m, int i, int j, int k, re
 }
 
 // ---------------------------------------------------------------- PPA (src/fargo_ppa_*.c)
-// monotonised-centred slope (src/fargo_ppa_a.c:58-69)
-__device__ __forceinline__ real ppa_slope(real qm, real q, real qp) {
-  real dqm = (q - qm);
-  real dqp = (qp - q);
-  if (dqp * dqm <= real(0.0)) return real(0.0);
-  real s = real(0.5) * (qp - qm);
+// Products by a power of two are exact, so a sum with one is a single FMA with
+// the same result: 3 q - 2 qR = fma(-2, qR, 3 q), and so on.
+// monotonised-centred slope (src/fargo_ppa_a.c:58-69) from the differences
+// dqm = q - qm and dqp = qp - q and the centred one s = (qp - qm)/2
+__device__ __forceinline__ real ppa_slope_d(real dqm, real dqp, real s) {
   real work = fabs(s);
-  if (real(2.0) * fabs(dqm) < work) work = real(2.0) * fabs(dqm);
-  if (real(2.0) * fabs(dqp) < work) work = real(2.0) * fabs(dqp);
-  return (s < 0) ? -work : work;
+  const real tm = real(2.0) * fabs(dqm), tp = real(2.0) * fabs(dqp);
+  if (tm < work) work = tm;
+  if (tp < work) work = tp;
+  const real r = (s < 0) ? -work : work;
+  return (dqp * dqm <= real(0.0)) ? real(0.0) : r;
 }
-// interface value q_{i+1/2} (src/fargo_ppa_b.c:52-55)
-__device__ __forceinline__ real ppa_face(real q, real qp, real s, real sp) {
-  return q + real(0.5) * (qp - q) - real(1.0) / real(6.0) * (sp - s);
+__device__ __forceinline__ real ppa_slope(real qm, real q, real qp) {
+  return ppa_slope_d(q - qm, qp - q, real(0.5) * (qp - qm));
 }
+// interface value q_{i+1/2} (src/fargo_ppa_b.c:52-55), dqp = qp - q
+__device__ __forceinline__ real ppa_face_d(real q, real dqp, real s, real sp) {
+  return fma(real(0.5), dqp, q) - real(1.0) / real(6.0) * (sp - s);
+}
+__device__ __forceinline__ real ppa_face(real q, real qp, real s, real sp) { return ppa_face_d(q, qp - q, s, sp); }
 // Colella-Woodward monotonicity (src/fargo_ppa_c.c:52-63)
 __device__ __forceinline__ void ppa_limit(real q, real& qL, real& qR) {
   if ((qR - q) * (q - qL) < real(0.0)) {
     qL = q;
     qR = q;
   }
-  real diff = qR - qL;
-  real cord = q - real(0.5) * (qL + qR);
-  if (real(6.0) * diff * cord > diff * diff) qL = real(3.0) * q - real(2.0) * qR;
-  if (-diff * diff > real(6.0) * diff * cord) qR = real(3.0) * q - real(2.0) * qL;
+  const real diff = qR - qL;
+  const real cord = fma(real(-0.5), qL + qR, q);
+  const real dc = real(6.0) * diff * cord, dd = diff * diff;
+  if (dc > dd) qL = fma(real(-2.0), qR, real(3.0) * q);
+  if (-dd > dc) qR = fma(real(-2.0), qL, real(3.0) * q);
 }
-// the swept fraction ksi of ppa_flux_value, the same for every quantity of a cell
-__device__ __forceinline__ real ppa_ksi(real v, real dt, real zsx) {
-  return qdiv(fabs(v * dt), zsx);  // v dt / zsx where v > 0, else -v dt / zsx
+// The parabola's average over the swept fraction k of the upwind cell
+// (src/fargo_ppa_d.c:62-70): the left cell (qm, qLm, qRm), its right end swept
+// (up), or this cell (q, qL, qR), its left end swept (down)
+__device__ __forceinline__ real ppa_swept_up(real k, real qm, real qLm, real qRm) {
+  real qs = qRm + k * (qm - qRm);
+  qs += k * (real(1.0) - k) * (fma(real(2.0), qm, -qRm) - qLm);
+  return qs;
 }
-__device__ __forceinline__ real ppa_flux_ksi(real v, real ksi, real qm, real qLm, real qRm, real q, real qL, real qR) {
-  real qs;
-  if (v > real(0.0)) {
-    qs = qRm + ksi * (qm - qRm);
-    qs += ksi * (real(1.0) - ksi) * (real(2.0) * qm - qRm - qLm);
-  } else {
-    qs = qL + ksi * (q - qL);
-    qs += ksi * (real(1.0) - ksi) * (real(2.0) * q - qR - qL);
-  }
+__device__ __forceinline__ real ppa_swept_down(real k, real q, real qL, real qR) {
+  real qs = qL + k * (q - qL);
+  qs += k * (real(1.0) - k) * (fma(real(2.0), q, -qR) - qL);
   return qs;
 }
 // parabolic average over the swept zone (src/fargo_ppa_d.c:62-70)
 __device__ __forceinline__ real ppa_flux_value(real v, real dt, real zsx, real qm, real qLm, real qRm,
                                                  real q, real qL, real qR) {
-  real qs;
-  if (v > real(0.0)) {
-    real ksi = qdiv(v * dt, zsx);
-    qs = qRm + ksi * (qm - qRm);
-    qs += ksi * (real(1.0) - ksi) * (real(2.0) * qm - qRm - qLm);
-  } else {
-    real ksi = qdiv(-v * dt, zsx);
-    qs = qL + ksi * (q - qL);
-    qs += ksi * (real(1.0) - ksi) * (real(2.0) * q - qR - qL);
-  }
-  return qs;
+  const real k = qdiv(fabs(v * dt), zsx);  // v dt / zsx where v > 0, else -v dt / zsx
+  return (v > real(0.0)) ? ppa_swept_up(k, qm, qLm, qRm) : ppa_swept_down(k, q, qL, qR);
 }
 
 // ---------------------------------------------------------------- conservative updates
@@ -561,9 +556,10 @@ __device__ __forceinline__ real ppa_flux_value(real v, real dt, real zsx, real q
 __device__ __forceinline__ real flux_x(const dmesh& m, int i, int j, int k, real dt, real a, real b) {
   return mul_invvol(m, mul_surfx(m, a - b, j, k) * dt, i, j, k);
 }
-// the same with the cell's InvVol divisor shared by its quantities
-__device__ __forceinline__ real flux_x(const dmesh& m, int j, int k, real dt, real a, real b, const Recip& V) {
-  return mul_invvol(m, mul_surfx(m, a - b, j, k) * dt, j, V);
+// the same from the difference d of the face flows, with the cell's InvVol
+// divisor shared by its quantities
+__device__ __forceinline__ real flux_x(const dmesh& m, int j, int k, real dt, real d, const Recip& V) {
+  return mul_invvol(m, mul_surfx(m, d, j, k) * dt, j, V);
 }
 // src/update_y.c:68-70: (a*SurfY(j) - b*SurfY(j+1))*dt*InvVol
 __device__ __forceinline__ real flux_y(const dmesh& m, int i, int j, int k, real dt, real a, real b) {

@@ -1004,12 +1004,11 @@ __global__ void __launch_bounds__(BXF) kf_sweep_y3(dmesh m, real dt, const real*
 }
 
 // 3-D: momenta + Z sweep for rows j in [1, sy-2] (the Y sweep's stencil)
-template <int G, int DZ, int AD, int SPLIT>
-__global__ void __launch_bounds__(BXF) kf_sweep_z(dmesh m, real dt, const real* __restrict__ rho_in, const real* __restrict__ vxt,
+template <int G, int AD, int SPLIT>
+__device__ __forceinline__ void kd_sweep_z(const dim3 b, const dmesh& m, real dt, const real* __restrict__ rho_in, const real* __restrict__ vxt,
                                                   const real* __restrict__ vyt, const real* __restrict__ vzt, const real* __restrict__ e_in,
                                                   real* __restrict__ rho_out, real* __restrict__ q0, real* __restrict__ q1, real* __restrict__ q2, real* __restrict__ q3,
                                                   real* __restrict__ q4, real* __restrict__ q5, real* __restrict__ e_out, int planes_per, real of) {
-  const dim3 b = blockIdx;
   const int i = b.x * blockDim.x + threadIdx.x;
   if (i >= m.nx) return;
   const int j = 1 + (SPLIT ? (int)b.y >> 1 : (int)b.y);
@@ -1021,354 +1020,53 @@ __global__ void __launch_bounds__(BXF) kf_sweep_z(dmesh m, real dt, const real* 
   else column_sweep<6 + AD>(col, r0, r1, dt);
 }
 
-// The ring X sweep with the cell state in registers.  Thread t owns cells
-// i = t + s*blockDim.x (s < CPT) of the ring; LDS holds q = Q/rho, the slopes
-// (then the limited qL) and the faces (then qR, then the face fluxes) of the
-// quantities this workgroup carries, plus the advection velocity.  GRP 0: one
-// workgroup per ring carries every quantity; GRP 1/2: two workgroups per ring
-// (blockIdx.x = 2*ring + grp - 1), each with the density and half of the
-// quantities, so that each needs about half the LDS and more workgroups fit
-// on a CU.  Group 1 carries Mpx, Mmx (and Mpy in 3-D) and writes the density,
-// Vx, VxMed and Nshift; group 2 carries the other momenta and the energy.
-// Every quantity goes through the same arithmetic as in the reference's
-// routine sequence, so any split gives the same bits.
-template <int DZ, int AD, int GRP>
-struct XQuant {
-  static constexpr int NM = DZ ? 6 : 4;
-  static constexpr int NQ = NM + AD;  // quantities of the whole ring
-  static constexpr int NA = DZ ? 3 : 2;  // group 1: Mpx, Mmx (, Mpy)
-  static constexpr int NL = GRP == 0 ? NQ : GRP == 1 ? NA : NQ - NA;  // carried here
-  static constexpr int first = GRP == 2 ? NA : 0;  // global index of local quantity 0
+// ------------------------------------------------------------------ the X sweep
+// The X sweep of one ring, or of a tile of one, by one wave with the cells in
+// registers: ComputeResidual, the van Leer pass with the cell residual, the PPA
+// pass with the uniform residual, AdvectSHIFT and NewVelocity_x, the arithmetic
+// of the reference's routines cell for cell.  Lane L holds the CPT consecutive
+// cells L*CPT .. L*CPT+CPT-1 of the wave's 64*CPT.
+//
+// Every neighbour the sweep reads is i +- 1: within a lane a register, across
+// lanes the value of the lane before or after, by a rotation of the whole wave
+// (DPP wave_ror:1 / wave_rol:1).  No LDS, no barrier.
+//   RING = 1: the ring has exactly 64*CPT cells, whose periodicity the rotation
+//     is; VxMed is summed in the wave (f3d_ring::literal).
+//   RING = 0: a tile, the cells from tile*(64*CPT - 2 kXHalo) - kXHalo on
+//     (indexes wrapped around the ring), of which the 64*CPT - 2 kXHalo inside
+//     the halos are updated: the van Leer pass reaches 2 cells, the PPA pass 3
+//     more, NewVelocity_x 1.  The rotations wrap the tile's ends into each other,
+//     and what that puts into the halos does not reach the updated cells.  VxMed
+//     comes from kd_vmed.  Each tile writes only its own cells, at their shifted
+//     positions, so tiles that overlap (the last of a ring, a ring shorter than a
+//     tile) write each cell once.
+//
+// Bound by the issue of FP64 instructions and their dependences.  A transported
+// quantity meets the others only through the density and its face values, so
+// the density goes first through both passes, leaving per cell the densities
+// and faces of either pass, and then every quantity goes through both passes
+// from its load to its store before the next one is begun (its successor's load
+// in flight): only one quantity is live at a time, whatever their number, and
+// the loop over them is a loop.  Measured against all quantities held through
+// each pass in turn (256 registers, two waves per SIMD, spills in 3-D) or in LDS (13 barriers a ring):
+// 384x128 14.5 -> 8.5 us, 1250x437 31.6 -> 25.6, five fluids 1024x512 111 -> 96,
+// 3-D 500x150x45 275 -> 187, 256x96x32 45.6 -> 40; FP32 4096x1024 97 -> 94.
+struct XFluid {
+  const real* rho_in;
+  const real* vxt;
+  const real* in[7];  // Mpx, Mmx, Mpy, Mmy (, Mpz, Mmz) (, energy)
+  real* out[7];       // the same after the sweep, from Mpy on
+  real* rho_out;
+  real* vx_out;
+  double* vxmed;
+  int* nshift;
+};
+struct XTab {
+  XFluid f[8];
 };
 
-// An empty asm that "changes" the LDS row stride after each barrier: the
-// compiler then computes each phase's LDS addresses in that phase instead of
-// holding every phase's addresses in registers from the start (measured:
-// 118 -> 82 registers with the VPRE form, 4 -> 5 waves per SIMD).
-#define XR_REFRESH() asm volatile("" : "+s"(nxv))
-// VPRE: VxMed of the ring from kf_vmed (the kernel then carries no sum).
-template <int G, int DZ, int AD, int CPT, int GRP, int VPRE>
-__device__ __forceinline__ void xsweep_ring(const dmesh& m, int ring, double dt64, const real* __restrict__ rho_in,
-                                            const real* __restrict__ vxt, const real* const* qin,
-                                            const real* __restrict__ e_in, real* __restrict__ e_out,
-                                            real* __restrict__ rho_out, real* __restrict__ vx_out,
-                                            real* const* qout, double* __restrict__ vxmed_out,
-                                            int* __restrict__ nshift_out, real omegaframe, int fargo) {
-  using XQ = XQuant<DZ, AD, GRP>;
-  constexpr int NL = XQ::NL;
-  constexpr int N = NL + 1;  // + the density (local index NL)
-  constexpr int NM = XQ::NM;
-  extern __shared__ double lds_d[];
-  const int nx = m.nx;
-  const real dt = (real)dt64;
-  const int P = (N * nx + 1) & ~1;  // N * nx rounded up to 8-byte multiples
-  real* AQ = (real*)lds_d;   // q = Q/rho (or rho): N * nx
-  real* SL = AQ + P;         // slopes, then limited qL: N * nx
-  real* FC = SL + P;         // faces, then qR, then face fluxes: N * nx
-  real* V = FC + P;          // advection velocity: nx
-  double* sh = (double*)(((size_t)(V + nx) + 15) & ~(size_t)15);  // 4
-  const int j = m.nghy + ring % m.ny;
-  const int k = DZ ? m.nghz + ring / m.ny : 0;
-  const int base = j * m.pitch + k * m.stride;
-  const int t = threadIdx.x, nt = blockDim.x;
-  real st[CPT][N];
-  double vt[CPT];
-  real vu[CPT];
-#pragma unroll
-  for (int s = 0; s < CPT; s++) {
-    const int i = t + s * nt;
-    if (i < nx) {
-      st[s][NL] = rho_in[base + i];
-#pragma unroll
-      for (int c = 0; c < NL; c++) {
-        const int q = XQ::first + c;
-        st[s][c] = (q < NM) ? qin[q][base + i] : e_in[base + i];
-      }
-      vt[s] = vxt[base + i];
-    }
-  }
-  double vmed;
-  if constexpr (VPRE) {
-    // VxMed of this ring from kf_vmed, run before this launch
-    vmed = vxmed_out[j + k * m.sy];
-  } else {
-    // ComputeVmed(Vx_temp) (src/compute_vmed.c:14-30), FP64, by the first
-    // wave, staged through the start of the LDS (free until the barrier)
-    if (t < 64) {
-      const double sum = wave_ring_sum<8>(vxt + base, m, lds_d);
-      if (t == 0) sh[0] = vmed_full(sum / (m.XMAX - m.XMIN), m, j, k);
-    }
-    __syncthreads();
-    vmed = sh[0];
-  }
-  // ComputeResidual (src/compute_residual.c:68-73), FP64: cell residual into V
-  // (the stored velocity is the deviation from V0 in the precision form)
-  int ns = 0;
-  const double vb = cell::vbase(m, j, k);
-#pragma unroll
-  for (int s = 0; s < CPT; s++) {
-    const int i = t + s * nt;
-    if (i < nx) {
-      if (fargo) {
-        const double zs = zone_size_x64<G>(m, i, j, k);
-        const double ntilde = qdivd(vmed * dt64, zs);
-        const double nround = floor(ntilde + 0.5);
-        if (i == 0) sh[1] = nround;
-        if constexpr (cell::kFix64) V[i] = (real)(vt[s] - (vmed - vb));
-        else V[i] = (real)(vt[s] - vmed);
-        vu[s] = (real)qdivd((ntilde - nround) * zs, dt64);
-      } else {
-        if constexpr (cell::kFix64) V[i] = (real)(vt[s] + vb);
-        else V[i] = (real)vt[s];
-      }
-    }
-  }
-  __syncthreads();  // V complete
-  if (fargo) {
-    ns = (int)sh[1];
-    if (GRP != 2 && t == 0) {
-      nshift_out[j + k * m.sy] = ns;
-      if (!VPRE) vxmed_out[j + k * m.sy] = vmed;
-    }
-  }
-  int nxv = nx;  // LDS row stride, re-read after each barrier (keeps the
-  // addresses of each phase out of the registers of the others)
-  // X_advection (src/transport.c:208-226), twice with FARGO
-  for (int pass = 0; pass < (fargo ? 2 : 1); pass++) {
-    const bool ppa = (pass == 1);
-    if (ppa) {
-      __syncthreads();
-      XR_REFRESH();  // the last update read V of the neighbours
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) V[i] = vu[s];
-      }
-    }
-    // q = Q/rho (DivideByRho) and, for the density, q = rho
-#pragma unroll
-    for (int s = 0; s < CPT; s++) {
-      const int i = t + s * nt;
-      if (i < nx) {
-        const real r = st[s][NL];
-        const Recip R = recip(r);
-#pragma unroll
-        for (int c = 0; c < NL; c++) AQ[c * nxv + i] = rdiv(st[s][c], R);
-        AQ[NL * nxv + i] = r;
-      }
-    }
-    __syncthreads();
-      XR_REFRESH();
-    if (!ppa) {
-      // VanLeerX_a (src/vanleer_x_a.c:60-68).  The gradient at face i,
-      // (q_i - q_{i-1}) / zone_i, is cell i's left and cell i-1's right
-      // gradient: computed once per face into FC (free until VanLeerX_b).
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) {
-          const int im = ixm_of(i, nx);
-          const Recip Zi = recip(zone_size_x<G>(m, i, j, k));
-#pragma unroll
-          for (int c = 0; c < N; c++) {
-            const real* a = AQ + c * nxv;
-            FC[c * nxv + i] = rdiv(a[i] - a[im], Zi);
-          }
-        }
-      }
-      __syncthreads();
-      XR_REFRESH();
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) {
-          const int ip = ixp_of(i, nx);
-#pragma unroll
-          for (int c = 0; c < N; c++) SL[c * nxv + i] = vanleer_slope(FC[c * nxv + i], FC[c * nxv + ip]);
-        }
-      }
-      __syncthreads();
-      XR_REFRESH();
-      // VanLeerX_b (src/vanleer_x_b.c:60-65)
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) {
-          const int im = ixm_of(i, nx);
-          const real zi = zone_size_x<G>(m, i, j, k), zm = zone_size_x<G>(m, im, j, k);
-          const real v = V[i];
-#pragma unroll
-          for (int c = 0; c < N; c++) {
-            const real* a = AQ + c * nxv;
-            const real* sl = SL + c * nxv;
-            FC[c * nxv + i] = vanleer_face(v, dt, a[im], sl[im], zm, a[i], sl[i], zi);
-          }
-        }
-      }
-      __syncthreads();
-      XR_REFRESH();
-    } else {
-      // VanLeerX_PPA_a: monotonised-centred slope (src/fargo_ppa_a.c:58-69)
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) {
-          const int im = ixm_of(i, nx), ip = ixp_of(i, nx);
-#pragma unroll
-          for (int c = 0; c < N; c++) {
-            const real* a = AQ + c * nxv;
-            SL[c * nxv + i] = cell::ppa_slope(a[im], a[i], a[ip]);
-          }
-        }
-      }
-      __syncthreads();
-      XR_REFRESH();
-      // VanLeerX_PPA_b: face value q_{i+1/2} = qR of cell i = qL of cell i+1
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) {
-          const int ip = ixp_of(i, nx);
-#pragma unroll
-          for (int c = 0; c < N; c++) {
-            const real* a = AQ + c * nxv;
-            const real* sl = SL + c * nxv;
-            FC[c * nxv + i] = cell::ppa_face(a[i], a[ip], sl[i], sl[ip]);
-          }
-        }
-      }
-      __syncthreads();
-      XR_REFRESH();
-      // VanLeerX_PPA_c (src/fargo_ppa_c.c): the limited (qL, qR) of each cell;
-      // qL goes to SL (slopes are no longer read), qR to FC once every
-      // neighbour has read its face
-      real qr[CPT][N];
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) {
-          const int im = ixm_of(i, nx);
-#pragma unroll
-          for (int c = 0; c < N; c++) {
-            real qL = FC[c * nxv + im], qR = FC[c * nxv + i];
-            cell::ppa_limit(AQ[c * nxv + i], qL, qR);
-            SL[c * nxv + i] = qL;
-            qr[s][c] = qR;
-          }
-        }
-      }
-      __syncthreads();
-      XR_REFRESH();
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) {
-#pragma unroll
-          for (int c = 0; c < N; c++) FC[c * nxv + i] = qr[s][c];
-        }
-      }
-      __syncthreads();
-      XR_REFRESH();
-      // VanLeerX_PPA_d: parabolic average over the swept zone (src/fargo_ppa_d.c:62-70);
-      // the fluxes replace qR in FC once every neighbour has read it
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) {
-          const int im = ixm_of(i, nx);
-          const real v = V[i];
-          const real ksi = cell::ppa_ksi(v, dt, zone_size_x<G>(m, i, j, k));
-#pragma unroll
-          for (int c = 0; c < N; c++) {
-            const real* a = AQ + c * nxv;
-            const real* qL = SL + c * nxv;
-            const real* qR = FC + c * nxv;
-            qr[s][c] = cell::ppa_flux_ksi(v, ksi, a[im], qL[im], qR[im], a[i], qL[i], qR[i]);
-          }
-        }
-      }
-      __syncthreads();
-      XR_REFRESH();
-#pragma unroll
-      for (int s = 0; s < CPT; s++) {
-        const int i = t + s * nt;
-        if (i < nx) {
-#pragma unroll
-          for (int c = 0; c < N; c++) FC[c * nxv + i] = qr[s][c];
-        }
-      }
-      __syncthreads();
-      XR_REFRESH();
-    }
-    // UpdateX for every quantity and UpdateDensityX last (src/update_x.c:69-71,
-    // src/update_density_x.c:66-68), on the registers
-#pragma unroll
-    for (int s = 0; s < CPT; s++) {
-      const int i = t + s * nt;
-      if (i < nx) {
-        const int ip = ixp_of(i, nx);
-        const real v0 = V[i], v1 = V[ip];
-        const real* ds = FC + NL * nxv;
-        const Recip Vi = invvol_recip(m, i, k);
-#pragma unroll
-        for (int c = 0; c < NL; c++) {
-          const real* f = FC + c * nxv;
-          st[s][c] += cell::flux_x(m, j, k, dt, v0 * f[i] * ds[i], v1 * f[ip] * ds[ip], Vi);
-        }
-        st[s][NL] += cell::flux_x(m, j, k, dt, v0 * ds[i], v1 * ds[ip], Vi);
-      }
-    }
-  }
-  // AdvectSHIFT (src/advect_shift.c:45-58): cell i moves to i + ns (mod nx).
-  // Quantities other than the density, Mpx and Mmx go to their shifted
-  // positions straight from the registers.
-#pragma unroll
-  for (int s = 0; s < CPT; s++) {
-    const int i = t + s * nt;
-    if (i < nx) {
-      int it = (i + ns) % nx;
-      if (it < 0) it += nx;
-#pragma unroll
-      for (int c = 0; c < NL; c++) {
-        const int q = XQ::first + c;
-        if (q >= 2) {
-          if (q < NM) qout[q - 2][base + it] = st[s][c];
-          else e_out[base + it] = st[s][c];
-        }
-      }
-      if (GRP != 2) {
-        // density, Mpx, Mmx of the shifted ring into AQ for NewVelocity_x
-        // (the AQ reads of the last pass ended before its final barrier)
-        AQ[0 * nx + it] = st[s][0];
-        AQ[1 * nx + it] = st[s][1];
-        AQ[2 * nx + it] = st[s][NL];
-        rho_out[base + it] = st[s][NL];
-      }
-    }
-  }
-  if (GRP != 2) {
-    __syncthreads();
-      XR_REFRESH();
-    // NewVelocity_x (src/newvel_x.c:78-86)
-#pragma unroll
-    for (int s = 0; s < CPT; s++) {
-      const int i = t + s * nt;
-      if (i < nx) {
-        const int im = ixm_of(i, nx);
-        const real* R = AQ + 2 * nx;
-        vx_out[base + i] = cell::newvel_x<G>(m, i, j, k, R[i], R[im], AQ[1 * nx + i], AQ[0 * nx + im], omegaframe);
-      }
-    }
-  }
-}
-
-// A ring of 64*CPT cells held by one wave, CPT consecutive cells per lane:
-// lane L holds cells L*CPT .. L*CPT+CPT-1.  The ring is periodic, so the left
-// neighbour of a lane's first cell is the last cell of the lane before (lane
-// 63 for lane 0) and the right neighbour of its last cell the first cell of
-// the lane after: one rotation per array, no LDS and no barrier.
 template <int CPT>
-struct WRing {
+struct Cells {
   template <class T>
   __device__ __forceinline__ static void left(const T (&a)[CPT], T (&out)[CPT]) {
     out[0] = from_left(a[CPT - 1]);
@@ -1383,219 +1081,288 @@ struct WRing {
   }
 };
 
-// The X sweep of one ring by one wave (rings of exactly 64*CPT cells), the
-// cell state in registers: the same arithmetic as xsweep_ring, cell for cell
-// (ComputeResidual, VanLeerX_a/b, VanLeerX_PPA_a-d, UpdateX and
-// UpdateDensityX for both passes, AdvectSHIFT, NewVelocity_x), with every
-// neighbour read from a register or from the next lane.  Each quantity goes
-// through a pass on its own after the density's faces (which every update
-// reads), so only one quantity's stencil arrays are live at a time.  VxMed
-// is summed in the wave (f3d_ring::literal) from the velocities it holds.
-// TILE = 1: the wave holds a tile of a longer ring instead, the 64*CPT cells
-// from tile*(64*CPT - 2 kXHalo) - kXHalo on (indexes wrapped around the
-// ring), and updates the 64*CPT - 2 kXHalo cells inside the halos, the same
-// reach as kf_sweep_x_tile's: the rotations wrap the tile's two ends into
-// each other, and what that puts into the halo cells does not reach the
-// updated ones.  VxMed then comes from kf_vmed.
-template <int G, int DZ, int AD, int CPT, int TILE = 0>
-__device__ __forceinline__ void xsweep_wave(const dmesh& m, int ring, double dt64, const real* __restrict__ rho_in,
-                                            const real* __restrict__ vxt, const real* const* qin,
-                                            const real* __restrict__ e_in, real* __restrict__ e_out,
-                                            real* __restrict__ rho_out, real* __restrict__ vx_out,
-                                            real* const* qout, double* __restrict__ vxmed,
-                                            int* __restrict__ nshift_out, real omegaframe, int fargo,
-                                            int tile = 0) {
-  using W = WRing<CPT>;
-  constexpr int NM = DZ ? 6 : 4;
-  constexpr int NQ = NM + AD;  // transported quantities besides the density
-  constexpr int TOUT = 64 * CPT - 2 * kXHalo;  // cells a tile updates
-  const int nx = m.nx;         // == 64 * CPT for a whole ring
+__host__ __device__ constexpr int x_tile_out(int cpt) { return 64 * cpt - 2 * kXHalo; }
+
+// group g of ng: the density and quantities [c0, c1); group 0 holds Mpx and
+// Mmx and writes the density, Vx, VxMed and Nshift (every group of a tile goes
+// through the density's passes for itself)
+__device__ __forceinline__ void x_group(int g, int ng, int nq, int& c0, int& c1) {
+  c0 = ng == 1 ? 0 : 2 * g;
+  c1 = (g == ng - 1) ? nq : 2 * g + 2;
+}
+
+template <int G, int DZ, int CPT, int RING>
+__device__ __forceinline__ void xsweep(const dmesh& m, int ring, int tile, int grp, int ngrp, double dt64,
+                                       const XFluid& T, int nq, real omegaframe, int fargo) {
+  using W = Cells<CPT>;
+  constexpr int TOUT = x_tile_out(CPT);
+  const real* __restrict__ rho_in = T.rho_in;
+  const int nx = m.nx;
   const real dt = (real)dt64;
   const int lane = (int)threadIdx.x;
   const int j = m.nghy + ring % m.ny;
   const int k = DZ ? m.nghz + ring / m.ny : 0;
-  const int base = j * m.pitch + k * m.stride;
-  // this lane's first cell on the ring (a tile's may lie outside [0, nx))
+  const int base = j * m.pitch + k * m.stride, l2 = j + k * m.sy;
+  int c0, c1;
+  x_group(grp, ngrp, nq, c0, c1);
+  // this lane's cells: tile positions u0 .. u0+CPT-1, ring indexes ix
   const int t0 = tile * TOUT;
-  const int u0 = TILE ? t0 - kXHalo + lane * CPT : lane * CPT;
-  int ix[CPT];  // the cells' indexes on the ring
+  const int u0 = RING ? lane * CPT : t0 - kXHalo + lane * CPT;
+  int ix[CPT];
+  if (RING) {
 #pragma unroll
-  for (int s = 0; s < CPT; s++) {
-    int g = u0 + s;
-    if (TILE) {
-      g %= nx;
-      if (g < 0) g += nx;
-    }
-    ix[s] = g;
+    for (int s = 0; s < CPT; s++) ix[s] = u0 + s;
+  } else {
+    ix[0] = u0 % nx;
+    if (ix[0] < 0) ix[0] += nx;
+#pragma unroll
+    for (int s = 1; s < CPT; s++) ix[s] = ix[s - 1] + 1 < nx ? ix[s - 1] + 1 : 0;
   }
-  real rho[CPT], st[NQ][CPT];
+  auto load = [&](const real* __restrict__ p, real (&a)[CPT]) {
+#pragma unroll
+    for (int s = 0; s < CPT; s++) a[s] = p[base + ix[s]];
+  };
+  real rho[CPT], st[CPT];
   double vt[CPT];
+  load(rho_in, rho);
 #pragma unroll
-  for (int s = 0; s < CPT; s++) {
-    rho[s] = rho_in[base + ix[s]];
-#pragma unroll
-    for (int c = 0; c < NQ; c++) st[c][s] = (c < NM) ? qin[c][base + ix[s]] : e_in[base + ix[s]];
-    vt[s] = vxt[base + ix[s]];
-  }
+  for (int s = 0; s < CPT; s++) vt[s] = T.vxt[base + ix[s]];
+  load(T.in[c0], st);
   // ComputeResidual (src/compute_residual.c:68-73), FP64: the cell residual
-  // velocity for the van Leer pass, the uniform one for the PPA pass
-  real vel[CPT], vu[CPT];
+  // velocity v for the van Leer pass, the uniform one w for the PPA pass
+  real v[CPT], w[CPT];
   int ns = 0;
+  const double vb = cell::vbase(m, j, k);
   if (fargo) {
     double vmed;
-    if constexpr (TILE) {
-      vmed = vxmed[j + k * m.sy];  // from kf_vmed
-    } else {
+    if constexpr (RING) {
       // ComputeVmed(Vx_temp) (src/compute_vmed.c:14-30): the ring's weights
       // are in the lanes already, consecutive ones in each
-      double w[CPT];
+      double wt[CPT];
 #pragma unroll
-      for (int s = 0; s < CPT; s++) w[s] = vt[s] * (m.xmin64[ix[s] + 1] - m.xmin64[ix[s]]);
-      vmed = vmed_full(f3d_ring::literal<CPT>(w, 0.0, 0, 64) / (m.XMAX - m.XMIN), m, j, k);
+      for (int s = 0; s < CPT; s++) wt[s] = vt[s] * (m.xmin64[ix[s] + 1] - m.xmin64[ix[s]]);
+      vmed = vmed_full(f3d_ring::literal<CPT>(wt, 0.0, 0, 64) / (m.XMAX - m.XMIN), m, j, k);
+    } else {
+      vmed = T.vxmed[l2];
     }
-    const double vb = cell::vbase(m, j, k);
-    double nr0 = 0.0;
 #pragma unroll
     for (int s = 0; s < CPT; s++) {
       const double zs = zone_size_x64<G>(m, ix[s], j, k);
       const double ntilde = qdivd(vmed * dt64, zs);
       const double nround = floor(ntilde + 0.5);
-      if (s == 0) nr0 = nround;
-      if constexpr (cell::kFix64) vel[s] = (real)(vt[s] - (vmed - vb));
-      else vel[s] = (real)(vt[s] - vmed);
-      vu[s] = (real)qdivd((ntilde - nround) * zs, dt64);
+      if constexpr (cell::kFix64) v[s] = (real)(vt[s] - (vmed - vb));
+      else v[s] = (real)(vt[s] - vmed);
+      w[s] = (real)qdivd((ntilde - nround) * zs, dt64);
     }
-    // the shift of the ring is that of its cell 0: lane 0's, or for a tile
-    // the same expression at i = 0
-    if constexpr (TILE) ns = (int)floor(qdivd(vmed * dt64, zone_size_x64<G>(m, 0, j, k)) + 0.5);
-    else
-      ns = (int)__hiloint2double(__builtin_amdgcn_readlane(__double2hiint(nr0), 0),
-                                 __builtin_amdgcn_readlane(__double2loint(nr0), 0));
-    if (lane == 0 && (!TILE || tile == 0)) {
-      nshift_out[j + k * m.sy] = ns;
-      if (!TILE) vxmed[j + k * m.sy] = vmed;
+    // the shift of the ring is that of its cell 0
+    ns = (int)floor(qdivd(vmed * dt64, zone_size_x64<G>(m, 0, j, k)) + 0.5);
+    if (lane == 0 && tile == 0 && grp == 0) {
+      T.nshift[l2] = ns;
+      if (RING) T.vxmed[l2] = vmed;
     }
   } else {
-    const double vb = cell::vbase(m, j, k);
 #pragma unroll
     for (int s = 0; s < CPT; s++) {
-      if constexpr (cell::kFix64) vel[s] = (real)(vt[s] + vb);
-      else vel[s] = (real)vt[s];
+      if constexpr (cell::kFix64) v[s] = (real)(vt[s] + vb);
+      else v[s] = (real)vt[s];
     }
   }
-  // per-cell mesh factors shared by the quantities
-  real zs[CPT], zsl[CPT];
-  Recip Vi[CPT];
+  // van Leer pass: the factor of the upwind slope in the face value
+  // (src/vanleer_x_b.c:60-65: q_{i-1} + (z_{i-1} - v dt)/2 s_{i-1} where v > 0,
+  // else q_i - (z_i + v dt)/2 s_i)
+  Recip Z[CPT], V[CPT];
+  real A[CPT];
+  {
+    real zs[CPT], zl[CPT];
+#pragma unroll
+    for (int s = 0; s < CPT; s++) {
+      zs[s] = zone_size_x<G>(m, ix[s], j, k);
+      Z[s] = recip(zs[s]);
+      V[s] = invvol_recip(m, ix[s], k);
+    }
+    W::left(zs, zl);
+#pragma unroll
+    for (int s = 0; s < CPT; s++)
+      A[s] = v[s] > real(0.0) ? real(0.5) * (zl[s] - v[s] * dt) : -(real(0.5) * (zs[s] + v[s] * dt));
+  }
+  auto vanleer = [&](const real (&q)[CPT], real (&fc)[CPT]) {
+    real ql[CPT], g[CPT], gr[CPT], sl[CPT], sll[CPT];
+    W::left(q, ql);
+    // VanLeerX_a (src/vanleer_x_a.c:60-68), the gradient once per face
+#pragma unroll
+    for (int s = 0; s < CPT; s++) g[s] = rdiv(q[s] - ql[s], Z[s]);
+    W::right(g, gr);
+#pragma unroll
+    for (int s = 0; s < CPT; s++) sl[s] = vanleer_slope(g[s], gr[s]);
+    W::left(sl, sll);
+#pragma unroll
+    for (int s = 0; s < CPT; s++) {
+      const bool pos = v[s] > real(0.0);
+      fc[s] = (pos ? ql[s] : q[s]) + A[s] * (pos ? sll[s] : sl[s]);
+    }
+  };
+  // PPA pass: the swept fraction (src/fargo_ppa_d.c:62-70); the uniform
+  // residual has one sign along a ring but for the rounding of its zone sizes
+  real K[CPT];
+  bool up = true, down = true;
 #pragma unroll
   for (int s = 0; s < CPT; s++) {
-    zs[s] = zone_size_x<G>(m, ix[s], j, k);
-    Vi[s] = invvol_recip(m, ix[s], k);
+    K[s] = fargo ? rdiv(fabs(w[s] * dt), Z[s]) : real(0.0);
+    up = up && w[s] > real(0.0);
+    down = down && !(w[s] > real(0.0));
   }
-  W::left(zs, zsl);
-
-  // X_advection (src/transport.c:208-226), twice with FARGO
-  for (int pass = 0; pass < (fargo ? 2 : 1); pass++) {
-    const bool ppa = (pass == 1);
-    if (ppa) {
+  const bool all_up = __all(up), all_down = __all(down);
+  auto ppa = [&](const real (&q)[CPT], real (&fc)[CPT]) {
+    real ql[CPT], qr[CPT], d[CPT], dr[CPT], sl[CPT], slr[CPT], fr[CPT], qL[CPT], qR[CPT];
+    W::left(q, ql);
+    W::right(q, qr);
 #pragma unroll
-      for (int s = 0; s < CPT; s++) vel[s] = vu[s];
-    }
-    real vr[CPT];
-    W::right(vel, vr);
-    Recip Rr[CPT];
-    real ksi[CPT];
+    for (int s = 0; s < CPT; s++) d[s] = q[s] - ql[s];
+    W::right(d, dr);
+    // VanLeerX_PPA_a (src/fargo_ppa_a.c:58-69)
+#pragma unroll
+    for (int s = 0; s < CPT; s++) sl[s] = cell::ppa_slope_d(d[s], dr[s], real(0.5) * (qr[s] - ql[s]));
+    W::right(sl, slr);
+    // VanLeerX_PPA_b (src/fargo_ppa_b.c:52-55): q at face i+1/2
+#pragma unroll
+    for (int s = 0; s < CPT; s++) fr[s] = cell::ppa_face_d(q[s], dr[s], sl[s], slr[s]);
+    W::left(fr, qL);
+    // VanLeerX_PPA_c (src/fargo_ppa_c.c:52-63)
 #pragma unroll
     for (int s = 0; s < CPT; s++) {
-      Rr[s] = recip(rho[s]);  // DivideByRho of every quantity (the density before this pass)
-      ksi[s] = ppa ? cell::ppa_ksi(vel[s], dt, zs[s]) : real(0.0);
+      qR[s] = fr[s];
+      cell::ppa_limit(q[s], qL[s], qR[s]);
     }
-    // the face value (van Leer) or swept-zone average (PPA) of q at each cell's
-    // left face, for one quantity
-    auto faces = [&](const real (&q)[CPT], real (&fc)[CPT]) {
-      real ql[CPT], qr[CPT];
-      W::left(q, ql);
-      W::right(q, qr);
-      if (!ppa) {
-        // VanLeerX_a (src/vanleer_x_a.c:60-68), gradient once per face
-        real g[CPT], gr[CPT], sl[CPT], sll[CPT];
+    // VanLeerX_PPA_d: the upwind cell is the left one (up) or this one
+    if (all_down) {
 #pragma unroll
-        for (int s = 0; s < CPT; s++) g[s] = rdiv(q[s] - ql[s], recip(zs[s]));
-        W::right(g, gr);
+      for (int s = 0; s < CPT; s++) fc[s] = cell::ppa_swept_down(K[s], q[s], qL[s], qR[s]);
+    } else {
+      real qLl[CPT], qRl[CPT];
+      W::left(qL, qLl);
+      W::left(qR, qRl);
+      if (all_up) {
 #pragma unroll
-        for (int s = 0; s < CPT; s++) sl[s] = vanleer_slope(g[s], gr[s]);
-        W::left(sl, sll);
-        // VanLeerX_b (src/vanleer_x_b.c:60-65)
-#pragma unroll
-        for (int s = 0; s < CPT; s++) fc[s] = vanleer_face(vel[s], dt, ql[s], sll[s], zsl[s], q[s], sl[s], zs[s]);
+        for (int s = 0; s < CPT; s++) fc[s] = cell::ppa_swept_up(K[s], ql[s], qLl[s], qRl[s]);
       } else {
-        // VanLeerX_PPA_a/b/c/d (src/fargo_ppa_a.c:58-69, src/fargo_ppa_b.c:52-55,
-        // src/fargo_ppa_c.c:52-63, src/fargo_ppa_d.c:62-70)
-        real sl[CPT], slr[CPT], fr[CPT], qL[CPT], qR[CPT];
-#pragma unroll
-        for (int s = 0; s < CPT; s++) sl[s] = cell::ppa_slope(ql[s], q[s], qr[s]);
-        W::right(sl, slr);
-#pragma unroll
-        for (int s = 0; s < CPT; s++) fr[s] = cell::ppa_face(q[s], qr[s], sl[s], slr[s]);  // q at face i+1/2
-        W::left(fr, qL);
-#pragma unroll
-        for (int s = 0; s < CPT; s++) {
-          qR[s] = fr[s];
-          cell::ppa_limit(q[s], qL[s], qR[s]);
-        }
-        real qLl[CPT], qRl[CPT];
-        W::left(qL, qLl);
-        W::left(qR, qRl);
 #pragma unroll
         for (int s = 0; s < CPT; s++)
-          fc[s] = cell::ppa_flux_ksi(vel[s], ksi[s], ql[s], qLl[s], qRl[s], q[s], qL[s], qR[s]);
+          fc[s] = w[s] > real(0.0) ? cell::ppa_swept_up(K[s], ql[s], qLl[s], qRl[s])
+                                   : cell::ppa_swept_down(K[s], q[s], qL[s], qR[s]);
       }
-    };
-    // the density's faces first: every quantity's update reads them
-    real fd[CPT], fdr[CPT];
-    faces(rho, fd);
-    W::right(fd, fdr);
-    // UpdateX of every quantity (src/update_x.c:69-71)
+    }
+  };
+  // UpdateX (src/update_x.c:69-71): a += (f_i - f_{i+1}) SurfX dt InvVol with
+  // the face flows f = x y (the FP32 build subtracts from the unrounded product)
+  auto update = [&](real (&a)[CPT], const real (&x)[CPT], const real (&y)[CPT]) {
+    real f[CPT], fr[CPT];
+    {
+#pragma clang fp contract(off)
 #pragma unroll
-    for (int c = 0; c < NQ; c++) {
-      real q[CPT], fc[CPT], fcr[CPT];
+      for (int s = 0; s < CPT; s++) f[s] = x[s] * y[s];
+    }
+    W::right(f, fr);
 #pragma unroll
-      for (int s = 0; s < CPT; s++) q[s] = rdiv(st[c][s], Rr[s]);
-      faces(q, fc);
-      W::right(fc, fcr);
+    for (int s = 0; s < CPT; s++) {
+      const real d = cell::kFix64 ? fma(x[s], y[s], -fr[s]) : f[s] - fr[s];
+      a[s] += cell::flux_x(m, j, k, dt, d, V[s]);
+    }
+  };
+  // the density through both passes: its faces, its values before either, and
+  // those after both (VanLeerX_b, VanLeerX_PPA_d, src/update_density_x.c:66-68)
+  real fd1[CPT], fd2[CPT], rho2[CPT];
+  Recip R1[CPT], R2[CPT];
+#pragma unroll
+  for (int s = 0; s < CPT; s++) R1[s] = recip(rho[s]);
+  vanleer(rho, fd1);
+  update(rho, v, fd1);
+  if (fargo) {
+#pragma unroll
+    for (int s = 0; s < CPT; s++) {
+      R2[s] = recip(rho[s]);
+      rho2[s] = rho[s];
+    }
+    ppa(rho, fd2);
+    update(rho2, w, fd2);
+  } else {
+#pragma unroll
+    for (int s = 0; s < CPT; s++) rho2[s] = rho[s];
+  }
+  // one quantity through both passes
+  auto advance = [&](real (&a)[CPT]) {
+    real q[CPT], fc[CPT];
+#pragma unroll
+    for (int s = 0; s < CPT; s++) q[s] = rdiv(a[s], R1[s]);
+    vanleer(q, fc);
+#pragma unroll
+    for (int s = 0; s < CPT; s++) fc[s] = v[s] * fc[s];
+    update(a, fc, fd1);
+    if (fargo) {
+#pragma unroll
+      for (int s = 0; s < CPT; s++) q[s] = rdiv(a[s], R2[s]);
+      ppa(q, fc);
+#pragma unroll
+      for (int s = 0; s < CPT; s++) fc[s] = w[s] * fc[s];
+      update(a, fc, fd2);
+    }
+  };
+  // AdvectSHIFT (src/advect_shift.c:45-58): cell i moves to i + ns (mod nx); a
+  // tile writes the cells inside its halos that lie on the ring
+  int to[CPT];
+  bool mine[CPT];
+  {
+    int sh = ns % nx;
+    if (sh < 0) sh += nx;
+#pragma unroll
+    for (int s = 0; s < CPT; s++) {
+      to[s] = ix[s] + sh;
+      if (to[s] >= nx) to[s] -= nx;
+      mine[s] = RING || (u0 + s >= t0 && u0 + s < t0 + TOUT && u0 + s < nx);
+    }
+  }
+  real mp[CPT];  // Mpx after the sweep
+  for (int c = c0; c < c1; c++) {
+    real nxt[CPT];
+    load(T.in[min(c + 1, c1 - 1)], nxt);
+    advance(st);
+    if (c == 0) {
+#pragma unroll
+      for (int s = 0; s < CPT; s++) mp[s] = st[s];
+    } else if (c == 1) {
+      // the density, and NewVelocity_x (src/newvel_x.c:78-86) at the
+      // destination from the moved cell and its left neighbour
+      real rl[CPT], ml[CPT];
+      W::left(rho2, rl);
+      W::left(mp, ml);
 #pragma unroll
       for (int s = 0; s < CPT; s++)
-        st[c][s] += cell::flux_x(m, j, k, dt, vel[s] * fc[s] * fd[s], vr[s] * fcr[s] * fdr[s], Vi[s]);
+        if (mine[s]) {
+          T.rho_out[base + to[s]] = rho2[s];
+          T.vx_out[base + to[s]] = cell::newvel_x<G>(m, to[s], j, k, rho2[s], rl[s], st[s], ml[s], omegaframe);
+        }
+    } else {
+      real* __restrict__ o = T.out[c];
+#pragma unroll
+      for (int s = 0; s < CPT; s++)
+        if (mine[s]) o[base + to[s]] = st[s];
     }
-    // UpdateDensityX last (src/update_density_x.c:66-68)
 #pragma unroll
-    for (int s = 0; s < CPT; s++) rho[s] += cell::flux_x(m, j, k, dt, vel[s] * fd[s], vr[s] * fdr[s], Vi[s]);
-  }
-  // AdvectSHIFT (src/advect_shift.c:45-58): cell i moves to i + ns (mod nx);
-  // NewVelocity_x (src/newvel_x.c:78-86) at the destination, from the moved
-  // cell and its left neighbour
-  real rl[CPT], mpl[CPT];
-  W::left(rho, rl);
-  W::left(st[0], mpl);
-#pragma unroll
-  for (int s = 0; s < CPT; s++) {
-    // a tile writes the cells inside its halos that lie on the ring
-    if (TILE && (u0 + s < t0 || u0 + s >= t0 + TOUT || u0 + s >= nx)) continue;
-    int it = (ix[s] + ns) % nx;
-    if (it < 0) it += nx;
-#pragma unroll
-    for (int c = 2; c < NQ; c++) {
-      if (c < NM) qout[c - 2][base + it] = st[c][s];
-      else e_out[base + it] = st[c][s];
-    }
-    rho_out[base + it] = rho[s];
-    vx_out[base + it] = cell::newvel_x<G>(m, it, j, k, rho[s], rl[s], st[1][s], mpl[s], omegaframe);
+    for (int s = 0; s < CPT; s++) st[s] = nxt[s];
   }
 }
 
-// LDS bytes of xsweep_ring for n carried quantities + the density
-inline size_t xsweep_ring_lds(int nx, int ncarried) {
-  const size_t P = ((size_t)(ncarried + 1) * nx + 1) & ~(size_t)1;
-  return std::max((3 * P + nx) * sizeof(real) + 64, (f3d_ring::lds_doubles(8) + 8) * sizeof(double));
+// blocks [f*per, (f+1)*per) take fluid f; a ring's tiles, and a tile's groups,
+// are consecutive (XCD-contiguous order)
+template <int G, int DZ, int CPT, int RING>
+__global__ void __launch_bounds__(64, CPT >= 3 ? 2 : CPT == 2 ? 3 : 6)
+kf_sweep_x(dmesh m, double dt64, XTab T, int nrings, int ntiles, int ngrp, int nq, real omegaframe,
+           int fargo) {
+  int b = xcd_linear();
+  const int g = b % ngrp;
+  b /= ngrp;
+  const int tile = b % ntiles;
+  b /= ntiles;
+  xsweep<G, DZ, CPT, RING>(m, b % nrings, tile, g, ngrp, dt64, T.f[b / nrings], nq, omegaframe, fargo);
 }
 
 // ComputeVmed(Vx_temp) (src/compute_vmed.c:14-30) for the X sweeps: one wave
@@ -1645,221 +1412,22 @@ __global__ void __launch_bounds__(BXF) kf_sweep_y2v(dmesh m, real dt, Y2Tab T, i
                                T.q[fl][1], T.q[fl][2], T.q[fl][3], T.e_out[fl], rows_per, of);
 }
 
-// X sweep of rings too long for LDS: a workgroup of T threads owns a tile of
-// T - 2H cells and loads H = 6 halo cells on each side (the van Leer pass
-// needs 2, the PPA pass 3 more of the van Leer result, NewVelocity_x the left
-// neighbour), so no tile waits for another; thread t owns tile position t.
-// VxMed comes from kf_vmed.  The outputs go to their shifted positions
-// directly (AdvectSHIFT, src/advect_shift.c:45-58) with NewVelocity_x computed
-// at the destination cell from the source cell and its left neighbour.
-__host__ __device__ constexpr int x_tile_cells(int threads) { return threads - 2 * kXHalo; }
-template <int G, int DZ, int AD, int T>
-__device__ __forceinline__ void kd_sweep_x_tile(const dim3 bid, const dmesh& m, double dt64, const real* rho_in, const real* vxt, const real* mpx, const real* mmx, const real* mpy, const real* mmy, const real* mpz, const real* mmz, const real* e_in, real* e_out, real* rho_out, real* vx_out, real* mpy_o, real* mmy_o, real* mpz_o, real* mmz_o, const double* vxmed, int* nshift_out, real omegaframe, int fargo) {
-  constexpr int H = kXHalo, W = T, TW = x_tile_cells(T);
-  static_assert(2 * H <= TW, "tile narrower than its halos");
-  const real dt = (real)dt64;
-  constexpr int NM = DZ ? 6 : 4;
-  constexpr int NQ = NM + AD;
-  constexpr int N = NQ + 1;
-  // q = Q/rho, slopes (then limited qL), faces (then qR, then face fluxes),
-  // the advection velocity of the pass (the cell residual, then the uniform
-  // one); the cell state stays in registers
-  __shared__ real AQ[N * W], SL[N * W], FC[N * W];
-  __shared__ real V[W];
-  const int nx = m.nx;
-  const int ring = bid.y;
-  const int j = m.nghy + ring % m.ny;
-  const int k = DZ ? m.nghz + ring / m.ny : 0;
-  const int base = j * m.pitch + k * m.stride;
-  const int i0 = bid.x * TW;
-  const int p = threadIdx.x;
-  const double vmed = vxmed[j + k * m.sy];
-  const real* qin[7] = {mpx, mmx, mpy, mmy, DZ ? mpz : e_in, DZ ? mmz : e_in, e_in};
-  auto gidx = [&](int q) {
-    int g = (i0 - H + q) % nx;
-    return g < 0 ? g + nx : g;
-  };
-  // the integer shift of the ring: ComputeResidual at i = 0 (src/compute_residual.c:68-71)
-  const int ns = fargo ? (int)floor(qdivd(vmed * dt64, zone_size_x64<G>(m, 0, j, k)) + 0.5) : 0;
-  if (fargo && bid.x == 0 && p == 0) nshift_out[j + k * m.sy] = ns;
-  const int g = gidx(p);
-  real st[N];
-  st[NQ] = rho_in[base + g];
-#pragma unroll
-  for (int c = 0; c < NQ; c++) st[c] = (c < NM) ? qin[c][base + g] : e_in[base + g];
-  const real zs = zone_size_x<G>(m, g, j, k);
-  // the left neighbour's zone (the upwind face reads it)
-  const real zsm = zone_size_x<G>(m, gidx(p - 1), j, k);
-  real vp, vu = real(0.0);  // this cell's advection velocity in the current pass; the uniform residual
-  {
-    const double v = vxt[base + g];
-    if (fargo) {
-      // the residual split in FP64 (src/compute_residual.c:68-73)
-      const double zs64 = zone_size_x64<G>(m, g, j, k);
-      const double ntilde = qdivd(vmed * dt64, zs64);
-      const double nround = floor(ntilde + 0.5);
-      if constexpr (cell::kFix64) vp = (real)(v - (vmed - cell::vbase(m, j, k)));
-      else vp = (real)(v - vmed);
-      vu = (real)qdivd((ntilde - nround) * zs64, dt64);
-    } else {
-      if constexpr (cell::kFix64) vp = (real)(v + cell::vbase(m, j, k));
-      else vp = (real)v;
-    }
-    V[p] = vp;
+// The 3-D Z sweep, and in the same launch (V.vxt[0] given) the VxMed pass of the
+// X sweep as in kf_sweep_y2v: the first nvm workgroups sum one ring each, the
+// others are the sweep's grid gz in launch order.
+template <int G, int AD, int SPLIT>
+__global__ void __launch_bounds__(BXF) kf_sweep_z(dmesh m, real dt, const real* __restrict__ rho_in, const real* __restrict__ vxt,
+                                                  const real* __restrict__ vyt, const real* __restrict__ vzt, const real* __restrict__ e_in,
+                                                  real* __restrict__ rho_out, real* __restrict__ q0, real* __restrict__ q1, real* __restrict__ q2, real* __restrict__ q3,
+                                                  real* __restrict__ q4, real* __restrict__ q5, real* __restrict__ e_out, int planes_per, real of,
+                                                  double* __restrict__ vxmed, int nvm, dim3 gz) {
+  const int lin = (int)blockIdx.x - nvm;
+  if (lin < 0) {
+    kd_vmed<G, 1, 8>(dim3(blockIdx.x), m, vxt, vxmed);
+    return;
   }
-  for (int pass = 0; pass < (fargo ? 2 : 1); pass++) {
-    // valid range of the state entering this pass: [lo, hi)
-    const int lo = pass ? 2 : 0, hi = pass ? W - 2 : W;
-    if (p >= lo && p < hi) {
-      const real r = st[NQ];
-      const Recip R = recip(r);
-#pragma unroll
-      for (int c = 0; c < NQ; c++) AQ[c * W + p] = rdiv(st[c], R);
-      AQ[NQ * W + p] = r;
-    }
-    __syncthreads();  // also orders the first pass after the stores of V
-    if (pass) {
-      // the uniform residual: every read of the cell residual ended before
-      // the barrier above
-      vp = vu;
-      V[p] = vu;
-    }
-    int ulo, uhi;  // positions updated by this pass
-    if (!pass) {
-      // the gradient at face p, (q_p - q_{p-1}) / zone_p, once per face into
-      // FC: the left gradient of cell p and the right one of cell p-1
-      if (p >= 1) {
-        const Recip Z = recip(zs);
-#pragma unroll
-        for (int c = 0; c < N; c++) {
-          const real* a = AQ + c * W;
-          FC[c * W + p] = rdiv(a[p] - a[p - 1], Z);
-        }
-      }
-      __syncthreads();
-      if (p >= 1 && p < W - 1) {
-#pragma unroll
-        for (int c = 0; c < N; c++) SL[c * W + p] = vanleer_slope(FC[c * W + p], FC[c * W + p + 1]);
-      }
-      __syncthreads();
-      if (p >= 2 && p < W - 1) {
-#pragma unroll
-        for (int c = 0; c < N; c++) {
-          const real* a = AQ + c * W;
-          const real* sl = SL + c * W;
-          FC[c * W + p] = vanleer_face(vp, dt, a[p - 1], sl[p - 1], zsm, a[p], sl[p], zs);
-        }
-      }
-      __syncthreads();
-      ulo = 2;
-      uhi = W - 2;
-    } else {
-      if (p >= 3 && p < W - 3) {
-#pragma unroll
-        for (int c = 0; c < N; c++) {
-          const real* a = AQ + c * W;
-          SL[c * W + p] = cell::ppa_slope(a[p - 1], a[p], a[p + 1]);
-        }
-      }
-      __syncthreads();
-      if (p >= 3 && p < W - 4) {
-#pragma unroll
-        for (int c = 0; c < N; c++) {
-          const real* a = AQ + c * W;
-          const real* sl = SL + c * W;
-          FC[c * W + p] = cell::ppa_face(a[p], a[p + 1], sl[p], sl[p + 1]);
-        }
-      }
-      __syncthreads();
-      // limited (qL, qR): qL into SL (slopes are no longer read), qR into FC
-      // once every neighbour has read its face
-      real qr[N];
-      const bool lim = p >= 4 && p < W - 4;
-      if (lim) {
-#pragma unroll
-        for (int c = 0; c < N; c++) {
-          real qL = FC[c * W + p - 1], qR = FC[c * W + p];
-          cell::ppa_limit(AQ[c * W + p], qL, qR);
-          SL[c * W + p] = qL;
-          qr[c] = qR;
-        }
-      }
-      __syncthreads();
-      if (lim) {
-#pragma unroll
-        for (int c = 0; c < N; c++) FC[c * W + p] = qr[c];
-      }
-      __syncthreads();
-      // face fluxes into FC once every neighbour has read qR
-      const bool flx = p >= 5 && p < W - 4;
-      if (flx) {
-        const real ksi = cell::ppa_ksi(vp, dt, zs);
-#pragma unroll
-        for (int c = 0; c < N; c++) {
-          const real* a = AQ + c * W;
-          const real* qL = SL + c * W;
-          const real* qR = FC + c * W;
-          qr[c] = cell::ppa_flux_ksi(vp, ksi, a[p - 1], qL[p - 1], qR[p - 1], a[p], qL[p], qR[p]);
-        }
-      }
-      __syncthreads();
-      if (flx) {
-#pragma unroll
-        for (int c = 0; c < N; c++) FC[c * W + p] = qr[c];
-      }
-      __syncthreads();
-      ulo = 5;
-      uhi = W - 5;
-    }
-    // UpdateX / UpdateDensityX (src/update_x.c:69-71, src/update_density_x.c:66-68), on the registers
-    if (p >= ulo && p < uhi) {
-      const real v0 = vp, v1 = V[p + 1];
-      const real* ds = FC + NQ * W;
-      const Recip Vg = invvol_recip(m, g, k);
-#pragma unroll
-      for (int c = 0; c < NQ; c++) {
-        const real* f = FC + c * W;
-        st[c] += cell::flux_x(m, j, k, dt, v0 * f[p] * ds[p], v1 * f[p + 1] * ds[p + 1], Vg);
-      }
-      st[NQ] += cell::flux_x(m, j, k, dt, v0 * ds[p], v1 * ds[p + 1], Vg);
-    }
-    if (pass == 0 && fargo) __syncthreads();  // the PPA pass rewrites AQ and V
-  }
-  // the updated density and Mpx of positions [H-1, H+TW) for NewVelocity_x
-  // (AQ is free: its last reads were before the final barrier of the pass)
-  if (p >= H - 1 && p < H + TW) {
-    AQ[0 * W + p] = st[0];
-    AQ[1 * W + p] = st[NQ];
-  }
-  __syncthreads();
-  // outputs of the tile's cells [H, H+TW) at their shifted positions
-  // (AdvectSHIFT, src/advect_shift.c:45-58), NewVelocity_x computed at the
-  // destination from the source cell and its left neighbour
-  if (p >= H && p < H + TW) {
-    const int i = i0 + p - H;
-    if (i < nx) {
-      int d = (i + ns) % nx;
-      if (d < 0) d += nx;
-      vx_out[base + d] = cell::newvel_x<G>(m, d, j, k, st[NQ], AQ[1 * W + p - 1], st[1], AQ[0 * W + p - 1],
-                                           omegaframe);
-      rho_out[base + d] = st[NQ];
-#pragma unroll
-      for (int c = 2; c < NQ; c++) {
-        if (c < NM) (c == 2 ? mpy_o : c == 3 ? mmy_o : c == 4 ? mpz_o : mmz_o)[base + d] = st[c];
-        else e_out[base + d] = st[c];
-      }
-    }
-  }
-}
-template <int G, int DZ, int AD, int T>
-__global__ void __launch_bounds__(T) kf_sweep_x_tile(dmesh m, double dt64, const real* __restrict__ rho_in, const real* __restrict__ vxt,
-                                                      const real* __restrict__ mpx, const real* __restrict__ mmx, const real* __restrict__ mpy,
-                                                      const real* __restrict__ mmy, const real* __restrict__ mpz, const real* __restrict__ mmz,
-                                                      const real* __restrict__ e_in, real* __restrict__ e_out, real* __restrict__ rho_out,
-                                                      real* __restrict__ vx_out, real* __restrict__ mpy_o, real* __restrict__ mmy_o, real* __restrict__ mpz_o,
-                                                      real* __restrict__ mmz_o, const double* __restrict__ vxmed, int* __restrict__ nshift_out,
-                                                      real omegaframe, int fargo) {
-  kd_sweep_x_tile<G, DZ, AD, T>(xcd_bid(), m, dt64, rho_in, vxt, mpx, mmx, mpy, mmy, mpz, mmz, e_in, e_out, rho_out, vx_out, mpy_o, mmy_o, mpz_o, mmz_o, vxmed, nshift_out, omegaframe, fargo);
+  const dim3 b(lin % gz.x, (lin / gz.x) % gz.y, lin / (gz.x * gz.y));
+  kd_sweep_z<G, AD, SPLIT>(b, m, dt, rho_in, vxt, vyt, vzt, e_in, rho_out, q0, q1, q2, q3, q4, q5, e_out, planes_per, of);
 }
 
 // NewVelocity_y/z on active faces and Stockholm damping on active cells.
@@ -2498,12 +2066,12 @@ static int rows_y_of(const dmesh& m, int nf) {
 // the quantities), 0 one, -1 automatic: measured on MI355X, the split only
 // pays when a sweep has fewer waves than the GPU has SIMDs (small 2-D grids)
 static int g_colsplit = -1;
-// X-sweep kernel choice: 0 automatic, 1 ring in LDS, 2 tiles in LDS, 3 one
-// wave per ring with the cells in registers (rings of 256 cells), 4 tiles of
-// one wave each with the cells in registers
+// X-sweep form: 0 (and 1) automatic, 2 tiles of g_xtile cells, 3 one wave per
+// ring on rings of 256 cells, 4 tiles of 256 cells
 static int g_xmode = 0;
-// ring X sweep: 1 two workgroups per ring (half of the quantities each), 0
-// one; -1 automatic
+static int g_xtile = 128;
+// X sweep's quantities: 1 dealt to several waves, two each, 0 one wave, -1
+// automatic
 static int g_xsplit = -1;
 // CFL kernel form, bit 0: ring minima to an array and a one-workgroup
 // second MIN pass (else one atomic MIN per ring); bit 1: the ring sums of
@@ -2669,7 +2237,7 @@ static int finish_step(f3d_hip_ctx* ctx, Scratch* S, double dt, int end_of_step,
 
 // momenta and the Z (3-D) and Y sweeps of every fluid into its transport set
 // (2-D: one Y-sweep launch over the fluids; 3-D: one pair of launches per fluid)
-// vm (2-D only): the X sweep's VxMed pass rides in the Y sweep's launch
+// vm: the X sweep's VxMed pass rides in the Y (2-D) or Z (3-D) sweep's launch
 static int yz_sweeps(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* fl, const TSet* tl,
                      const VmTab* vm = nullptr) {
   const dmesh& m = S->m;
@@ -2692,9 +2260,20 @@ static int yz_sweeps(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* 
       // eight separate buffers: six Z-swept momenta, the Z-swept density and energy
       real* const* Z = &S->f[FS_Z0];
       dim3 gz((m.nx + BXF - 1) / BXF, (m.sy - 2) * sp, (m.nz + rz - 1) / rz);
+      const int nvm = vm ? m.ny * m.nz : 0;
+      const dim3 g1(nvm + gz.x * gz.y * gz.z);
+      const int ad = (ctx->ph.eos == 2);
       f3d_stage_begin(ctx, F3D_ST_SWEEP_Z);
-      FDISPATCH_ADS(ctx, kf_sweep_z, gz, rdt, f.Density, f.Vx_temp, f.Vy_temp, f.Vz_temp, f.Energy, Z[6], Z[0], Z[1],
-                    Z[2], Z[3], Z[4], Z[5], Z[7], rz, of);
+#define SWZ(G_, AD_, SP_)                                                                                         \
+  hipLaunchKernelGGL((kf_sweep_z<G_, AD_, SP_>), g1, dim3(BXF), 0, ctx->stream, m, rdt, f.Density, f.Vx_temp, f.Vy_temp, \
+                     f.Vz_temp, f.Energy, Z[6], Z[0], Z[1], Z[2], Z[3], Z[4], Z[5], Z[7], rz, of,                 \
+                     vm ? vm->vxmed[q] : nullptr, nvm, gz)
+#define SWZ_G(G_) \
+  do { if (ad) { if (split) SWZ(G_, 1, 1); else SWZ(G_, 1, 0); } else { if (split) SWZ(G_, 0, 1); else SWZ(G_, 0, 0); } } while (0)
+      if (m.geom == SPH) SWZ_G(SPH); else SWZ_G(CYL);
+#undef SWZ_G
+#undef SWZ
+      F3D_LAUNCH_CHECK(ctx);
       f3d_stage_end(ctx, F3D_ST_SWEEP_Z);
       dim3 gy((m.nx + BXF - 1) / BXF, ((m.ny + ry - 1) / ry) * sp, m.nz);
       f3d_stage_begin(ctx, F3D_ST_SWEEP_Y);
@@ -2740,7 +2319,6 @@ static int yz_sweeps(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* 
 static int x_vmed(f3d_hip_ctx* ctx, Scratch* S, int nf, const RF* f, const TSet* t, hipStream_t st) {
   const dmesh& m = S->m;
   const int nrings = m.ny * (m.dimz ? m.nz : 1);
-  F3D_REQUIRE(ctx, (size_t)m.nx * sizeof(double) <= 64 * 1024, "ring too long for the VxMed pass");
   F3D_REQUIRE(ctx, nf >= 1 && nf <= 8, "VxMed pass: 1 to 8 fluids");
   VmTab T;
   memset(&T, 0, sizeof(T));
@@ -2767,57 +2345,11 @@ static int x_vmed(f3d_hip_ctx* ctx, Scratch* S, int nf, const RF* f, const TSet*
   return 0;
 }
 
-// tile width of the tiled X sweep (cells per workgroup): 64, 128 or 256
-static int g_xtile = 128;
-
-// Where the X sweep's VxMed comes from: 0 = the ring kernel's own sum,
-// 1 = kf_vmed on the side stream, overlapping the Z/Y sweeps, 2 = kf_vmed on
-// the stream just before the X sweep; -1 = chosen here.  The tiled sweep
-// always takes it from kf_vmed.  Measured on MI355X: below about four ring
-// workgroups per CU the ring kernel's own sum costs least; above, the pass
-// pays, on the stream for short rings (a sum of <= 512 terms takes under
-// 3 us) and on the side stream for long ones, whose sums it hides.
+// Where the X sweep by tiles takes VxMed from: 1 = kf_vmed on the side stream,
+// overlapping the Z/Y sweeps, 2 = kf_vmed on the stream just before the X sweep,
+// else (and with 1 unless f3d_fused_set_y2v(0)) the pass in the Y sweep's launch
+// (2-D) or the Z sweep's (3-D).  A wave that holds a whole ring sums it itself.
 static int g_xvmed = -1;
-static int x_vmed_form(const dmesh& m, int nf, bool tiles) {
-  const int nrings = m.ny * (m.dimz ? m.nz : 1);
-  if (tiles) return (g_xvmed == 2) ? 2 : 1;
-  if (g_xvmed >= 0) return g_xvmed;
-  if (nrings * nf < 1024) return 0;
-  return m.nx <= 512 ? 2 : 1;
-}
-
-// X sweep by tiles (rings longer than the LDS ring kernel holds), once
-// VxMed of every ring is known.
-static int x_sweep_tiled(f3d_hip_ctx* ctx, Scratch* S, double dt, const RF& f, const TSet& t) {
-  const dmesh& m = S->m;
-  const real of = (real)ctx->ph.OMEGAFRAME;
-  real* const* XM = t.xm;
-  const int nrings = m.ny * (m.dimz ? m.nz : 1);
-  const int ad = (ctx->ph.eos == 2);
-  const int T = g_xtile;
-  F3D_REQUIRE(ctx, m.nx >= 12, "the tiled X sweep needs at least 12 cells per ring");
-  f3d_stage_begin(ctx, F3D_ST_SWEEP_X);
-  dim3 g((m.nx + x_tile_cells(T) - 1) / x_tile_cells(T), nrings);
-#define XTILE1(G_, DZ_, AD_, T_)                                                                                \
-  hipLaunchKernelGGL((kf_sweep_x_tile<G_, DZ_, AD_, T_>), g, dim3(T_), 0, ctx->stream, m, dt, t.rhoy, f.Vx_temp, \
-                     t.m[0], t.m[1], t.m[2], t.m[3], t.m[4], t.m[5], t.ey, f.Energy, t.rhox, f.Vx, XM[0], XM[1],  \
-                     XM[2], XM[3], t.vxmed, t.nshift, of, ctx->ph.fargo)
-#define XTILE(G_, DZ_, AD_) \
-  do { if (T == 64) XTILE1(G_, DZ_, AD_, 64); else if (T == 256) XTILE1(G_, DZ_, AD_, 256); \
-       else XTILE1(G_, DZ_, AD_, 128); } while (0)
-  if (m.geom == SPH) {
-    if (m.dimz) { if (ad) XTILE(SPH, 1, 1); else XTILE(SPH, 1, 0); }
-    else { if (ad) XTILE(SPH, 0, 1); else XTILE(SPH, 0, 0); }
-  } else {
-    if (m.dimz) { if (ad) XTILE(CYL, 1, 1); else XTILE(CYL, 1, 0); }
-    else { if (ad) XTILE(CYL, 0, 1); else XTILE(CYL, 0, 0); }
-  }
-#undef XTILE
-#undef XTILE1
-  F3D_LAUNCH_CHECK(ctx);
-  f3d_stage_end(ctx, F3D_ST_SWEEP_X);
-  return 0;
-}
 
 // the side stream and its events, created on first use
 static int side_stream(f3d_hip_ctx* ctx) {
@@ -2829,220 +2361,86 @@ static int side_stream(f3d_hip_ctx* ctx) {
   return 0;
 }
 
-// Ring X sweep of nf fluids in one launch: nf consecutive blocks of
-// per_fluid workgroups, each block reading its fluid's arrays from the table.
-struct XTab {
-  const real* rho_in[8];
-  const real* vxt[8];
-  const real* q[8][6];
-  const real* e_in[8];
-  real* e_out[8];
-  real* rho_out[8];
-  real* vx_out[8];
-  real* qo[8][4];
-  double* vxmed[8];
-  int* nshift[8];
+// The form of the X sweep: cells per lane, whole rings or tiles, tiles per ring
+// and the groups the quantities are dealt to.  Measured on MI355X, FP64:
+//   - a wave of 1, 2, 3 or 4 cells per lane takes 2.4, 5.2, 8.2, 10.7 ns of the
+//     filled GPU (FP32: 1.34, 2.55, 4.06, 6.0), so the cheapest cover of a ring
+//     wins: rings of 4096 cells 4 per lane (adiabatic 4096x1024 in us: 196, 193,
+//     196, 189 for 1 .. 4 per lane), of 1024 cells 2 (five fluids 1024x512:
+//     102, 96, 102, 109), of 500 cells 3 (3-D 500x150x45: 187, 196, 186, 225);
+//   - below 2048 waves of one cell per lane the launch is a chain of latencies:
+//     one cell per lane and two quantities per wave (384x128: 8.5 us, 9.3 with
+//     all quantities in a wave, 13.4 with four cells per lane; 96x48: 7.2, 8.4,
+//     12.8);
+//   - many rings of 256 cells go whole, the sum of VxMed in the wave (3-D
+//     256x96x32: 42 us against 45 by tiles of one cell per lane and 7 for
+//     their sums).
+struct XForm {
+  int cpt, ring, ngrp, ntiles;
 };
-
-// One cell per thread, VxMed from the pass, no energy: 6 waves per SIMD fit
-// in 78 registers without spills (measured on the 3-D disk: 63.1 -> 61.0 us;
-// the energy form would spill)
-template <int G, int DZ, int AD, int CPT, int SPLIT, int VPRE>
-__global__ void __launch_bounds__(CPT == 2 ? 512 : 256, (CPT == 1 && VPRE && !AD) ? 6 : 1) kf_sweep_xr_fluids(dmesh m, double dt64, XTab T, int per_fluid,
-                                                           real omegaframe, int fargo) {
-  const int lin = xcd_linear();
-  const int fl = lin / per_fluid, b = lin % per_fluid;
-  real* qout[4] = {T.qo[fl][0], T.qo[fl][1], T.qo[fl][2], T.qo[fl][3]};
-  if (!SPLIT) {
-    xsweep_ring<G, DZ, AD, CPT, 0, VPRE>(m, b, dt64, T.rho_in[fl], T.vxt[fl], T.q[fl], T.e_in[fl], T.e_out[fl],
-                                   T.rho_out[fl], T.vx_out[fl], qout, T.vxmed[fl], T.nshift[fl], omegaframe, fargo);
-  } else if ((b & 1) == 0) {
-    xsweep_ring<G, DZ, AD, CPT, 1, VPRE>(m, b >> 1, dt64, T.rho_in[fl], T.vxt[fl], T.q[fl], T.e_in[fl], T.e_out[fl],
-                                   T.rho_out[fl], T.vx_out[fl], qout, T.vxmed[fl], T.nshift[fl], omegaframe, fargo);
-  } else {
-    xsweep_ring<G, DZ, AD, CPT, 2, VPRE>(m, b >> 1, dt64, T.rho_in[fl], T.vxt[fl], T.q[fl], T.e_in[fl], T.e_out[fl],
-                                   T.rho_out[fl], T.vx_out[fl], qout, T.vxmed[fl], T.nshift[fl], omegaframe, fargo);
+static XForm x_form(const f3d_hip_ctx* ctx, const dmesh& m, int nf) {
+  const long rings = (long)m.ny * (m.dimz ? m.nz : 1) * nf;
+  const int nq = (m.dimz ? 6 : 4) + (ctx->ph.eos == 2);
+  auto tiles = [&](int cpt) { return (m.nx + x_tile_out(cpt) - 1) / x_tile_out(cpt); };
+  const bool any = g_xmode == 0 || g_xmode == 1;
+  XForm x;
+  x.ring = m.nx == 256 && (g_xmode == 3 || (any && rings >= 2048));
+  x.cpt = g_xmode == 2 ? g_xtile / 64 : 4;
+  x.ngrp = 1;
+  if (!x.ring && (any || g_xmode == 3)) {
+    if (rings * tiles(1) < 2048) {
+      x.cpt = 1;
+      x.ngrp = nq / 2;
+    } else {
+      const double cost[2][5] = {{0, 2.4, 5.2, 8.2, 10.7}, {0, 1.34, 2.55, 4.06, 6.0}};
+      for (int c = 1; c <= 3; c++)
+        if (tiles(c) * cost[kPrec][c] < tiles(x.cpt) * cost[kPrec][x.cpt]) x.cpt = c;
+    }
   }
+  if (g_xsplit >= 0) x.ngrp = g_xsplit ? nq / 2 : 1;
+  if (x.ring) x.ngrp = 1;
+  x.ntiles = x.ring ? 1 : tiles(x.cpt);
+  return x;
 }
 
-// one wave per ring and fluid; blocks [f*nrings, (f+1)*nrings) take fluid f
-template <int G, int DZ, int AD, int CPT>
-__global__ void __launch_bounds__(64, 2) kf_sweep_xw(dmesh m, double dt64, XTab T, int nrings, real omegaframe,
-                                                  int fargo) {
-  const int lin = xcd_linear();
-  const int fl = lin / nrings, ring = lin % nrings;
-  real* qout[4] = {T.qo[fl][0], T.qo[fl][1], T.qo[fl][2], T.qo[fl][3]};
-  xsweep_wave<G, DZ, AD, CPT>(m, ring, dt64, T.rho_in[fl], T.vxt[fl], T.q[fl], T.e_in[fl], T.e_out[fl],
-                              T.rho_out[fl], T.vx_out[fl], qout, T.vxmed[fl], T.nshift[fl], omegaframe, fargo);
-}
-
-// tiles of long rings, one wave each (xsweep_wave with TILE = 1, four cells
-// per lane: 244 cells updated per tile); blocks [f*nrings*ntiles, ...) take
-// fluid f, a ring's tiles consecutive
-template <int G, int DZ, int AD>
-__global__ void __launch_bounds__(64, 2) kf_sweep_xtw(dmesh m, double dt64, XTab T, int nrings, int ntiles,
-                                                      real omegaframe, int fargo) {
-  const int lin = xcd_linear();
-  const int per = nrings * ntiles;
-  const int fl = lin / per, rt = lin % per;
-  real* qout[4] = {T.qo[fl][0], T.qo[fl][1], T.qo[fl][2], T.qo[fl][3]};
-  xsweep_wave<G, DZ, AD, 4, 1>(m, rt / ntiles, dt64, T.rho_in[fl], T.vxt[fl], T.q[fl], T.e_in[fl], T.e_out[fl],
-                               T.rho_out[fl], T.vx_out[fl], qout, T.vxmed[fl], T.nshift[fl], omegaframe, fargo,
-                               rt % ntiles);
-}
-
-// ring X sweep form: the split (two workgroups per ring) and its LDS bytes
-static void x_ring_form(const f3d_hip_ctx* ctx, const dmesh& m, int* split, size_t* shx) {
-  const int ad = (ctx->ph.eos == 2);
-  const int nq = (m.dimz ? 6 : 4) + ad, na = m.dimz ? 3 : 2;
-  // measured on MI355X: the split pays while a thread owns one cell of the
-  // ring or two of a short one (nx <= 512); beyond, its extra density work
-  // costs more than the occupancy it gains
-  *split = (g_xsplit < 0) ? (m.nx <= 512 ? 1 : 0) : g_xsplit;
-  *shx = *split ? xsweep_ring_lds(m.nx, na > nq - na ? na : nq - na) : xsweep_ring_lds(m.nx, nq);
-}
-
-// true when the ring X sweep runs (the ring fits in LDS and no tiles are asked for)
-static bool x_ring_fits(const f3d_hip_ctx* ctx, Scratch* S) {
-  int split;
-  size_t shx;
-  x_ring_form(ctx, S->m, &split, &shx);
-  const bool fits = shx <= 160 * 1024 && S->m.nx <= 1024;
-  return g_xmode == 1 || ((g_xmode == 0 || g_xmode == 3) && fits);
-}
-
-// the ring X sweeps' table of every fluid's arrays
-static void xtab_fill(XTab* T, int nf, const RF* f, const TSet* t) {
-  memset(T, 0, sizeof(*T));
-  for (int k = 0; k < nf; k++) {
-    T->rho_in[k] = t[k].rhoy; T->vxt[k] = f[k].Vx_temp;
-    for (int q = 0; q < 6; q++) T->q[k][q] = t[k].m[q];
-    T->e_in[k] = t[k].ey; T->e_out[k] = f[k].Energy; T->rho_out[k] = t[k].rhox; T->vx_out[k] = f[k].Vx;
-    for (int q = 0; q < 4; q++) T->qo[k][q] = t[k].xm[q];
-    T->vxmed[k] = t[k].vxmed; T->nshift[k] = t[k].nshift;
-  }
-}
-
-// The one-wave ring X sweep (kf_sweep_xw): rings of 256 cells (four per
-// lane; longer rings need more registers than two waves per SIMD leave),
-// chosen automatically from 2048 rings x fluids on (enough waves to fill the
-// GPU), or asked for with f3d_fused_set_xmode(3).
-static bool x_wave_form(const dmesh& m, int nf) {
-  if (m.nx != 256) return false;
-  if (g_xmode == 3) return true;
-  if (g_xmode != 0) return false;
-  return (long)m.ny * (m.dimz ? m.nz : 1) * nf >= 2048;
-}
-
-static int x_sweep_wave(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* f, const TSet* t) {
+// the X sweep of nf fluids in one launch
+static int x_sweep(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* f, const TSet* t, const XForm& x) {
   const dmesh& m = S->m;
   const real of = (real)ctx->ph.OMEGAFRAME;
-  const int ad = (ctx->ph.eos == 2);
-  F3D_REQUIRE(ctx, m.nx == 256, "one-wave X sweep: rings of 256 cells");
+  const int ad = (ctx->ph.eos == 2), nm = m.dimz ? 6 : 4, nrings = m.ny * (m.dimz ? m.nz : 1);
   F3D_REQUIRE(ctx, nf >= 1 && nf <= 8, "X sweep: 1 to 8 fluids");
-  const int nrings = m.ny * (m.dimz ? m.nz : 1);
   XTab T;
-  xtab_fill(&T, nf, f, t);
-  f3d_stage_begin(ctx, F3D_ST_SWEEP_X);
-#define XW0(G_, DZ_, AD_, CPT_)                                                                             \
-  hipLaunchKernelGGL((kf_sweep_xw<G_, DZ_, AD_, CPT_>), dim3(nrings * nf), dim3(64), 0, ctx->stream, m, dt, T, \
-                     nrings, of, ctx->ph.fargo)
-#define XW(G_, DZ_) \
-  do { if (ad) XW0(G_, DZ_, 1, 4); else XW0(G_, DZ_, 0, 4); } while (0)
-  if (m.geom == SPH) {
-    if (m.dimz) XW(SPH, 1); else XW(SPH, 0);
-  } else {
-    if (m.dimz) XW(CYL, 1); else XW(CYL, 0);
+  memset(&T, 0, sizeof(T));
+  for (int q = 0; q < nf; q++) {
+    XFluid& X = T.f[q];
+    X.rho_in = t[q].rhoy; X.vxt = f[q].Vx_temp; X.rho_out = t[q].rhox; X.vx_out = f[q].Vx;
+    X.vxmed = t[q].vxmed; X.nshift = t[q].nshift;
+    for (int c = 0; c < nm; c++) {
+      X.in[c] = t[q].m[c];
+      X.out[c] = c < 2 ? nullptr : t[q].xm[c - 2];
+    }
+    X.in[nm] = t[q].ey;
+    X.out[nm] = f[q].Energy;
   }
-#undef XW
-#undef XW0
-  F3D_LAUNCH_CHECK(ctx);
-  f3d_stage_end(ctx, F3D_ST_SWEEP_X);
-  return 0;
-}
-
-// Ring X sweep of nf fluids in one launch.
-// Tiles of one wave each (kf_sweep_xtw) for the rings the LDS ring kernel
-// does not take: automatic in 2-D (the 3-D forms need more registers than
-// two waves per SIMD leave and spill), or asked for with
-// f3d_fused_set_xmode(4).
-static bool x_wtile_form(const dmesh& m) { return g_xmode == 4 || (g_xmode == 0 && !m.dimz); }
-// ... and in place of the LDS ring kernel where the tiles make enough waves:
-// measured on MI355X, gas + 4 dust 1024x512 (12,800 waves) FP64 step 0.442 ->
-// 0.383 ms, FP32 0.299 -> 0.284 ms; the 384x128 disk (256 waves) 0.064 ->
-// 0.091 ms, so from 2048 waves on, in 2-D
-static bool x_wtile_pays(const dmesh& m, int nf) {
-  if (g_xmode == 4) return true;
-  if (g_xmode != 0 || m.dimz) return false;
-  const long ntiles = (m.nx + 243) / 244;
-  return (long)m.ny * ntiles * nf >= 2048;
-}
-
-static int x_sweep_wtiles(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* f, const TSet* t) {
-  const dmesh& m = S->m;
-  const real of = (real)ctx->ph.OMEGAFRAME;
-  const int ad = (ctx->ph.eos == 2);
-  F3D_REQUIRE(ctx, nf >= 1 && nf <= 8, "X sweep: 1 to 8 fluids");
-  const int nrings = m.ny * (m.dimz ? m.nz : 1);
-  const int ntiles = (m.nx + 243) / 244;
-  XTab T;
-  xtab_fill(&T, nf, f, t);
   f3d_stage_begin(ctx, F3D_ST_SWEEP_X);
-#define XTW(G_, DZ_, AD_)                                                                                     \
-  hipLaunchKernelGGL((kf_sweep_xtw<G_, DZ_, AD_>), dim3(nrings * ntiles * nf), dim3(64), 0, ctx->stream, m, dt, \
-                     T, nrings, ntiles, of, ctx->ph.fargo)
-#define XTW_G(G_, DZ_) \
-  do { if (ad) XTW(G_, DZ_, 1); else XTW(G_, DZ_, 0); } while (0)
+#define XS(G_, DZ_, CPT_, R_)                                                                                  \
+  hipLaunchKernelGGL((kf_sweep_x<G_, DZ_, CPT_, R_>), dim3(nrings * nf * x.ntiles * x.ngrp), dim3(64), 0,     \
+                     ctx->stream, m, dt, T, nrings, x.ntiles, x.ngrp, nm + ad, of, ctx->ph.fargo)
+#define XS_G(G_, DZ_)                      \
+  do {                                     \
+    if (x.ring) XS(G_, DZ_, 4, 1);         \
+    else if (x.cpt == 1) XS(G_, DZ_, 1, 0); \
+    else if (x.cpt == 2) XS(G_, DZ_, 2, 0); \
+    else if (x.cpt == 3) XS(G_, DZ_, 3, 0); \
+    else XS(G_, DZ_, 4, 0);                \
+  } while (0)
   if (m.geom == SPH) {
-    if (m.dimz) XTW_G(SPH, 1); else XTW_G(SPH, 0);
+    if (m.dimz) XS_G(SPH, 1); else XS_G(SPH, 0);
   } else {
-    if (m.dimz) XTW_G(CYL, 1); else XTW_G(CYL, 0);
+    if (m.dimz) XS_G(CYL, 1); else XS_G(CYL, 0);
   }
-#undef XTW_G
-#undef XTW
-  F3D_LAUNCH_CHECK(ctx);
-  f3d_stage_end(ctx, F3D_ST_SWEEP_X);
-  return 0;
-}
-
-static int x_sweep_ring(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* f, const TSet* t, int vpre) {
-  const dmesh& m = S->m;
-  const real of = (real)ctx->ph.OMEGAFRAME;
-  const int ad = (ctx->ph.eos == 2);
-  int split;
-  size_t shx;
-  x_ring_form(ctx, m, &split, &shx);
-  F3D_REQUIRE(ctx, shx <= 160 * 1024 && m.nx <= 1024, "ring too long for the LDS X sweep");
-  F3D_REQUIRE(ctx, nf >= 1 && nf <= 8, "X sweep: 1 to 8 fluids");
-  // one cell per thread up to 256 cells, else two (up to 512 threads)
-  const int cpt = (m.nx <= 256) ? 1 : 2;
-  const int nthreads = (((m.nx + cpt - 1) / cpt + 63) / 64) * 64;
-  const int per = m.ny * (m.dimz ? m.nz : 1) * (split ? 2 : 1);
-  XTab T;
-  xtab_fill(&T, nf, f, t);
-  dim3 gx(per * nf);
-  f3d_stage_begin(ctx, F3D_ST_SWEEP_X);
-#define XSWEEP0(G_, DZ_, AD_, CPT_, SP_, VP_)                                                                  \
-  hipLaunchKernelGGL((kf_sweep_xr_fluids<G_, DZ_, AD_, CPT_, SP_, VP_>), gx, dim3(nthreads), shx, ctx->stream, m, \
-                     dt, T, per, of, ctx->ph.fargo)
-#define XSWEEP1(G_, DZ_, AD_, CPT_, SP_) \
-  do { if (vpre) XSWEEP0(G_, DZ_, AD_, CPT_, SP_, 1); else XSWEEP0(G_, DZ_, AD_, CPT_, SP_, 0); } while (0)
-#define XSWEEP2(G_, DZ_, AD_, CPT_) \
-  do { if (split) XSWEEP1(G_, DZ_, AD_, CPT_, 1); else XSWEEP1(G_, DZ_, AD_, CPT_, 0); } while (0)
-#define XSWEEP(G_, DZ_, CPT_) \
-  do { if (ad) XSWEEP2(G_, DZ_, 1, CPT_); else XSWEEP2(G_, DZ_, 0, CPT_); } while (0)
-#define XSWEEP_G(G_, DZ_) \
-  do { if (cpt == 1) XSWEEP(G_, DZ_, 1); else XSWEEP(G_, DZ_, 2); } while (0)
-  if (m.geom == SPH) {
-    if (m.dimz) XSWEEP_G(SPH, 1); else XSWEEP_G(SPH, 0);
-  } else {
-    if (m.dimz) XSWEEP_G(CYL, 1); else XSWEEP_G(CYL, 0);
-  }
-#undef XSWEEP_G
-#undef XSWEEP0
-#undef XSWEEP1
-#undef XSWEEP2
-#undef XSWEEP
+#undef XS_G
+#undef XS
   F3D_LAUNCH_CHECK(ctx);
   f3d_stage_end(ctx, F3D_ST_SWEEP_X);
   return 0;
@@ -3063,14 +2461,11 @@ static int transport_fluids(f3d_hip_ctx* ctx, double dt, int nf, const f3d_field
     f[k] = fl ? rfields_of(fl[k], ctx->f) : rfields(ctx);
     if (tset_of(ctx, S, f[k], k, nf, &t[k])) return -1;
   }
-  const bool wave = x_wave_form(S->m, nf);
-  const bool tiles = !wave && !x_ring_fits(ctx, S);
-  const bool wtiles = !wave && (tiles ? x_wtile_form(S->m) : x_wtile_pays(S->m, nf));
-  // the one-wave sweep sums VxMed itself; the tiled ones take it from the pass
-  const int vpre = (ctx->ph.fargo && !wave) ? x_vmed_form(S->m, nf, tiles || wtiles) : 0;
-  // 2-D: the pass in the Y sweep's launch instead of on the second stream
-  const bool vin = vpre == 1 && !S->m.dimz && g_y2v != 0 && (g_vmed_terms < 0 || g_vmed_terms == 8) &&
-                   (size_t)S->m.nx * sizeof(double) <= 64 * 1024;
+  const XForm x = x_form(ctx, S->m, nf);
+  // a wave that holds a whole ring sums VxMed itself, tiles take it from the pass
+  const int vpre = (ctx->ph.fargo && !x.ring) ? (g_xvmed == 2 ? 2 : 1) : 0;
+  // the pass in the Y or Z sweep's launch instead of on the second stream
+  const bool vin = vpre == 1 && g_y2v != 0 && (g_vmed_terms < 0 || g_vmed_terms == 8);
   VmTab VT;
   memset(&VT, 0, sizeof(VT));
   for (int q = 0; q < nf; q++) {
@@ -3089,16 +2484,7 @@ static int transport_fluids(f3d_hip_ctx* ctx, double dt, int nf, const f3d_field
   if (yz_sweeps(ctx, S, dt, nf, f, t, vin ? &VT : nullptr)) return -1;
   if (vpre == 1 && !vin) F3D_CHECK(ctx, hipStreamWaitEvent(ctx->stream, ctx->side_done, 0));
   if (vpre == 2 && x_vmed(ctx, S, nf, f, t, ctx->stream)) return -1;
-  if (wave) {
-    if (x_sweep_wave(ctx, S, dt, nf, f, t)) return -1;
-  } else if (wtiles) {
-    if (x_sweep_wtiles(ctx, S, dt, nf, f, t)) return -1;
-  } else if (!tiles) {
-    if (x_sweep_ring(ctx, S, dt, nf, f, t, vpre != 0)) return -1;
-  } else {
-    for (int k = 0; k < nf; k++)
-      if (x_sweep_tiled(ctx, S, dt, f[k], t[k])) return -1;
-  }
+  if (x_sweep(ctx, S, dt, nf, f, t, x)) return -1;
   if (finish_step(ctx, S, dt, end_of_step, nf, f, t)) return -1;
   return 0;
 }
