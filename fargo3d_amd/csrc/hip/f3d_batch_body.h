@@ -324,12 +324,13 @@ __global__ void __launch_bounds__(BXF) kb_bound(const BInst* I, const int* off, 
              in.cs, in.b0, in.b1, in.ydexp0, in.ydexp1);
 }
 
-__global__ void __launch_bounds__(BXF) kb_sweep_y(const BInst* I, const int* off, int n, int rows_per) {
+template <int R>
+__global__ void __launch_bounds__(BXF) kb_sweep_y(const BInst* I, const int* off, int n) {
   const int ii = find_inst(off, n, blockIdx.x);
   const BInst& in = I[ii];
   const int gx = (in.m.nx + BXF - 1) / BXF;
-  kd_sweep_y2<CYL, 0, 0>(local2(blockIdx.x - off[ii], gx), in.m, (real)in.clk[0], in.rho, in.vxt, in.vyt, in.cs,
-                         in.rhoy, in.mpx, in.mmx, in.mpy, in.mmy, in.ey, rows_per, in.of);
+  kd_sweep_y2<CYL, 0, R>(local2(blockIdx.x - off[ii], gx), in.m, (real)in.clk[0], in.rho, in.vxt, in.vyt, in.cs,
+                         in.rhoy, in.mpx, in.mmx, in.mpy, in.mmy, in.ey, in.of);
 }
 
 // one wave per ring, 8 terms per lane (the instances' rings hold 256 to a few
@@ -421,7 +422,8 @@ static int batch_layout(f3d_batch* B) {
     c[BK_VMED][i] = m.ny;
     c[BK_FIN][i] = gx * m.ny;
     c[BK_POT][i] = B->has_ps[i] ? gx * m.sy : 0;
-    swy[i] = gx * ((m.ny + B->rows_y - 1) / B->rows_y);
+    const int ry = column_form(B->rows_y);
+    swy[i] = gx * ((m.ny + ry - 1) / ry) * (ry == 1 ? 2 : 1);
     xt[i] = ((m.nx + x_tile_out(B->tile / 64) - 1) / x_tile_out(B->tile / 64)) * m.ny;
   }
   for (int k = 0; k < BK_N; k++)
@@ -445,7 +447,10 @@ static void batch_launch(f3d_batch* B) {
   hipLaunchKernelGGL(kb_src_a, dim3(B->total[BK_SRCA]), dim3(BXF), 0, s, B->dI, B->doff[BK_SRCA], n);
   hipLaunchKernelGGL(kb_src_b, dim3(B->total[BK_SRCB]), dim3(BXF), 0, s, B->dI, B->doff[BK_SRCB], n);
   hipLaunchKernelGGL(kb_bound, dim3(B->total[BK_BND]), dim3(BXF), 0, s, B->dI, B->doff[BK_BND], n, 1);
-  hipLaunchKernelGGL(kb_sweep_y, dim3(B->swy_total), dim3(BXF), 0, s, B->dI, B->dswy, n, B->rows_y);
+  const int ry = column_form(B->rows_y);
+  if (ry == 4) hipLaunchKernelGGL(kb_sweep_y<4>, dim3(B->swy_total), dim3(BXF), 0, s, B->dI, B->dswy, n);
+  else if (ry == 2) hipLaunchKernelGGL(kb_sweep_y<2>, dim3(B->swy_total), dim3(BXF), 0, s, B->dI, B->dswy, n);
+  else hipLaunchKernelGGL(kb_sweep_y<1>, dim3(B->swy_total), dim3(BXF), 0, s, B->dI, B->dswy, n);
   hipLaunchKernelGGL(kb_vmed, dim3(B->total[BK_VMED]), dim3(64), 0, s, B->dI,
                      B->doff[BK_VMED], n);
   if (B->tile == 64) hipLaunchKernelGGL(kb_sweep_x<1>, dim3(B->xt_total), dim3(64), 0, s, B->dI, B->dxt, n);

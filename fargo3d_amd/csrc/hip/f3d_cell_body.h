@@ -451,26 +451,14 @@ __device__ __forceinline__ void potential_cells(const dmesh& m, int i0, int di, 
 }
 
 // ---------------------------------------------------------------- momenta / new velocities
-// src/momenta_x.c:76-84
+// src/momenta_x.c:76-84: the momentum of velocity v (a cell's own for Mmx, its
+// right neighbour's for Mpx).  Precision form: the deviation from rho l0, rho v'
+// r with the FP64 radius.
 template <int G>
-__device__ __forceinline__ void momenta_x(const dmesh& m, int i, int j, int k, real rho, real vx, real vxp,
-                                          real omegaframe, real& mmx, real& mpx) {
-  if constexpr (kFix64) {
-    // deviations from rho l0: rho vx' r (vx, vxp are deviations), with the
-    // FP64 radius
-    const double rcyl = rcyl64<G>(m, j, k);
-    mmx = (real)((double)vx * rcyl * (double)rho);
-    mpx = (real)((double)vxp * rcyl * (double)rho);
-    return;
-  }
-  if (G == SPH) {
-    real rcyl = m.ymed[j] * m.sinzmed[k];
-    mmx = (vx + rcyl * omegaframe) * rcyl * rho;
-    mpx = (vxp + rcyl * omegaframe) * rcyl * rho;
-  } else {
-    mmx = (vx + m.ymed[j] * omegaframe) * m.ymed[j] * rho;
-    mpx = (vxp + m.ymed[j] * omegaframe) * m.ymed[j] * rho;
-  }
+__device__ __forceinline__ real momentum_x(const dmesh& m, int j, int k, real rho, real v, real omegaframe) {
+  if constexpr (kFix64) return (real)((double)v * rcyl64<G>(m, j, k) * (double)rho);
+  const real rcyl = G == SPH ? m.ymed[j] * m.sinzmed[k] : m.ymed[j];
+  return (v + rcyl * omegaframe) * rcyl * rho;
 }
 
 // src/newvel_x.c:78-86
@@ -567,30 +555,6 @@ __device__ __forceinline__ real flux_y(const dmesh& m, int i, int j, int k, real
 }
 __device__ __forceinline__ real flux_z(const dmesh& m, int i, int j, int k, real dt, real a, real b) {
   return mul_invvol(m, (mul_surfz(m, a, i, j, k) - mul_surfz(m, b, i, j, k + 1)) * dt, i, j, k);
-}
-// The mesh factors of one cell's Y or Z flux difference, loaded once for
-// all its quantities: (a SurfA - b SurfB) dt InvVol with Surf = (. * fj) * fk
-// * Sxi[i] on either face, in the association of mul_surfy/mul_surfz and
-// mul_invvol.
-struct FluxMesh {
-  real aj, ak, bj, bk, si, iv;
-};
-__device__ __forceinline__ FluxMesh flux_y_mesh(const dmesh& m, int i, int j, int k) {
-  return FluxMesh{m.syj[j], m.syk[k], m.syj[j + 1], m.syk[k], m.sxi[i], m.invvj[j]};
-}
-__device__ __forceinline__ FluxMesh flux_z_mesh(const dmesh& m, int i, int j, int k) {
-  return FluxMesh{m.szj[j], m.szk[k], m.szj[j], m.szk[k + 1], m.sxi[i], m.invvj[j]};
-}
-// flux_y / flux_z below from those factors, with the InvVol divisor V
-__device__ __forceinline__ real flux_yz(const FluxMesh& F, real dt, real a, real b, const Recip& V) {
-  return rdiv(((((a * F.aj) * F.ak) * F.si - ((b * F.bj) * F.bk) * F.si) * dt) * F.iv, V);
-}
-// the same with the cell's InvVol divisor shared by its quantities
-__device__ __forceinline__ real flux_y(const dmesh& m, int i, int j, int k, real dt, real a, real b, const Recip& V) {
-  return mul_invvol(m, (mul_surfy(m, a, i, j, k) - mul_surfy(m, b, i, j + 1, k)) * dt, j, V);
-}
-__device__ __forceinline__ real flux_z(const dmesh& m, int i, int j, int k, real dt, real a, real b, const Recip& V) {
-  return mul_invvol(m, (mul_surfz(m, a, i, j, k) - mul_surfz(m, b, i, j, k + 1)) * dt, j, V);
 }
 
 // ---------------------------------------------------------------- cfl (src/cfl.c:174-253)

@@ -41,6 +41,10 @@ struct dmesh {
   // precision form only: V0(j,k), the FP64 ring profile the azimuthal
   // velocities are stored as deviations from (index j + k*sy); null in FP64
   const double* vb;
+  // the fused stages: zone sizes of the rows in Y, zy[j], and in Z, zz[j + k*sy],
+  // and their reciprocals for rdiv(), for kernels that read them through the
+  // scalar cache (null until the stages' scratch exists)
+  const mreal *zy, *rzy, *zz, *rzz;
 };
 
 __device__ __forceinline__ int lxp_of(int l, int i, int nx) { return (i < nx - 1) ? l + 1 : l - (nx - 1); }

@@ -64,6 +64,7 @@ struct Scratch {
   real* ddtemp[8];             // dust diffusion: the new density of fluid f before its copy back
   dmesh m;                     // the build's mesh view
   mreal* mesh_r;               // FP32 build: converted mesh arrays
+  mreal* zones;                // zone sizes and their reciprocals (dmesh zy .. rzz)
   real* bctab_r;               // FP32 build: converted boundary tables
   const real *ymin_dexp, *ymax_dexp, *zmin_dens, *zmax_dens;
 };
@@ -84,6 +85,7 @@ void scratch_free(void* p) {
     if (S->ddtemp[f]) (void)hipFree(S->ddtemp[f]);
   }
   if (S->mesh_r) (void)hipFree(S->mesh_r);
+  if (S->zones) (void)hipFree(S->zones);
   if (S->bctab_r) (void)hipFree(S->bctab_r);
   delete S;
 }
@@ -92,6 +94,22 @@ template <class T>
 __global__ void k_convert(const double* a, T* b, size_t n) {
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) b[t] = (T)a[t];
+}
+
+// zy, rzy (sy each) and zz, rzz (sy*sz each) of the mesh, one after the other
+__global__ void k_zones(dmesh m, mreal* t) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x, n2 = m.sy * m.sz;
+  if (q < m.sy) {
+    const real z = zone_size_y(m, q);
+    t[q] = z;
+    t[m.sy + q] = recip(z).r;
+  }
+  if (q < n2 && m.dimz) {
+    const int j = q % m.sy, k = q / m.sy;
+    const real z = m.geom == SPH ? zone_size_z<SPH>(m, j, k) : zone_size_z<CYL>(m, j, k);
+    t[2 * m.sy + q] = z;
+    t[2 * m.sy + n2 + q] = recip(z).r;
+  }
 }
 
 // The build's view of the handle's mesh: the FP64 build uses the handle's
@@ -133,8 +151,16 @@ int make_mesh(f3d_hip_ctx* ctx, Scratch* S) {
     S->zmin_dens = S->bctab_r + 2 * ny3;
     S->zmax_dens = S->bctab_r + 2 * ny3 + nz3;
   }
-  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return -1;
 #endif
+  dmesh& z = S->m;
+  const size_t n2 = (size_t)z.sy * z.sz;
+  if (hipMalloc(&S->zones, (2 * z.sy + 2 * n2) * sizeof(mreal)) != hipSuccess) return -1;
+  hipLaunchKernelGGL(k_zones, dim3((n2 + 255) / 256), dim3(256), 0, ctx->stream, z, S->zones);
+  z.zy = S->zones;
+  z.rzy = S->zones + z.sy;
+  z.zz = S->zones + 2 * z.sy;
+  z.rzz = z.zz + n2;
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return -1;
   return 0;
 }
 
@@ -648,192 +674,161 @@ __global__ void __launch_bounds__(WG) kf_substep3(dmesh m, real dt, const real* 
 }
 
 // --------------------------------------------------------------- transport
-// One directional van Leer sweep of one column (the Y or Z transport of
-// src/transport.c:81-127): NQ conserved quantities plus the density
-// (index NQ), rows r in [r0, r1).  Per row the quantity q = Q/rho
-// (src/divrho.c:56), the gradient at the lower face (dqm of
-// src/vanleer_y_a.c:63, equal to dqp of the row below), the slope and the
-// upwind face value (src/vanleer_y_b.c:60-65) are each computed once and
-// kept in a window of registers.
+// One directional van Leer sweep of R rows of one column (the Y or Z transport
+// of src/transport.c:81-127), rows r in [r0, min(r0 + R, r1)): the conserved
+// quantities c in [C0, C1) and, with C0 = 0, the density.  Every row the faces
+// read (r0-2 .. r0+R+1) is in registers at once: the density's values,
+// reciprocals and faces first, then one quantity after the other from its loads
+// to its stores, each with q = Q/rho (src/divrho.c:56), the gradient at the lower
+// face (dqm of src/vanleer_y_a.c:63, equal to dqp of the row below), the slope
+// and the upwind face value (src/vanleer_y_b.c:60-65) computed once per row.
+// Rows past r1 + 1 read that row again; rows past r1 are not stored.
+// What bounds it on MI355X is latency and memory together (FP64 issue is half of
+// the time at most).  Marching a thread along the column with two face values,
+// a slope and two rows of q of every quantity in registers made each row wait
+// for the one before, loaded each value twice, and its halo rows had left L2 by
+// then: the Y sweep of 500x150x45 fetched 489 MB, with the rows in registers
+// 224 MB.  Each quantity's loads go out before the arithmetic and the stores of
+// the one before, since loads retire in order behind earlier stores; without
+// that the same sweep takes 112 us.  Marching / this form, us per launch, FP64: Y of
+// 500x150x45 134.5 / 99.2, Z 128.0 / 108.7, Y of 256x96x32 28.2 / 22.6, Z 28.9 /
+// 29.1, 4096x1024 adiabatic 119.8 / 100.7, five fluids on 1024x512 60.5 / 54.9; FP32:
+// Y of 256x96x32 19.5 / 16.8, Z 20.4 / 22.4, 4096x1024 64.8 / 62.7.
 //   col.rho(r)      density at row r (not modified by the sweep)
-//   col.Q(c, r)     conserved quantity c at row r
-//   col.zs(r)       zone size of row r in the sweep direction
+//   col.raw(c, r)   what is loaded for quantity c at row r
+//   col.Q(c, r, x, rho) quantity c at row r from that
+//   col.add(c, r, x, rho, Q, d) Q + d; the FP32 build adds to the unrounded product
+//   col.zs(r)       zone size of row r in the sweep direction, with its reciprocal
 //   col.v(r)        velocity at the lower face of row r
-//   col.vol(r)      the divisor of row r's InvVol (rdiv(), shared by its quantities)
-//   col.fmesh(r)    the mesh factors of row r's flux difference (cell::FluxMesh)
-//   col.flux(F, a, b, V) conservative increment of a row from face fluxes a, b
+//   col.vol(r)      the divisor of row r's InvVol (rdiv())
+//   col.surf(r, f)  face flow f times the mesh factors of the lower face of row r
+//                   (but for Sxi, col.si())
+//   col.iv(r)       InvVj of row r
 //   col.out(c, r, value) store of the updated quantity (c == NQ: density)
 // In the precision form the first Col::NXQ quantities (the azimuthal momenta)
 // are deviations Q' = Q - rho l0(r) from the profile's angular momentum
 // (col.base(r) = l0 at row r, FP64); their q' = Q'/rho is carried, and
-//   - a gradient takes the profile's jump across the face, db(r) =
+//   - a gradient takes the profile's jump across the face, D(r) =
 //     l0(r) - l0(r-1), so the limiter sees the full gradient;
 //   - a face value is held relative to l0 of the row below the face (the
-//     upper row's q' enters with + db(r));
-//   - the update of row r uses its lower face relative to l0(r) (- db(r)):
+//     upper row's q' enters with + D(r));
+//   - the update of row r uses its lower face relative to l0(r) (- D(r)):
 //     Q'(r) + dt/V (F_rho(r) (q*(r) - l0(r)) - F_rho(r+1) (q*(r+1) - l0(r))),
 //     which is Q(r) + dt/V (F_rho q* - F_rho q*) - l0(r) (rho_new - rho):
 // the reference's update of the full momentum, rearranged so that every
 // FP32 operand is of the order of the deviation and of l0's jump across one
 // row, not of l0.  In the FP64 build NXQ is 0 and the arithmetic is the
 // reference's.
-// x + d for a deviation quantity; x itself (no addition) otherwise
-__device__ __forceinline__ real dsh(real x, real d, bool dev) { return dev ? x + d : x; }
-// Holds a value in its registers at this point of the program (an empty asm
-// statement that reads it), so that the load producing it stays above.
-__device__ __forceinline__ void pin(float x) { asm volatile("" ::"v"(x)); }
-__device__ __forceinline__ void pin(double x) { asm volatile("" ::"v"(x)); }
-
-template <int NQ, class Col>
-__device__ __forceinline__ void column_sweep(Col& col, int r0, int r1, real dt) {
-  constexpr int N = NQ + 1;
+template <int R, int NQ, int C0, int C1, class Col>
+__device__ __forceinline__ void column_rows(const Col& col, int r0, int r1, real dt) {
+  constexpr int T = R + 4;  // rows r0-2+t, t = 0 .. T-1 (past r1 + 1: that row again)
   constexpr int NXQ = cell::kFix64 ? Col::NXQ : 0;
-  auto db = [&](int r) -> real {
-    if constexpr (NXQ > 0) return (real)(col.base(r) - col.base(r - 1));
-    return real(0.0);
-  };
-  real A1[N], A2[N], G2[N], S1[N], F0[N], F1[N];
-  // db of the rows r, r+1, r+2 of the loop below (deviation quantities only)
-  real D0 = real(0.0), D1 = real(0.0), D2 = real(0.0);
-  {
-    real a[N][5];
+  auto row = [&](int t) { return min(r0 - 2 + t, r1 + 1); };
+  real rho[T], v[R + 1], A[R + 1], fd[R + 1], iv[R], D[T];
+  Recip Z[T], P[T], V[R];
 #pragma unroll
-    for (int t = 0; t < 5; t++) {
-      const int r = r0 - 2 + t;
-      const real rr = col.rho(r);
-      const Recip R = recip(rr);
+  for (int t = 0; t < T; t++) rho[t] = col.rho(row(t));
 #pragma unroll
-      for (int c = 0; c < NQ; c++) a[c][t] = rdiv(col.Q(c, r), R);
-      a[NQ][t] = rr;
-    }
-    real dm = real(0.0);
-    if constexpr (NXQ > 0) {
-      dm = db(r0 - 1);
-      D0 = db(r0);
-      D1 = db(r0 + 1);
-      D2 = db(r0 + 2);
-    }
-    const Recip Z0 = recip(col.zs(r0 - 1)), Z1 = recip(col.zs(r0)), Z2 = recip(col.zs(r0 + 1)),
-                Z3 = recip(col.zs(r0 + 2));
+  for (int f = 0; f <= R; f++) v[f] = col.v(min(r0 + f, r1));
 #pragma unroll
-    for (int c = 0; c < N; c++) {
-      const bool dev = c < NXQ;
-      const real g0 = rdiv(dsh(a[c][1] - a[c][0], dm, dev), Z0);
-      const real g1 = rdiv(dsh(a[c][2] - a[c][1], D0, dev), Z1);
-      const real g2 = rdiv(dsh(a[c][3] - a[c][2], D1, dev), Z2);
-      const real g3 = rdiv(dsh(a[c][4] - a[c][3], D2, dev), Z3);
-      const real sm = vanleer_slope(g0, g1);
-      const real s0 = vanleer_slope(g1, g2);
-      const real s1 = vanleer_slope(g2, g3);
-      F0[c] = vanleer_face(col.v(r0), dt, a[c][1], sm, col.zs(r0 - 1), dsh(a[c][2], D0, dev), s0,
-                           col.zs(r0));
-      F1[c] = vanleer_face(col.v(r0 + 1), dt, a[c][2], s0, col.zs(r0), dsh(a[c][3], D1, dev), s1,
-                           col.zs(r0 + 1));
-      A1[c] = a[c][3];
-      A2[c] = a[c][4];
-      G2[c] = g3;
-      S1[c] = s1;
-    }
+  for (int t = 1; t < T; t++) Z[t] = col.zs(row(t));
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    V[q] = col.vol(row(q + 2));
+    iv[q] = col.iv(row(q + 2));
   }
-  for (int r = r0; r < r1; r++) {
-    // Every load of the iteration before its first store: the quantities of
-    // row r (its update) and of row r+3 (entering the window).  The vector
-    // memory counter retires loads and stores in issue order, so a load
-    // issued after a store would wait for that store as well.
-    // On the last row no row enters, and row r is loaded in its place (no
-    // branch around the loads; the values are not used).
-    const bool more = r + 1 < r1;
-    const int rn = r + 3, rl = more ? rn : r;
-    real Qr[NQ], Qn[NQ];
+  if constexpr (NXQ > 0) {
 #pragma unroll
-    for (int c = 0; c < NQ; c++) Qr[c] = col.Q(c, r);
-    const real rhor = col.rho(r);
-    const real rr = col.rho(rl);
+    for (int t = 1; t < T; t++) D[t] = (real)(col.base(row(t)) - col.base(row(t) - 1));
+  }
+  const real si = col.si();
 #pragma unroll
-    for (int c = 0; c < NQ; c++) Qn[c] = col.Q(c, rl);
-    const real zsn = col.zs(rl);
-    const real v0 = col.v(r), v1 = col.v(r + 1), v2 = col.v(r + 2);
-    const real zs1 = col.zs(r + 1), zs2 = col.zs(r + 2);
-    const Recip V = col.vol(r);
-    const cell::FluxMesh FM = col.fmesh(r);
-    // the entering row's values are used only after the stores; held here, so
-    // that their loads are not moved below them
+  for (int t = 0; t < T; t++) P[t] = recip(rho[t]);
+  // the factor of the upwind slope in the face value
 #pragma unroll
-    for (int c = 0; c < NQ; c++) pin(Qn[c]);
-    pin(rr);
-    pin(zsn);
-    pin(v2);
-    // UpdateY/Z (src/update_y.c:68-70), then the density last (src/update_density_y.c:66-68)
+  for (int f = 0; f <= R; f++)
+    A[f] = v[f] > real(0.0) ? real(0.5) * (Z[f + 1].d - v[f] * dt) : -(real(0.5) * (Z[f + 2].d + v[f] * dt));
+  auto shift = [&](real x, int t, bool dev) { return NXQ > 0 && dev ? x + D[t] : x; };
+  // the upwind value at the lower face of rows r0 .. r0+R
+  auto faces = [&](const real (&q)[T], bool dev, real (&fc)[R + 1]) {
+    real g[T], s[T];
 #pragma unroll
-    for (int c = 0; c < NQ; c++) {
-      const real f0 = (c < NXQ) ? F0[c] - D0 : F0[c];
-      col.out(c, r, Qr[c] + col.flux(FM, v0 * f0 * F0[NQ], v1 * F1[c] * F1[NQ], V));
+    for (int t = 1; t < T; t++) g[t] = rdiv(shift(q[t] - q[t - 1], t, dev), Z[t]);
+#pragma unroll
+    for (int t = 1; t < T - 1; t++) s[t] = vanleer_slope(g[t], g[t + 1]);
+#pragma unroll
+    for (int f = 0; f <= R; f++) {
+      const bool pos = v[f] > real(0.0);
+      fc[f] = (pos ? q[f + 1] : shift(q[f + 2], f + 2, dev)) + A[f] * (pos ? s[f + 1] : s[f + 2]);
     }
-    col.out(NQ, r, rhor + col.flux(FM, v0 * F0[NQ], v1 * F1[NQ], V));
-    if (!more) break;
-    // advance the window by one row: row r+3 enters
-    const Recip R = recip(rr);
-    const Recip Zn = recip(zsn);
-    real D3 = real(0.0);
-    if constexpr (NXQ > 0) D3 = db(rn);
+  };
+  // UpdateY/Z (src/update_y.c:68-70, src/update_density_y.c:66-68) of the rows
+  // from what enters each through its lower face and leaves it through its
+  // upper one; the FP32 build subtracts from the unrounded product
+  auto update = [&](int c, const real* val, const real* fac, const real (&lower)[R + 1], const real (&upper)[R + 1]) {
+    real up[R + 1];
+    {
+#pragma clang fp contract(off)
 #pragma unroll
-    for (int c = 0; c < N; c++) {
-      const bool dev = c < NXQ;
-      const real an = (c < NQ) ? rdiv(Qn[c], R) : rr;
-      const real g3 = rdiv(dsh(an - A2[c], D3, dev), Zn);
-      const real s2 = vanleer_slope(G2[c], g3);
-      const real f2 = vanleer_face(v2, dt, A1[c], S1[c], zs1, dsh(A2[c], D2, dev), s2, zs2);
-      F0[c] = F1[c];
-      F1[c] = f2;
-      A1[c] = A2[c];
-      A2[c] = an;
-      G2[c] = g3;
-      S1[c] = s2;
+      for (int f = 0; f <= R; f++) up[f] = col.surf(min(r0 + f, r1), upper[f]) * si;
     }
-    D0 = D1;
-    D1 = D2;
-    D2 = D3;
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      const real lo = col.surf(row(q + 2), lower[q]);
+      const real d = cell::kFix64 ? fma(lo, si, -up[q + 1]) : lo * si - up[q + 1];
+      const real inc = rdiv((d * dt) * iv[q], V[q]);
+      real x = val[q] + inc;
+      if constexpr (cell::kFix64)
+        if (c < NQ) x = col.add(c, row(q + 2), fac[q], rho[q + 2], val[q], inc);
+      if (r0 + q < r1) col.out(c, r0 + q, x);
+    }
+  };
+  real raw[T];
+#pragma unroll
+  for (int t = 0; t < T; t++) raw[t] = col.raw(C0, row(t));
+  faces(rho, false, fd);
+#pragma unroll
+  for (int c = C0; c < C1; c++) {
+    const bool dev = c < NXQ;
+    real Q[T], q[T], fac[R], fc[R + 1], lower[R + 1], upper[R + 1];
+#pragma unroll
+    for (int t = 0; t < T; t++) Q[t] = col.Q(c, row(t), raw[t], rho[t]);
+#pragma unroll
+    for (int t = 0; t < R; t++) fac[t] = raw[t + 2];
+    // the next quantity's loads go out here, before this one's arithmetic and
+    // stores (loads retire in order behind earlier stores)
+    if (c + 1 < C1) {
+#pragma unroll
+      for (int t = 0; t < T; t++) raw[t] = col.raw(c + 1, row(t));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < T; t++) q[t] = rdiv(Q[t], P[t]);
+    faces(q, dev, fc);
+#pragma unroll
+    for (int f = 0; f <= R; f++) {
+      upper[f] = v[f] * fc[f] * fd[f];
+      lower[f] = NXQ > 0 && dev ? v[f] * (fc[f] - D[f + 2]) * fd[f] : upper[f];
+    }
+    update(c, Q + 2, fac, lower, upper);
+  }
+  if (C0 == 0) {
+    real f[R + 1];
+#pragma unroll
+    for (int t = 0; t <= R; t++) f[t] = v[t] * fd[t];
+    update(NQ, rho + 2, nullptr, f, f);
   }
 }
 
-// A column carrying part of the quantities: COUNT of them from FIRST on,
-// plus the density, which every part needs for q = Q/rho and the mass flux;
-// only the part with WRITE_RHO stores the density.  Splitting a column's
-// quantities over two threads doubles the threads of a sweep (more waves to
-// hide the FP64 latency) for one extra density sweep per column.
-template <class Col, int NQ, int FIRST, int COUNT, bool WRITE_RHO>
-struct ColPart {
-  // the deviation quantities of the column among those carried here
-  static constexpr int NXQ = FIRST < Col::NXQ ? (Col::NXQ - FIRST < COUNT ? Col::NXQ - FIRST : COUNT) : 0;
-  static_assert(FIRST == 0 || FIRST >= Col::NXQ, "the deviation quantities lead each part");
-  const Col& c;
-  __device__ __forceinline__ double base(int r) const { return c.base(r); }
-  __device__ __forceinline__ real rho(int r) const { return c.rho(r); }
-  __device__ __forceinline__ real Q(int q, int r) const { return c.Q(FIRST + q, r); }
-  __device__ __forceinline__ real zs(int r) const { return c.zs(r); }
-  __device__ __forceinline__ real v(int r) const { return c.v(r); }
-  __device__ __forceinline__ Recip vol(int r) const { return c.vol(r); }
-  __device__ __forceinline__ cell::FluxMesh fmesh(int r) const { return c.fmesh(r); }
-  __device__ __forceinline__ real flux(const cell::FluxMesh& F, real a, real b, const Recip& V) const {
-    return c.flux(F, a, b, V);
-  }
-  __device__ __forceinline__ void out(int q, int r, real val) const {
-    if (q < COUNT) c.out(FIRST + q, r, val);
-    else if (WRITE_RHO) c.out(NQ, r, val);
-  }
-};
-
-// the sweep of part grp of a column: 0 every quantity, 1 the first half and
-// the density, 2 the second half
-template <int NQ, class Col>
-__device__ __forceinline__ void column_sweep_part(const Col& col, int grp, int r0, int r1, real dt) {
-  constexpr int H = NQ / 2;
-  if (grp == 1) {
-    ColPart<Col, NQ, 0, H, true> p{col};
-    column_sweep<H>(p, r0, r1, dt);
+// rows [r0, r1) of at most R; with R = 1 part grp (0 or 1) of the quantities: a
+// mesh that needs that few rows per thread is short of waves (column_form_of())
+template <int R, int NQ, class Col>
+__device__ __forceinline__ void column_sweep(const Col& col, int r0, int r1, real dt, int grp) {
+  if constexpr (R == 1) {
+    if (grp == 0) column_rows<R, NQ, 0, NQ / 2>(col, r0, r1, dt);
+    else column_rows<R, NQ, NQ / 2, NQ>(col, r0, r1, dt);
   } else {
-    ColPart<Col, NQ, H, NQ - H, false> p{col};
-    column_sweep<NQ - H>(p, r0, r1, dt);
+    column_rows<R, NQ, 0, NQ>(col, r0, r1, dt);
   }
 }
 
@@ -847,29 +842,26 @@ struct ColY2 {
   const real *rho_in, *vxt, *vyt, *e_in;
   real* out_[6];
   int i, ixp;
-  real of, dt;
+  real of;
   __device__ __forceinline__ double base(int r) const { return cell::lbase<G>(*m, r, 0, (double)of); }
   __device__ __forceinline__ int L(int r) const { return i + r * m->pitch; }
   __device__ __forceinline__ real rho(int r) const { return rho_in[L(r)]; }
-  __device__ __forceinline__ real Q(int c, int r) const {
+  __device__ __forceinline__ real raw(int c, int r) const {
     const int l = L(r);
-    const real rr = rho_in[l];
-    if (c < 2) {
-      real mm, mp;
-      cell::momenta_x<G>(*m, i, r, 0, rr, vxt[l], vxt[ixp + r * m->pitch], of, mm, mp);
-      return c == 0 ? mp : mm;
-    }
-    if (c == 2) return vyt[l + m->pitch] * rr;
-    if (c == 3) return vyt[l] * rr;
-    return e_in[l];
+    return c == 0 ? vxt[ixp + r * m->pitch] : c == 1 ? vxt[l] : c == 2 ? vyt[l + m->pitch] : c == 3 ? vyt[l] : e_in[l];
   }
-  __device__ __forceinline__ real zs(int r) const { return zone_size_y(*m, r); }
+  __device__ __forceinline__ real Q(int c, int r, real x, real rr) const {
+    return c < 2 ? cell::momentum_x<G>(*m, r, 0, rr, x, of) : c < 4 ? x * rr : x;
+  }
+  __device__ __forceinline__ real add(int c, int, real x, real rr, real Q, real d) const {
+    return c == 2 || c == 3 ? fma(x, rr, d) : Q + d;
+  }
+  __device__ __forceinline__ Recip zs(int r) const { return Recip{m->zy[r], m->rzy[r]}; }
   __device__ __forceinline__ real v(int r) const { return vyt[L(r)]; }
   __device__ __forceinline__ Recip vol(int r) const { return invvol_recip(*m, i, 0); }
-  __device__ __forceinline__ cell::FluxMesh fmesh(int r) const { return cell::flux_y_mesh(*m, i, r, 0); }
-  __device__ __forceinline__ real flux(const cell::FluxMesh& F, real a, real b, const Recip& V) const {
-    return cell::flux_yz(F, dt, a, b, V);
-  }
+  __device__ __forceinline__ real surf(int r, real f) const { return (f * m->syj[r]) * m->syk[0]; }
+  __device__ __forceinline__ real iv(int r) const { return m->invvj[r]; }
+  __device__ __forceinline__ real si() const { return m->sxi[i]; }
   __device__ __forceinline__ void out(int c, int r, real val) const { out_[c][L(r)] = val; }
 };
 
@@ -883,45 +875,38 @@ struct ColZ {
   const real *rho_in, *vxt, *vyt, *vzt, *e_in;
   real* out_[8];
   int i, j, ixp;
-  real of, dt;
+  real of;
   __device__ __forceinline__ double base(int r) const { return cell::lbase<G>(*m, j, r, (double)of); }
   __device__ __forceinline__ int L(int r) const { return i + j * m->pitch + r * m->stride; }
   __device__ __forceinline__ real rho(int r) const { return rho_in[L(r)]; }
-  __device__ __forceinline__ real Q(int c, int r) const {
+  __device__ __forceinline__ real raw(int c, int r) const {
     const int l = L(r);
-    const real rr = rho_in[l];
     switch (c) {
-      case 0:
-      case 1: {
-        real mm, mp;
-        cell::momenta_x<G>(*m, i, j, r, rr, vxt[l], vxt[ixp + j * m->pitch + r * m->stride], of, mm, mp);
-        return c == 0 ? mp : mm;
-      }
-      case 2:
-        return vyt[l + m->pitch] * rr;
-      case 3:
-        return vyt[l] * rr;
-      case 4: {
-        real p = vzt[l + m->stride] * rr;
-        if (G == SPH) p *= m->ymed[j];
-        return p;
-      }
-      case 5: {
-        real q = vzt[l] * rr;
-        if (G == SPH) q *= m->ymed[j];
-        return q;
-      }
-      default:
-        return e_in[l];
+      case 0: return vxt[ixp + j * m->pitch + r * m->stride];
+      case 1: return vxt[l];
+      case 2: return vyt[l + m->pitch];
+      case 3: return vyt[l];
+      case 4: return vzt[l + m->stride];
+      case 5: return vzt[l];
+      default: return e_in[l];
     }
   }
-  __device__ __forceinline__ real zs(int r) const { return zone_size_z<G>(*m, j, r); }
+  __device__ __forceinline__ real Q(int c, int r, real x, real rr) const {
+    if (c < 2) return cell::momentum_x<G>(*m, j, r, rr, x, of);
+    if (c > 5) return x;
+    const real p = x * rr;
+    return c > 3 && G == SPH ? p * m->ymed[j] : p;
+  }
+  __device__ __forceinline__ real add(int c, int, real x, real rr, real Q, real d) const {
+    if (c < 2 || c > 5) return Q + d;
+    return c > 3 && G == SPH ? fma(x * rr, m->ymed[j], d) : fma(x, rr, d);
+  }
+  __device__ __forceinline__ Recip zs(int r) const { return Recip{m->zz[j + r * m->sy], m->rzz[j + r * m->sy]}; }
   __device__ __forceinline__ real v(int r) const { return vzt[L(r)]; }
   __device__ __forceinline__ Recip vol(int r) const { return invvol_recip(*m, i, r); }
-  __device__ __forceinline__ cell::FluxMesh fmesh(int r) const { return cell::flux_z_mesh(*m, i, j, r); }
-  __device__ __forceinline__ real flux(const cell::FluxMesh& F, real a, real b, const Recip& V) const {
-    return cell::flux_yz(F, dt, a, b, V);
-  }
+  __device__ __forceinline__ real surf(int r, real f) const { return (f * m->szj[j]) * m->szk[r]; }
+  __device__ __forceinline__ real iv(int r) const { return m->invvj[j]; }
+  __device__ __forceinline__ real si() const { return m->sxi[i]; }
   __device__ __forceinline__ void out(int c, int r, real val) const { out_[c][L(r)] = val; }
 };
 
@@ -935,34 +920,34 @@ struct ColY3 {
   const real* vyt;
   real* out_[8];
   int i, k;
-  real dt, of;
+  real of;
   __device__ __forceinline__ double base(int r) const { return cell::lbase<G>(*m, r, k, (double)of); }
   __device__ __forceinline__ int L(int r) const { return i + r * m->pitch + k * m->stride; }
   __device__ __forceinline__ real rho(int r) const { return rho_in[L(r)]; }
-  __device__ __forceinline__ real Q(int c, int r) const { return q_in[c][L(r)]; }
-  __device__ __forceinline__ real zs(int r) const { return zone_size_y(*m, r); }
+  __device__ __forceinline__ real raw(int c, int r) const { return q_in[c][L(r)]; }
+  __device__ __forceinline__ real Q(int, int, real x, real) const { return x; }
+  __device__ __forceinline__ real add(int, int, real, real, real Q, real d) const { return Q + d; }
+  __device__ __forceinline__ Recip zs(int r) const { return Recip{m->zy[r], m->rzy[r]}; }
   __device__ __forceinline__ real v(int r) const { return vyt[L(r)]; }
   __device__ __forceinline__ Recip vol(int r) const { return invvol_recip(*m, i, k); }
-  __device__ __forceinline__ cell::FluxMesh fmesh(int r) const { return cell::flux_y_mesh(*m, i, r, k); }
-  __device__ __forceinline__ real flux(const cell::FluxMesh& F, real a, real b, const Recip& V) const {
-    return cell::flux_yz(F, dt, a, b, V);
-  }
+  __device__ __forceinline__ real surf(int r, real f) const { return (f * m->syj[r]) * m->syk[k]; }
+  __device__ __forceinline__ real iv(int r) const { return m->invvj[r]; }
+  __device__ __forceinline__ real si() const { return m->sxi[i]; }
   __device__ __forceinline__ void out(int c, int r, real val) const { out_[c][L(r)] = val; }
 };
 
-// 2-D: momenta + Y sweep; rows [nghy + s*rows_per, ...) of the active range.
+// 2-D: momenta + Y sweep; rows [nghy + s*rows_per, ...) of the active range, R
+// at a time, block row s*ngrp + g taking group g of the quantities.
 // AD = 1 also transports the energy (e_in -> e_out).
-template <int G, int DZ, int AD, int SPLIT = 0>
-__device__ __forceinline__ void kd_sweep_y2(const dim3 bid, const dmesh& m, real dt, const real* __restrict__ rho_in, const real* __restrict__ vxt, const real* __restrict__ vyt, const real* __restrict__ e_in, real* __restrict__ rho_out, real* __restrict__ q0, real* __restrict__ q1, real* __restrict__ q2, real* __restrict__ q3, real* __restrict__ e_out, int rows_per, real of) {
+template <int G, int AD, int R>
+__device__ __forceinline__ void kd_sweep_y2(const dim3 bid, const dmesh& m, real dt, const real* __restrict__ rho_in, const real* __restrict__ vxt, const real* __restrict__ vyt, const real* __restrict__ e_in, real* __restrict__ rho_out, real* __restrict__ q0, real* __restrict__ q1, real* __restrict__ q2, real* __restrict__ q3, real* __restrict__ e_out, real of) {
   const int i = bid.x * blockDim.x + threadIdx.x;
   if (i >= m.nx) return;
-  const int seg = SPLIT ? (int)bid.y >> 1 : (int)bid.y;
-  const int r0 = m.nghy + seg * rows_per;
-  const int r1 = min(r0 + rows_per, m.ny + m.nghy);
-  ColY2<G> col{&m, rho_in, vxt, vyt, e_in, {q0, q1, q2, q3, AD ? e_out : rho_out, rho_out}, i, ixp_of(i, m.nx), of,
-               dt};
-  if (SPLIT) column_sweep_part<4 + AD>(col, 1 + ((int)bid.y & 1), r0, r1, dt);
-  else column_sweep<4 + AD>(col, r0, r1, dt);
+  const int seg = R == 1 ? (int)bid.y >> 1 : (int)bid.y, grp = (int)bid.y & 1;
+  const int r0 = m.nghy + seg * R;
+  const int r1 = min(r0 + R, m.ny + m.nghy);
+  const ColY2<G> col{&m, rho_in, vxt, vyt, e_in, {q0, q1, q2, q3, AD ? e_out : rho_out, rho_out}, i, ixp_of(i, m.nx), of};
+  column_sweep<R, 4 + AD>(col, r0, r1, dt, grp);
 }
 // 2-D Y sweep of every fluid in one launch: blockIdx.z is the fluid
 struct Y2Tab {
@@ -974,50 +959,48 @@ struct Y2Tab {
   real* q[8][4];
   real* e_out[8];
 };
-template <int G, int DZ, int AD, int SPLIT>
-__global__ void __launch_bounds__(BXF) kf_sweep_y2(dmesh m, real dt, Y2Tab T, int rows_per, real of) {
+template <int G, int AD, int R>
+__global__ void __launch_bounds__(BXF) kf_sweep_y2(dmesh m, real dt, Y2Tab T, real of) {
   const dim3 b = xcd_bid();
   const int fl = (int)b.z;
-  kd_sweep_y2<G, DZ, AD, SPLIT>(b, m, dt, T.rho_in[fl], T.vxt[fl], T.vyt[fl], T.e_in[fl], T.rho_out[fl], T.q[fl][0],
-                                T.q[fl][1], T.q[fl][2], T.q[fl][3], T.e_out[fl], rows_per, of);
+  kd_sweep_y2<G, AD, R>(b, m, dt, T.rho_in[fl], T.vxt[fl], T.vyt[fl], T.e_in[fl], T.rho_out[fl], T.q[fl][0], T.q[fl][1],
+                        T.q[fl][2], T.q[fl][3], T.e_out[fl], of);
 }
 
 // 3-D: Y sweep of the Z-swept fields
-template <int G, int DZ, int AD, int SPLIT>
+template <int G, int AD, int R>
 __global__ void __launch_bounds__(BXF) kf_sweep_y3(dmesh m, real dt, const real* __restrict__ rho_in, const real* __restrict__ z0,
                                                    const real* __restrict__ z1, const real* __restrict__ z2, const real* __restrict__ z3,
                                                    const real* __restrict__ z4, const real* __restrict__ z5, const real* __restrict__ ze,
                                                    const real* __restrict__ vyt, real* __restrict__ rho_out, real* __restrict__ q0, real* __restrict__ q1,
                                                    real* __restrict__ q2, real* __restrict__ q3, real* __restrict__ q4, real* __restrict__ q5, real* __restrict__ e_out,
-                                                   int rows_per, real of) {
+                                                   real of) {
   const dim3 b = xcd_bid();
   const int i = b.x * blockDim.x + threadIdx.x;
   if (i >= m.nx) return;
   const int k = m.nghz + (int)b.z;
-  const int seg = SPLIT ? (int)b.y >> 1 : (int)b.y;
-  const int r0 = m.nghy + seg * rows_per;
-  const int r1 = min(r0 + rows_per, m.ny + m.nghy);
-  ColY3<G> col{&m, rho_in, {z0, z1, z2, z3, z4, z5, ze}, vyt,
-               {q0, q1, q2, q3, q4, q5, AD ? e_out : rho_out, rho_out}, i, k, dt, of};
-  if (SPLIT) column_sweep_part<6 + AD>(col, 1 + ((int)b.y & 1), r0, r1, dt);
-  else column_sweep<6 + AD>(col, r0, r1, dt);
+  const int seg = R == 1 ? (int)b.y >> 1 : (int)b.y, grp = (int)b.y & 1;
+  const int r0 = m.nghy + seg * R;
+  const int r1 = min(r0 + R, m.ny + m.nghy);
+  const ColY3<G> col{&m, rho_in, {z0, z1, z2, z3, z4, z5, ze}, vyt,
+                     {q0, q1, q2, q3, q4, q5, AD ? e_out : rho_out, rho_out}, i, k, of};
+  column_sweep<R, 6 + AD>(col, r0, r1, dt, grp);
 }
 
 // 3-D: momenta + Z sweep for rows j in [1, sy-2] (the Y sweep's stencil)
-template <int G, int AD, int SPLIT>
+template <int G, int AD, int R>
 __device__ __forceinline__ void kd_sweep_z(const dim3 b, const dmesh& m, real dt, const real* __restrict__ rho_in, const real* __restrict__ vxt,
                                                   const real* __restrict__ vyt, const real* __restrict__ vzt, const real* __restrict__ e_in,
                                                   real* __restrict__ rho_out, real* __restrict__ q0, real* __restrict__ q1, real* __restrict__ q2, real* __restrict__ q3,
-                                                  real* __restrict__ q4, real* __restrict__ q5, real* __restrict__ e_out, int planes_per, real of) {
+                                                  real* __restrict__ q4, real* __restrict__ q5, real* __restrict__ e_out, real of) {
   const int i = b.x * blockDim.x + threadIdx.x;
   if (i >= m.nx) return;
-  const int j = 1 + (SPLIT ? (int)b.y >> 1 : (int)b.y);
-  const int r0 = m.nghz + (int)b.z * planes_per;
-  const int r1 = min(r0 + planes_per, m.nz + m.nghz);
-  ColZ<G> col{&m, rho_in, vxt, vyt, vzt, e_in, {q0, q1, q2, q3, q4, q5, AD ? e_out : rho_out, rho_out}, i, j,
-              ixp_of(i, m.nx), of, dt};
-  if (SPLIT) column_sweep_part<6 + AD>(col, 1 + ((int)b.y & 1), r0, r1, dt);
-  else column_sweep<6 + AD>(col, r0, r1, dt);
+  const int j = 1 + (R == 1 ? (int)b.y >> 1 : (int)b.y), grp = (int)b.y & 1;
+  const int r0 = m.nghz + (int)b.z * R;
+  const int r1 = min(r0 + R, m.nz + m.nghz);
+  const ColZ<G> col{&m, rho_in, vxt, vyt, vzt, e_in, {q0, q1, q2, q3, q4, q5, AD ? e_out : rho_out, rho_out}, i, j,
+                    ixp_of(i, m.nx), of};
+  column_sweep<R, 6 + AD>(col, r0, r1, dt, grp);
 }
 
 // ------------------------------------------------------------------ the X sweep
@@ -1394,8 +1377,8 @@ __global__ void __launch_bounds__(64) kf_vmed(dmesh m, VmTab T, int nrings) {
 // writes the Vx_temp they read.  The ring sums are one dependent chain each,
 // latency bound, so their waves run beside the sweep's without the second
 // stream and its events.
-template <int G, int AD, int SPLIT>
-__global__ void __launch_bounds__(BXF) kf_sweep_y2v(dmesh m, real dt, Y2Tab T, int rows_per, real of, VmTab V,
+template <int G, int AD, int R>
+__global__ void __launch_bounds__(BXF) kf_sweep_y2v(dmesh m, real dt, Y2Tab T, real of, VmTab V,
                                                     int nrings, int nvm, dim3 gy) {
   const int lin = (int)blockIdx.x;
   if (lin < nvm) {
@@ -1408,18 +1391,18 @@ __global__ void __launch_bounds__(BXF) kf_sweep_y2v(dmesh m, real dt, Y2Tab T, i
   const int p = x * q + min(x, r) + (L >> 3);
   const dim3 b(p % gy.x, (p / gy.x) % gy.y, p / (gy.x * gy.y));
   const int fl = (int)b.z;
-  kd_sweep_y2<G, 0, AD, SPLIT>(b, m, dt, T.rho_in[fl], T.vxt[fl], T.vyt[fl], T.e_in[fl], T.rho_out[fl], T.q[fl][0],
-                               T.q[fl][1], T.q[fl][2], T.q[fl][3], T.e_out[fl], rows_per, of);
+  kd_sweep_y2<G, AD, R>(b, m, dt, T.rho_in[fl], T.vxt[fl], T.vyt[fl], T.e_in[fl], T.rho_out[fl], T.q[fl][0],
+                        T.q[fl][1], T.q[fl][2], T.q[fl][3], T.e_out[fl], of);
 }
 
 // The 3-D Z sweep, and in the same launch (V.vxt[0] given) the VxMed pass of the
 // X sweep as in kf_sweep_y2v: the first nvm workgroups sum one ring each, the
 // others are the sweep's grid gz in launch order.
-template <int G, int AD, int SPLIT>
+template <int G, int AD, int R>
 __global__ void __launch_bounds__(BXF) kf_sweep_z(dmesh m, real dt, const real* __restrict__ rho_in, const real* __restrict__ vxt,
                                                   const real* __restrict__ vyt, const real* __restrict__ vzt, const real* __restrict__ e_in,
                                                   real* __restrict__ rho_out, real* __restrict__ q0, real* __restrict__ q1, real* __restrict__ q2, real* __restrict__ q3,
-                                                  real* __restrict__ q4, real* __restrict__ q5, real* __restrict__ e_out, int planes_per, real of,
+                                                  real* __restrict__ q4, real* __restrict__ q5, real* __restrict__ e_out, real of,
                                                   double* __restrict__ vxmed, int nvm, dim3 gz) {
   const int lin = (int)blockIdx.x - nvm;
   if (lin < 0) {
@@ -1427,7 +1410,7 @@ __global__ void __launch_bounds__(BXF) kf_sweep_z(dmesh m, real dt, const real* 
     return;
   }
   const dim3 b(lin % gz.x, (lin / gz.x) % gz.y, lin / (gz.x * gz.y));
-  kd_sweep_z<G, AD, SPLIT>(b, m, dt, rho_in, vxt, vyt, vzt, e_in, rho_out, q0, q1, q2, q3, q4, q5, e_out, planes_per, of);
+  kd_sweep_z<G, AD, R>(b, m, dt, rho_in, vxt, vyt, vzt, e_in, rho_out, q0, q1, q2, q3, q4, q5, e_out, of);
 }
 
 // NewVelocity_y/z on active faces and Stockholm damping on active cells.
@@ -2049,23 +2032,25 @@ static int fused_boundaries(f3d_hip_ctx* ctx, Scratch* S, real* dens, real* vx, 
   return 0;
 }
 
-// tuning knobs of the column sweeps (rows per thread, f3d_fused_set_tiling;
-// rows_y 0: automatic).  Measured on MI355X: 4 rows in Y on the 256x96x32,
-// 4096x1024 and 1024x512 disks (2 rows: 4096x1024 step 0.554 -> 0.579 ms),
-// 2 rows on the 384x128 disk (0.0587 -> 0.0571 ms), so 2 rows where 4 would
-// leave the launch under 1024 waves; 6 planes in Z (the 32 planes then take
-// 6 workgroup rows, one wave of launches at 3 waves per SIMD: 42.6 -> 41.3 us
-// against 3 planes)
-static int g_rows_y = 0, g_rows_z = 6;
-static int rows_y_of(const dmesh& m, int nf) {
-  if (g_rows_y > 0) return g_rows_y;
-  const long w4 = (long)((m.nx + BXF - 1) / BXF) * (m.dimz ? m.nz : nf) * ((m.ny + 3) / 4);
-  return w4 < 1024 ? 2 : 4;
-}
-// column sweeps: 1 two threads per column (each with the density and half of
-// the quantities), 0 one, -1 automatic: measured on MI355X, the split only
-// pays when a sweep has fewer waves than the GPU has SIMDs (small 2-D grids)
+// tuning knobs of the column sweeps: rows and planes per thread
+// (f3d_fused_set_tiling, 0 automatic) and whether two threads share a row's
+// quantities (f3d_fused_set_colsplit: 1 always, 0 never, -1 automatic)
+static int g_rows_y = 0, g_rows_z = 0;
 static int g_colsplit = -1;
+// the column sweeps' forms: 4 or 2 rows per thread, or one row by two threads
+static int column_form(int rows) { return rows >= 4 ? 4 : rows >= 2 ? 2 : 1; }
+// The form of a column sweep of `rows` rows whose row has w waves.  Fewer rows
+// per thread repeat more of the halo's work but make more waves; with 256 CUs a
+// launch under about 2 waves per SIMD is bound by the length of one wave.
+// Measured on MI355X (us, 4 / 2 / 1 rows): 4096x1024 100.7 / 119.0 / 193.0,
+// 2048x256 (2048 waves of 4 rows) 18.1 / 18.9 / 27.0, 768x256 (768) 11.6 / 11.2 /
+// 14.3, 256x256 (512 of 2 rows) 10.0 / 8.1 / 9.0, 96x40x12 (480 of 2) 11.4 / 8.5 /
+// 8.6, 384x128 (384 of 2) 9.6 / 8.2 / 7.8, 96x48 10.0 / 8.0 / 6.4.
+static int column_form_of(int knob, long w, int rows) {
+  if (g_colsplit == 1) return 1;
+  int r = knob > 0 ? column_form(knob) : w * ((rows + 3) / 4) >= 2048 ? 4 : w * ((rows + 1) / 2) >= 448 ? 2 : 1;
+  return g_colsplit == 0 && r == 1 ? 2 : r;
+}
 // X-sweep form: 0 (and 1) automatic, 2 tiles of g_xtile cells, 3 one wave per
 // ring on rings of 256 cells, 4 tiles of 256 cells
 static int g_xmode = 0;
@@ -2243,15 +2228,21 @@ static int yz_sweeps(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* 
   const dmesh& m = S->m;
   const real of = (real)ctx->ph.OMEGAFRAME;
   const real rdt = (real)dt;
-  const int ry = rows_y_of(m, nf), rz = g_rows_z;
-  const long waves = (long)((m.nx + BXF - 1) / BXF) * (m.dimz ? (long)m.nz * ((m.ny + ry - 1) / ry)
-                                                               : (long)nf * ((m.ny + ry - 1) / ry));
-  const int split = g_colsplit >= 0 ? g_colsplit : (waves < 1024 ? 1 : 0);
-  const int sp = split ? 2 : 1;  // threads per column
-#define FDISPATCH_ADS(ctx_, KERN, grid, ...)                                             \
-  do {                                                                                  \
-    if (split) FDISPATCH_AD_T(ctx_, KERN, 1, grid, dim3(BXF), 0, __VA_ARGS__);         \
-    else FDISPATCH_AD_T(ctx_, KERN, 0, grid, dim3(BXF), 0, __VA_ARGS__);               \
+  const long wx = (m.nx + BXF - 1) / BXF;
+  const int ry = column_form_of(g_rows_y, wx * (m.dimz ? m.nz : nf), m.ny);
+  const int rz = m.dimz ? column_form_of(g_rows_z, wx * (m.sy - 2), m.nz) : 0;
+  const int gy_grp = ry == 1 ? 2 : 1, gz_grp = rz == 1 ? 2 : 1;
+  const int ad = (ctx->ph.eos == 2);
+#define COL_R(ROWS_, M_, ...)                  \
+  do {                                       \
+    if (ROWS_ == 4) M_(4, __VA_ARGS__);      \
+    else if (ROWS_ == 2) M_(2, __VA_ARGS__); \
+    else M_(1, __VA_ARGS__);                 \
+  } while (0)
+#define COL_GA(M_)                                                                      \
+  do {                                                                                   \
+    if (m.geom == SPH) { if (ad) M_(SPH, 1); else M_(SPH, 0); }                         \
+    else { if (ad) M_(CYL, 1); else M_(CYL, 0); }                                       \
   } while (0)
   if (m.dimz) {
     for (int q = 0; q < nf; q++) {
@@ -2259,26 +2250,30 @@ static int yz_sweeps(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* 
       const TSet& t = tl[q];
       // eight separate buffers: six Z-swept momenta, the Z-swept density and energy
       real* const* Z = &S->f[FS_Z0];
-      dim3 gz((m.nx + BXF - 1) / BXF, (m.sy - 2) * sp, (m.nz + rz - 1) / rz);
+      const dim3 gz((m.nx + BXF - 1) / BXF, (m.sy - 2) * gz_grp, (m.nz + rz - 1) / rz);
       const int nvm = vm ? m.ny * m.nz : 0;
       const dim3 g1(nvm + gz.x * gz.y * gz.z);
-      const int ad = (ctx->ph.eos == 2);
       f3d_stage_begin(ctx, F3D_ST_SWEEP_Z);
-#define SWZ(G_, AD_, SP_)                                                                                         \
-  hipLaunchKernelGGL((kf_sweep_z<G_, AD_, SP_>), g1, dim3(BXF), 0, ctx->stream, m, rdt, f.Density, f.Vx_temp, f.Vy_temp, \
-                     f.Vz_temp, f.Energy, Z[6], Z[0], Z[1], Z[2], Z[3], Z[4], Z[5], Z[7], rz, of,                 \
+#define SWZ1(R_, G_, AD_)                                                                                         \
+  hipLaunchKernelGGL((kf_sweep_z<G_, AD_, R_>), g1, dim3(BXF), 0, ctx->stream, m, rdt, f.Density, f.Vx_temp, f.Vy_temp, \
+                     f.Vz_temp, f.Energy, Z[6], Z[0], Z[1], Z[2], Z[3], Z[4], Z[5], Z[7], of,         \
                      vm ? vm->vxmed[q] : nullptr, nvm, gz)
-#define SWZ_G(G_) \
-  do { if (ad) { if (split) SWZ(G_, 1, 1); else SWZ(G_, 1, 0); } else { if (split) SWZ(G_, 0, 1); else SWZ(G_, 0, 0); } } while (0)
-      if (m.geom == SPH) SWZ_G(SPH); else SWZ_G(CYL);
-#undef SWZ_G
+#define SWZ(G_, AD_) COL_R(rz, SWZ1, G_, AD_)
+      COL_GA(SWZ);
 #undef SWZ
+#undef SWZ1
       F3D_LAUNCH_CHECK(ctx);
       f3d_stage_end(ctx, F3D_ST_SWEEP_Z);
-      dim3 gy((m.nx + BXF - 1) / BXF, ((m.ny + ry - 1) / ry) * sp, m.nz);
+      const dim3 gy((m.nx + BXF - 1) / BXF, ((m.ny + ry - 1) / ry) * gy_grp, m.nz);
       f3d_stage_begin(ctx, F3D_ST_SWEEP_Y);
-      FDISPATCH_ADS(ctx, kf_sweep_y3, gy, rdt, Z[6], Z[0], Z[1], Z[2], Z[3], Z[4], Z[5], Z[7], f.Vy_temp, t.rhoy,
-                    t.m[0], t.m[1], t.m[2], t.m[3], t.m[4], t.m[5], t.ey, ry, of);
+#define SWY1(R_, G_, AD_)                                                                                          \
+  hipLaunchKernelGGL((kf_sweep_y3<G_, AD_, R_>), gy, dim3(BXF), 0, ctx->stream, m, rdt, Z[6], Z[0], Z[1], Z[2], Z[3], Z[4], \
+                     Z[5], Z[7], f.Vy_temp, t.rhoy, t.m[0], t.m[1], t.m[2], t.m[3], t.m[4], t.m[5], t.ey, of)
+#define SWY(G_, AD_) COL_R(ry, SWY1, G_, AD_)
+      COL_GA(SWY);
+#undef SWY
+#undef SWY1
+      F3D_LAUNCH_CHECK(ctx);
       f3d_stage_end(ctx, F3D_ST_SWEEP_Y);
     }
   } else {
@@ -2290,27 +2285,28 @@ static int yz_sweeps(f3d_hip_ctx* ctx, Scratch* S, double dt, int nf, const RF* 
       for (int c = 0; c < 4; c++) T.q[q][c] = tl[q].m[c];
       T.e_out[q] = tl[q].ey;
     }
-    dim3 gy((m.nx + BXF - 1) / BXF, ((m.ny + ry - 1) / ry) * sp, nf);
+    const dim3 gy((m.nx + BXF - 1) / BXF, ((m.ny + ry - 1) / ry) * gy_grp, nf);
+    const int nrings = m.ny, nvm = nrings * nf;
+    const dim3 g1(nvm + gy.x * gy.y * gy.z);
     f3d_stage_begin(ctx, F3D_ST_SWEEP_Y);
-    if (vm) {
-      const int nrings = m.ny, nvm = nrings * nf;
-      const dim3 g1(nvm + gy.x * gy.y * gy.z);
-      const int ad = (ctx->ph.eos == 2);
-#define Y2V(G_, AD_, SP_)                                                                                     \
-  hipLaunchKernelGGL((kf_sweep_y2v<G_, AD_, SP_>), g1, dim3(BXF), 0, ctx->stream, m, rdt, T, ry, of, *vm, nrings, \
+#define Y2V1(R_, G_, AD_)                                                                                            \
+  hipLaunchKernelGGL((kf_sweep_y2v<G_, AD_, R_>), g1, dim3(BXF), 0, ctx->stream, m, rdt, T, of, *vm, nrings, \
                      nvm, gy)
-#define Y2V_G(G_) \
-  do { if (ad) { if (split) Y2V(G_, 1, 1); else Y2V(G_, 1, 0); } else { if (split) Y2V(G_, 0, 1); else Y2V(G_, 0, 0); } } while (0)
-      if (m.geom == SPH) Y2V_G(SPH); else Y2V_G(CYL);
-#undef Y2V_G
+#define Y2V(G_, AD_) COL_R(ry, Y2V1, G_, AD_)
+#define Y21(R_, G_, AD_) \
+  hipLaunchKernelGGL((kf_sweep_y2<G_, AD_, R_>), gy, dim3(BXF), 0, ctx->stream, m, rdt, T, of)
+#define Y2(G_, AD_) COL_R(ry, Y21, G_, AD_)
+    if (vm) COL_GA(Y2V);
+    else COL_GA(Y2);
+#undef Y2
+#undef Y21
 #undef Y2V
-      F3D_LAUNCH_CHECK(ctx);
-    } else {
-      FDISPATCH_ADS(ctx, kf_sweep_y2, gy, rdt, T, ry, of);
-    }
+#undef Y2V1
+    F3D_LAUNCH_CHECK(ctx);
     f3d_stage_end(ctx, F3D_ST_SWEEP_Y);
   }
-#undef FDISPATCH_ADS
+#undef COL_GA
+#undef COL_R
   return 0;
 }
 

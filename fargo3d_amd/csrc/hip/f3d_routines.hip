@@ -266,7 +266,8 @@ __global__ void k_momenta_x(dmesh m, Range r, const double* rho, const double* v
                             double omegaframe) {
   CELL_INDEX;
   double a, b;
-  cell::momenta_x<G>(m, i, j, k, rho[l], vx[l], vx[lxp_of(l, i, m.nx)], omegaframe, a, b);
+  a = cell::momentum_x<G>(m, j, k, rho[l], vx[l], omegaframe);
+  b = cell::momentum_x<G>(m, j, k, rho[l], vx[lxp_of(l, i, m.nx)], omegaframe);
   mmx[l] = a;
   mpx[l] = b;
 }

@@ -81,6 +81,7 @@ int f3d_hip_create(const f3d_mesh_desc* d, f3d_hip_ctx** out) {
   m.ymed64 = m.ymed; m.sinzmed64 = m.sinzmed; m.sxi64 = m.sxi;
   m.zmed64 = m.zmed; m.sinzmin64 = m.sinzmin; m.coszmin64 = m.coszmin;
   m.vb = nullptr;  // the FP64 form stores full azimuthal velocities
+  m.zy = m.rzy = m.zz = m.rzz = nullptr;
   c->meshlen = total;
   *out = c;
   return 0;

@@ -278,8 +278,8 @@ int f3d_fused_transport(f3d_hip_ctx *ctx, double dt, int end_of_step);
  * fluids in one launch.  VxMed and Nshift end with the last fluid's values. */
 int f3d_fused_transport_fluids(f3d_hip_ctx *ctx, double dt, int nf, const f3d_fields *fl);
 /* Rows (Y sweep; 0: automatic, the default) and planes (Z sweep) one thread
- * marches through; a tuning knob that does not change results.  Returns -2
- * for rows_y below 0 or rows_z below 1. */
+ * updates, rounded down to 4, 2 or 1 (automatic until set); a tuning knob that
+ * does not change results.  Returns -2 for rows_y below 0 or rows_z below 1. */
 int f3d_fused_set_tiling(int rows_y, int rows_z);
 /* X-sweep kernel: 0 automatic (one wave per ring with the cells in
  * registers for rings of 256 cells from 2048 rings x fluids on, else the
@@ -303,10 +303,10 @@ int f3d_fused_set_xtile(int cells);
  * rings x fluids on); the tiled sweep always uses the pass.  Results do not
  * depend on it.  Returns -2 for other values. */
 int f3d_fused_set_xvmed(int form);
-/* Column (Y and Z) sweeps: 1 two threads per column, each with the density
- * and half of the quantities, 0 one thread per column, -1 automatic (split
- * only for sweeps with fewer waves than SIMDs); results do not depend on it.
- * Returns -2 for other values. */
+/* Column (Y and Z) sweeps: 1 one row by two threads, each with the density
+ * and half of the quantities, 0 never so (at least two rows per thread), -1
+ * automatic (on the smallest meshes); results do not depend on it.  Returns -2
+ * for other values. */
 int f3d_fused_set_colsplit(int split);
 /* Form of the fused CFL, bits: 1 ring minima to an array and a
  * one-workgroup second pass (else one 64-bit atomic MIN per ring); 2 the
