@@ -70,6 +70,9 @@ int f3d_hip_create(const f3d_mesh_desc* d, f3d_hip_ctx** out) {
   if (e == hipSuccess) e = hipMalloc(&c->dred, (c->n2 + 64) * sizeof(double));
   if (e == hipSuccess) e = hipHostMalloc((void**)&c->hres, 64 * sizeof(double), hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&c->dhres, c->hres, 0);
+  // pinned memory comes back with what its last owner left in it, and a handle's
+  // first wait must not see another's sequence number (cfl_seq) there
+  if (e == hipSuccess) memset(c->hres, 0, 64 * sizeof(double));
   if (e != hipSuccess) {
     snprintf(g_create_err, sizeof(g_create_err), "f3d_hip_create: %s", hipGetErrorString(e));
     f3d_hip_destroy(c);
