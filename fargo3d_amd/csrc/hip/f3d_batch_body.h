@@ -55,7 +55,10 @@ struct BInst {
 };
 
 // the stages, each with its own per-instance workgroup counts
-enum { BK_CFL = 0, BK_SRCA, BK_SRCB, BK_BND, BK_SWY, BK_VMED, BK_XT, BK_FIN, BK_POT, BK_N };
+// BK_SRC2 the sources of the instances with viscosity and a potential in one
+// pass, BK_SRCA and BK_SRCB those of the others in two; BK_PRE VxMed for the
+// CFL, BK_VMED for the X sweep
+enum { BK_CFL = 0, BK_SRC2, BK_SRCA, BK_SRCB, BK_BND, BK_SWY, BK_VMED, BK_XT, BK_FIN, BK_POT, BK_PRE, BK_N };
 
 __device__ __forceinline__ int find_inst(const int* off, int n, int b) {
   int lo = 0, hi = n;  // off[lo] <= b < off[hi]
@@ -70,35 +73,64 @@ __device__ __forceinline__ int find_inst(const int* off, int n, int b) {
 // local 2-D workgroup index of a grid gx wide
 __device__ __forceinline__ dim3 local2(int lb, int gx) { return dim3(lb % gx, lb / gx, 0); }
 
-__global__ void __launch_bounds__(WG) kb_cfl(const BInst* I, const int* off, int n) {
+// One wave per ring, VxMed from kb_pre: the disks of a batch have many rings of
+// a few hundred cells, of which four waves with four cells per lane leave
+// half idle (44.2 us with 256 threads, 35.8 with 64 or 128).
+__global__ void __launch_bounds__(64) kb_cfl(const BInst* I, const int* off, int n) {
   const int ii = find_inst(off, n, blockIdx.x);
   const BInst& in = I[ii];
-  kd_cfl<CYL, 0, 0>((int)blockIdx.x - off[ii], in.m, in.cs, in.rho, in.vx, in.vy, in.vy, in.vx, in.vxmed,
+  kd_cfl<CYL, 0, 1>((int)blockIdx.x - off[ii], in.m, in.cs, in.rho, in.vx, in.vy, in.vy, in.vx, in.vxmed,
                     in.res, 0, in.cp, nullptr);
 }
 
 // Potential (src/potential.c:51-208) of every instance with planets, FP64:
 // the star's term, each planet's softened term and its indirect term, at the
 // planets' positions at the start of the step (cylindrical 2-D disks).
-__global__ void __launch_bounds__(BXF) kb_potential(const BInst* I, const int* off, int n) {
-  const int ii = find_inst(off, n, blockIdx.x);
-  const BInst& in = I[ii];
-  const int gx = (in.m.nx + BXF - 1) / BXF;
-  const dim3 b = local2(blockIdx.x - off[ii], gx);
-  const int i = b.x * BXF + threadIdx.x;
-  if (i >= in.m.nx) return;
+// A thread takes kPotCells cells of a row, which share the star's term and the
+// planets' distances; the divisions are rdivd()'s.
+constexpr int kPotCells = 4;
+__device__ __forceinline__ void bp_potential(const BInst& in, const dim3 b) {
+  const int i0 = b.x * (kPotCells * BXF) + threadIdx.x, nx = in.m.nx;
   const int j = b.y;
   const BPsys& P = *in.ps;
-  const double r = in.ymed64[j], XC = r * in.cosx64[i], YC = r * in.sinx64[i], ZC = in.zc;
-  double pot = -1.0 / sqrt(r * r + ZC * ZC);
+  const double r = in.ymed64[j], ZC = in.zc;
+  const double star = qdivd(-1.0, sqrt(r * r + ZC * ZC));
+  double pot[kPotCells];
+#pragma unroll
+  for (int u = 0; u < kPotCells; u++) pot[u] = star;
   for (int p = 0; p < P.n; p++) {
-    const double xp = P.x[p], yp = P.y[p], zp = P.z[p], mp = P.pm[p];
+    const double xp = P.x[p], yp = P.y[p], zp = P.z[p], mp = P.pm[p], s2 = P.ps2[p];
     const double d = sqrt(xp * xp + yp * yp + zp * zp);
-    const double dist = (XC - xp) * (XC - xp) + (YC - yp) * (YC - yp) + (ZC - zp) * (ZC - zp);
-    if (P.indirect) pot += mp * (XC * xp + YC * yp + ZC * zp) / (d * d * d);
-    pot += -mp / sqrt(dist + P.ps2[p]);
+    const RecipD D3 = recipd(d * d * d);
+#pragma unroll
+    for (int u = 0; u < kPotCells; u++) {
+      const int i = min(i0 + u * BXF, nx - 1);
+      const double XC = r * in.cosx64[i], YC = r * in.sinx64[i];
+      const double dist = (XC - xp) * (XC - xp) + (YC - yp) * (YC - yp) + (ZC - zp) * (ZC - zp);
+      if (P.indirect) pot[u] += rdivd(mp * (XC * xp + YC * yp + ZC * zp), D3);
+      pot[u] += qdivd(-mp, sqrt(dist + s2));
+    }
   }
-  in.pot[(size_t)j * in.m.pitch + i] = pot;
+#pragma unroll
+  for (int u = 0; u < kPotCells; u++)
+    if (i0 + u * BXF < nx) in.pot[(size_t)j * in.m.pitch + i0 + u * BXF] = pot[u];
+}
+
+// What the CFL and the sources wait for, in one launch: VxMed of the rings the
+// CFL reads (every active row and the one above), one wave each, in the first
+// npre workgroups, and the potential in the others.  Two sequential ring sums in
+// each of the CFL's workgroups left two of its four waves idle meanwhile: for 16
+// disks up to 1536x384, potential and CFL 23.5 + 71.0 us, now 24.0 + 35.8.
+__global__ void __launch_bounds__(64) kb_pre(const BInst* I, const int* offv, int npre, const int* offp, int n) {
+  if ((int)blockIdx.x < npre) {
+    const int ii = find_inst(offv, n, blockIdx.x);
+    const BInst& in = I[ii];
+    kd_vmed_row<CYL, 0, 8>(in.m.nghy + ((int)blockIdx.x - offv[ii]), 0, in.m, in.vx, in.vxmed);
+    return;
+  }
+  const int b = (int)blockIdx.x - npre, ii = find_inst(offp, n, b);
+  const BInst& in = I[ii];
+  bp_potential(in, local2(b - offp[ii], (in.m.nx + kPotCells * BXF - 1) / (kPotCells * BXF)));
 }
 
 // Tapered mass and squared smoothing length of each planet at time t
@@ -124,26 +156,30 @@ __device__ void bp_prepare(BPsys& P, double t) {
 // stays in registers; slots at or beyond P.n are skipped (and hold 1.0).
 template <int NP>
 __device__ __forceinline__ void bp_deriv(const BPsys& P, const double (&q)[6 * NP], double (&d)[6 * NP], double dt) {
-  double rad[NP];
+  // one reciprocal per distance for the three quotients by it: one thread's
+  // serial chain bounds the launch (23.4 -> 15.1 us with one planet)
+  RecipD rad[NP];
 #pragma unroll
-  for (int i = 0; i < NP; i++) rad[i] = sqrt(q[i] * q[i] + q[NP + i] * q[NP + i] + q[2 * NP + i] * q[2 * NP + i]);
+  for (int i = 0; i < NP; i++)
+    rad[i] = recipd(sqrt(q[i] * q[i] + q[NP + i] * q[NP + i] + q[2 * NP + i] * q[2 * NP + i]));
 #pragma unroll
   for (int i = 0; i < NP; i++) {
     double a[3];
 #pragma unroll
-    for (int c = 0; c < 3; c++) a[c] = -q[c * NP + i] / rad[i] / rad[i] / rad[i];
+    for (int c = 0; c < 3; c++) a[c] = rdivd(rdivd(rdivd(-q[c * NP + i], rad[i]), rad[i]), rad[i]);
 #pragma unroll
     for (int k = 0; k < NP; k++) {
       if (k >= P.n) continue;
       if (P.indirect) {
-        const double cf = P.m[k] / rad[k] / rad[k] / rad[k];
+        const double cf = rdivd(rdivd(rdivd(P.m[k], rad[k]), rad[k]), rad[k]);
 #pragma unroll
         for (int c = 0; c < 3; c++) a[c] -= cf * q[c * NP + k];
       }
       if (k != i && P.feelothers[i]) {
         const double dx = q[k] - q[i], dy = q[NP + k] - q[NP + i], dz = q[2 * NP + k] - q[2 * NP + i];
         const double sd = sqrt(dx * dx + dy * dy + dz * dz);
-        const double cf = P.m[k] / sd / sd / sd;
+        const RecipD S = recipd(sd);
+        const double cf = rdivd(rdivd(rdivd(P.m[k], S), S), S);
         a[0] += cf * dx;
         a[1] += cf * dy;
         a[2] += cf * dz;
@@ -298,6 +334,23 @@ __global__ void __launch_bounds__(64) kb_dt(BInst* I, int n) {
   c[2] += dt;
 }
 
+// the one-pass sources (kd_src_fused2), kBSrcRows rows per lane: 58.5 us for 16
+// disks up to 1536x384, 62.4 with 8 rows, the two passes 68.4
+constexpr int kBSrcRows = 4;
+__global__ void __launch_bounds__(64) kb_src2(const BInst* I, const int* off, int n) {
+  const int ii = find_inst(off, n, blockIdx.x);
+  const BInst& in = I[ii];
+  const dim3 b = local2(blockIdx.x - off[ii], (in.m.nx + kSrcCols - 1) / kSrcCols);
+  const real dt = (real)in.clk[0];
+  const int je = in.m.ny + in.m.nghy;
+  if (in.vp.model == 1)
+    kd_src_fused2<CYL, 1, 1>(b, in.m, dt, in.rho, in.cs, in.vx, in.vy, in.pot, in.vxt, in.vyt, in.e2, in.vp, (real)0,
+                             in.of64, in.domega, kBSrcRows, je);
+  else
+    kd_src_fused2<CYL, 1, 2>(b, in.m, dt, in.rho, in.cs, in.vx, in.vy, in.pot, in.vxt, in.vyt, in.e2, in.vp, (real)0,
+                             in.of64, in.domega, kBSrcRows, je);
+}
+
 __global__ void __launch_bounds__(BXF) kb_src_a(const BInst* I, const int* off, int n) {
   const int ii = find_inst(off, n, blockIdx.x);
   const BInst& in = I[ii];
@@ -324,21 +377,23 @@ __global__ void __launch_bounds__(BXF) kb_bound(const BInst* I, const int* off, 
              in.cs, in.b0, in.b1, in.ydexp0, in.ydexp1);
 }
 
+// the Y sweep with the X sweep's VxMed in the same launch (kf_sweep_y2v; 57.2 us,
+// two launches 48.1 + 19.8): one
+// wave per ring in the first nvm workgroups, 8 terms per lane (the instances'
+// rings hold 256 to a few thousand cells)
 template <int R>
-__global__ void __launch_bounds__(BXF) kb_sweep_y(const BInst* I, const int* off, int n) {
-  const int ii = find_inst(off, n, blockIdx.x);
+__global__ void __launch_bounds__(BXF) kb_sweep_y(const BInst* I, const int* offv, int nvm, const int* off, int n) {
+  if ((int)blockIdx.x < nvm) {
+    const int ii = find_inst(offv, n, blockIdx.x);
+    const BInst& in = I[ii];
+    kd_vmed<CYL, 0, 8>(dim3(blockIdx.x - offv[ii]), in.m, in.vxt, in.vxmed);
+    return;
+  }
+  const int b = (int)blockIdx.x - nvm, ii = find_inst(off, n, b);
   const BInst& in = I[ii];
   const int gx = (in.m.nx + BXF - 1) / BXF;
-  kd_sweep_y2<CYL, 0, R>(local2(blockIdx.x - off[ii], gx), in.m, (real)in.clk[0], in.rho, in.vxt, in.vyt, in.cs,
-                         in.rhoy, in.mpx, in.mmx, in.mpy, in.mmy, in.ey, in.of);
-}
-
-// one wave per ring, 8 terms per lane (the instances' rings hold 256 to a few
-// thousand cells)
-__global__ void __launch_bounds__(64) kb_vmed(const BInst* I, const int* off, int n) {
-  const int ii = find_inst(off, n, blockIdx.x);
-  const BInst& in = I[ii];
-  kd_vmed<CYL, 0, 8>(dim3(blockIdx.x - off[ii]), in.m, in.vxt, in.vxmed);
+  kd_sweep_y2<CYL, 0, R>(local2(b - off[ii], gx), in.m, (real)in.clk[0], in.rho, in.vxt, in.vyt, in.cs, in.rhoy,
+                         in.mpx, in.mmx, in.mpy, in.mmy, in.ey, in.of);
 }
 
 // tiles of 64*CPT cells, one wave each
@@ -379,6 +434,7 @@ struct f3d_batch {
   int nxmax = 0;
   int rows_y = 4, tile = 128;
   std::vector<int> has_ps;  // instance has a planetary system on the device
+  std::vector<int> src2;    // its sources run in one pass
   int npmax = 0;            // the largest planet count
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -416,12 +472,14 @@ static int batch_layout(f3d_batch* B) {
     const f3d::dmesh& m = f3d_sim_ctx(B->sims[i])->m;
     const int gx = (m.nx + BXF - 1) / BXF;
     c[BK_CFL][i] = m.ny;
-    c[BK_SRCA][i] = gx * (m.sy - 2);
-    c[BK_SRCB][i] = gx * m.ny;
+    c[BK_PRE][i] = m.ny + 1;
+    c[BK_SRC2][i] = B->src2[i] ? (m.nx + kSrcCols - 1) / kSrcCols * ((m.ny + kBSrcRows - 1) / kBSrcRows) : 0;
+    c[BK_SRCA][i] = B->src2[i] ? 0 : gx * (m.sy - 2);
+    c[BK_SRCB][i] = B->src2[i] ? 0 : gx * m.ny;
     c[BK_BND][i] = gx * 2;  // one block row per side, all ghost layers per thread
     c[BK_VMED][i] = m.ny;
     c[BK_FIN][i] = gx * m.ny;
-    c[BK_POT][i] = B->has_ps[i] ? gx * m.sy : 0;
+    c[BK_POT][i] = B->has_ps[i] ? (m.nx + kPotCells * BXF - 1) / (kPotCells * BXF) * m.sy : 0;
     const int ry = column_form(B->rows_y);
     swy[i] = gx * ((m.ny + ry - 1) / ry) * (ry == 1 ? 2 : 1);
     xt[i] = ((m.nx + x_tile_out(B->tile / 64) - 1) / x_tile_out(B->tile / 64)) * m.ny;
@@ -437,22 +495,26 @@ static int batch_layout(f3d_batch* B) {
 static void batch_launch(f3d_batch* B) {
   const int n = B->n;
   hipStream_t s = B->stream;
-  if (B->total[BK_POT])
-    hipLaunchKernelGGL(kb_potential, dim3(B->total[BK_POT]), dim3(BXF), 0, s, B->dI, B->doff[BK_POT], n);
-  hipLaunchKernelGGL(kb_cfl, dim3(B->total[BK_CFL]), dim3(WG), cfl_lds(0), s, B->dI, B->doff[BK_CFL], n);
+  hipLaunchKernelGGL(kb_pre, dim3(B->total[BK_PRE] + B->total[BK_POT]), dim3(64), 0, s, B->dI, B->doff[BK_PRE],
+                     B->total[BK_PRE], B->doff[BK_POT], n);
+  hipLaunchKernelGGL(kb_cfl, dim3(B->total[BK_CFL]), dim3(64), cfl_lds(1), s, B->dI, B->doff[BK_CFL], n);
   if (B->npmax <= 1) hipLaunchKernelGGL(kb_dt<1>, dim3((n + 63) / 64), dim3(64), 0, s, B->dI, n);
   else if (B->npmax <= 2) hipLaunchKernelGGL(kb_dt<2>, dim3((n + 63) / 64), dim3(64), 0, s, B->dI, n);
   else if (B->npmax <= 4) hipLaunchKernelGGL(kb_dt<4>, dim3((n + 63) / 64), dim3(64), 0, s, B->dI, n);
   else hipLaunchKernelGGL(kb_dt<kBP>, dim3((n + 63) / 64), dim3(64), 0, s, B->dI, n);
-  hipLaunchKernelGGL(kb_src_a, dim3(B->total[BK_SRCA]), dim3(BXF), 0, s, B->dI, B->doff[BK_SRCA], n);
-  hipLaunchKernelGGL(kb_src_b, dim3(B->total[BK_SRCB]), dim3(BXF), 0, s, B->dI, B->doff[BK_SRCB], n);
+  if (B->total[BK_SRC2])
+    hipLaunchKernelGGL(kb_src2, dim3(B->total[BK_SRC2]), dim3(64), 0, s, B->dI, B->doff[BK_SRC2], n);
+  if (B->total[BK_SRCB]) {
+    hipLaunchKernelGGL(kb_src_a, dim3(B->total[BK_SRCA]), dim3(BXF), 0, s, B->dI, B->doff[BK_SRCA], n);
+    hipLaunchKernelGGL(kb_src_b, dim3(B->total[BK_SRCB]), dim3(BXF), 0, s, B->dI, B->doff[BK_SRCB], n);
+  }
   hipLaunchKernelGGL(kb_bound, dim3(B->total[BK_BND]), dim3(BXF), 0, s, B->dI, B->doff[BK_BND], n, 1);
   const int ry = column_form(B->rows_y);
-  if (ry == 4) hipLaunchKernelGGL(kb_sweep_y<4>, dim3(B->swy_total), dim3(BXF), 0, s, B->dI, B->dswy, n);
-  else if (ry == 2) hipLaunchKernelGGL(kb_sweep_y<2>, dim3(B->swy_total), dim3(BXF), 0, s, B->dI, B->dswy, n);
-  else hipLaunchKernelGGL(kb_sweep_y<1>, dim3(B->swy_total), dim3(BXF), 0, s, B->dI, B->dswy, n);
-  hipLaunchKernelGGL(kb_vmed, dim3(B->total[BK_VMED]), dim3(64), 0, s, B->dI,
-                     B->doff[BK_VMED], n);
+  const int nvm = B->total[BK_VMED];
+  const dim3 gy(nvm + B->swy_total);
+  if (ry == 4) hipLaunchKernelGGL(kb_sweep_y<4>, gy, dim3(BXF), 0, s, B->dI, B->doff[BK_VMED], nvm, B->dswy, n);
+  else if (ry == 2) hipLaunchKernelGGL(kb_sweep_y<2>, gy, dim3(BXF), 0, s, B->dI, B->doff[BK_VMED], nvm, B->dswy, n);
+  else hipLaunchKernelGGL(kb_sweep_y<1>, gy, dim3(BXF), 0, s, B->dI, B->doff[BK_VMED], nvm, B->dswy, n);
   if (B->tile == 64) hipLaunchKernelGGL(kb_sweep_x<1>, dim3(B->xt_total), dim3(64), 0, s, B->dI, B->dxt, n);
   else if (B->tile == 256) hipLaunchKernelGGL(kb_sweep_x<4>, dim3(B->xt_total), dim3(64), 0, s, B->dI, B->dxt, n);
   else hipLaunchKernelGGL(kb_sweep_x<2>, dim3(B->xt_total), dim3(64), 0, s, B->dI, B->dxt, n);
@@ -547,6 +609,7 @@ f3d_batch* f3d_batch_create(int n, const char* const* parfiles, const char* cons
   if (hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking) != hipSuccess) return fail("stream creation failed");
   std::vector<BPsys> hps(n);
   B->has_ps.assign(n, 0);
+  B->src2.assign(n, 0);
   if (hipMalloc(&B->dclk, clk.size() * sizeof(double)) != hipSuccess ||
       hipMalloc(&B->dres, 2 * (size_t)n * sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc(&B->dps, (size_t)n * sizeof(BPsys)) != hipSuccess)
@@ -593,6 +656,7 @@ f3d_batch* f3d_batch_create(int n, const char* const* parfiles, const char* cons
     b.of64 = c->ph.OMEGAFRAME;
     b.visc = c->ph.visc != 0 && c->ph.fluidtype == 1;
     b.potential = c->ph.potential;
+    B->src2[i] = b.visc && b.potential && (b.vp.model == 1 || b.vp.model == 2);
     b.stockholm = c->ph.stockholm;
     b.fargo = c->ph.fargo;
     b.domega = (real)0;

@@ -595,9 +595,8 @@ __device__ __forceinline__ double cfl_sumsq(const dmesh& m, int i, int j, int k,
     vxxp = vx1 - vxmed;
   }
   const double c0 = cs[l];
-  double soundspeed2, viscosity;
-  if (cp.iso) soundspeed2 = c0 * c0;
-  else soundspeed2 = qdivd(cp.gamma * (cp.gamma - 1) * c0, (double)rho[l]);
+  double soundspeed2 = 0.0, viscosity;
+  if (!cp.iso) soundspeed2 = qdivd(cp.gamma * (cp.gamma - 1) * c0, (double)rho[l]);
   if (cp.alpha_visc) {
     const double y = m.ymed64[j];
     const double sq = sqrt(y * y * y / (1.0 * 1.0));
@@ -606,7 +605,9 @@ __device__ __forceinline__ double cfl_sumsq(const dmesh& m, int i, int j, int k,
   } else {
     viscosity = cp.nu;
   }
-  const double soundspeed = sqrt(soundspeed2);
+  // isothermal: sqrt(c0*c0) is |c0| in binary floating point (the square's
+  // rounding error is too small to move the root)
+  const double soundspeed = cp.iso ? fabs(c0) : sqrt(soundspeed2);
   // every quotient below divides by one of the three zone sizes: one
   // reciprocal each, shared (RecipD), with zmin's the one of the smallest
   const double zx = zone_size_x64<G>(m, i, j, k), zy = zone_size_y64(m, j);

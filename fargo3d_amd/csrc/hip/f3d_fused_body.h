@@ -348,17 +348,20 @@ __global__ void __launch_bounds__(WG) kf_cfl(dmesh m, const real* __restrict__ c
   kd_cfl<G, DZ, PRE>(xcd_linear(), m, cs, rho, vx, vy, vz, vxm, vxmed, result, slot, cp, ringmin);
 }
 
-// ComputeVmed (src/compute_vmed.c:14-30) of rings j = NGHY .. NGHY+nry-1 of
-// every active plane: one wave per ring, one sequential sum in i order with
-// S terms per lane (wave_ring_sum).
+// ComputeVmed (src/compute_vmed.c:14-30) of ring (j, k) by one wave, one
+// sequential sum in i order with S terms per lane (wave_ring_sum).
+template <int G, int DZ, int S>
+__device__ __forceinline__ void kd_vmed_row(int j, int k, const dmesh& m, const real* __restrict__ v, double* __restrict__ vxmed) {
+  __shared__ double sh[f3d_ring::lds_doubles(S)];
+  const double sum = wave_ring_sum<S>(v + j * m.pitch + k * m.stride, m, sh);
+  if (threadIdx.x == 0) vxmed[j + k * m.sy] = vmed_full(sum / (m.XMAX - m.XMIN), m, j, k);
+}
+// the same of rings j = NGHY .. NGHY+nry-1 of every active plane
 template <int G, int DZ, int S>
 __global__ void __launch_bounds__(64) kf_vmed_rings(dmesh m, const real* __restrict__ v, double* __restrict__ vxmed, int nry) {
   const int j = m.nghy + (int)(blockIdx.x % nry);
   const int k = DZ ? m.nghz + (int)(blockIdx.x / nry) : 0;
-  const int base = j * m.pitch + k * m.stride;
-  __shared__ double sh[f3d_ring::lds_doubles(S)];
-  const double sum = wave_ring_sum<S>(v + base, m, sh);
-  if (threadIdx.x == 0) vxmed[j + k * m.sy] = vmed_full(sum / (m.XMAX - m.XMIN), m, j, k);
+  kd_vmed_row<G, DZ, S>(j, k, m, v, vxmed);
 }
 
 // The cfl of nf fluids in one launch: nf consecutive blocks of nrings
@@ -573,17 +576,16 @@ struct StressAt {
 };
 constexpr int kSrcCols = 62;  // cells a wave of kf_src_fused2 updates
 template <int G, int MODE, int VM>
-__global__ void __launch_bounds__(64) kf_src_fused2(dmesh m, real dt, const real* __restrict__ rho,
-                                                    const real* __restrict__ energy, const real* __restrict__ vx,
-                                                    const real* __restrict__ vy, const double* __restrict__ pot,
-                                                    real* __restrict__ vxt, real* __restrict__ vyt,
-                                                    real* __restrict__ e2, cell::ViscPar vp, real gm1,
-                                                    double omegaframe, real domega, int rows_per, int jend) {
+__device__ __forceinline__ void kd_src_fused2(const dim3 b, const dmesh& m, real dt, const real* __restrict__ rho,
+                                              const real* __restrict__ energy, const real* __restrict__ vx,
+                                              const real* __restrict__ vy, const double* __restrict__ pot,
+                                              real* __restrict__ vxt, real* __restrict__ vyt,
+                                              real* __restrict__ e2, cell::ViscPar vp, real gm1,
+                                              double omegaframe, real domega, int rows_per, int jend) {
   constexpr int iso = MODE == 1;
   vp.model = VM == 1 ? 1 : 2;
   vp.iso = VM != 3;
   const int lane = (int)threadIdx.x;
-  const dim3 b = xcd_bid();
   const int is = kSrcCols * (int)b.x - 1 + lane;  // this lane's stress column
   const int i = is < 0 ? is + m.nx : (is >= m.nx ? is - m.nx : is);
   const bool upd = lane >= 1 && lane <= kSrcCols && is < m.nx;
@@ -628,6 +630,16 @@ __global__ void __launch_bounds__(64) kf_src_fused2(dmesh m, real dt, const real
     Tm = T0;
     T0 = Tp;
   }
+}
+template <int G, int MODE, int VM>
+__global__ void __launch_bounds__(64) kf_src_fused2(dmesh m, real dt, const real* __restrict__ rho,
+                                                    const real* __restrict__ energy, const real* __restrict__ vx,
+                                                    const real* __restrict__ vy, const double* __restrict__ pot,
+                                                    real* __restrict__ vxt, real* __restrict__ vyt,
+                                                    real* __restrict__ e2, cell::ViscPar vp, real gm1,
+                                                    double omegaframe, real domega, int rows_per, int jend) {
+  kd_src_fused2<G, MODE, VM>(xcd_bid(), m, dt, rho, energy, vx, vy, pot, vxt, vyt, e2, vp, gm1, omegaframe, domega,
+                             rows_per, jend);
 }
 
 // kf_src_b of every fluid in one launch (isothermal runs): blockIdx.z =
@@ -1359,10 +1371,7 @@ template <int G, int DZ, int S>
 __device__ __forceinline__ void kd_vmed(const dim3 bid, const dmesh& m, const real* vxt, double* vxmed) {
   const int j = m.nghy + (int)(bid.x % m.ny);
   const int k = DZ ? m.nghz + (int)(bid.x / m.ny) : 0;
-  const int base = j * m.pitch + k * m.stride;
-  __shared__ double sh[f3d_ring::lds_doubles(S)];
-  const double sum = wave_ring_sum<S>(vxt + base, m, sh);
-  if (threadIdx.x == 0) vxmed[j + k * m.sy] = vmed_full(sum / (m.XMAX - m.XMIN), m, j, k);
+  kd_vmed_row<G, DZ, S>(j, k, m, vxt, vxmed);
 }
 template <int G, int DZ, int S>
 __global__ void __launch_bounds__(64) kf_vmed(dmesh m, VmTab T, int nrings) {
