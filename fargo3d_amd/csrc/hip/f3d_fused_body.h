@@ -2086,13 +2086,20 @@ static int g_y2v = -1;
 // atomic MIN per ring), 2 VxMed from kf_vmed_rings, 4 (with 2) one wave per
 // workgroup.  Measured on MI355X: the array and its MIN pass, which hands
 // dt to the host itself, pay on every mesh (the atomic form's copy and event
-// cost more: 384x128 step 0.0609 -> 0.0561 ms, 4096x1024 alike); the VxMed
-// pass for many or long rings, one wave per ring for rings of <= 256 cells.
+// cost more: 384x128 step 0.0609 -> 0.0561 ms, 4096x1024 alike).  The VxMed pass
+// (us, in-kernel sums / pass) for many rings, 256x96x32 35.8 / 18.7, five fluids
+// on 1024x512 40.5 / 27.4, and for the conversions and longer sums of FP32
+// deviations, 600x300 x3 19.4 / 17.0, 1024x512 21.4 / 19.2, 4096x1024 57.9 / 50.3;
+// in FP64 two sums side by side in the ring's own workgroup are as fast or
+// faster, 1024x512 14.3 / 16.5, 1250x437 17.1 / 18.5, 4096x1024 49.7 / 52.  Among many
+// rings one wave each, four / one wave: 256x96x32 33.0 / 18.7, 500x150x45 65.4 / 45.4,
+// 1024x512 x5 27.0 / 27.3.
 static int cfl_mode(const dmesh& m, int nf) {
   if (g_cflmode >= 0) return g_cflmode;
   const int nrings = m.ny * (m.dimz ? m.nz : 1) * nf;
-  int mode = 1 | (nrings >= 2048 ? 2 : 0) | (m.nx >= 1024 ? 2 : 0);
-  if ((mode & 2) && m.nx <= 256) mode |= 4;
+  int mode = 1;
+  if (nrings >= 2048 || (cell::kFix64 && m.nx >= 512)) mode |= 2;
+  if (nrings >= 2048 && m.nx < 1024) mode |= 4;
   return mode;
 }
 
@@ -2101,7 +2108,9 @@ static int cfl_mode(const dmesh& m, int nf) {
 // 13.6 with 8), else 8 (7150 rings of 500 cells 10.3 us against 13.7 with 16
 // and 11.9 with 4).
 static int g_vmed_terms = -1;
-static int vmed_terms(int nx) { return g_vmed_terms > 0 ? g_vmed_terms : nx >= 2048 ? 16 : 8; }
+static int vmed_terms(int nx) {
+  return g_vmed_terms > 0 ? g_vmed_terms : nx >= (cell::kFix64 ? 512 : 2048) ? 16 : 8;
+}
 
 // VxMed of every active ring and of the ring above the last (the shear limit
 // reads ring j+1), for the CFL kernel's pre-pass form: one wave per ring
