@@ -12,20 +12,20 @@
 // intermediates on chip:
 //
 //   kf_cfl         ring-owning: VxMed of the ring and of the next ring
-//                  (sequential sums, in parallel, or from kf_vmed_rings),
+//                  (ordered sums, in parallel, or from kf_vmed_rings),
 //                  per-cell CFL, shear limit, one MIN per ring (atomic, or
 //                  into an array that kf_cfl_fin reduces) -> dt, 8 bytes to host
 //   kf_src_a       viscous stress and artificial pressure at every cell the
 //                  next kernel reads
 //   kf_src_b       SubStep1 + addviscosity + SubStep2_b on active cells
 //   (boundaries)   mid-step ghost fill on V_temp
-//   kf_sweep_z     3-D: momenta + Z sweep, one thread per (i,j) column
-//                  marching in k over a register window
-//   kf_sweep_y     momenta (2-D) + Y sweep, columns marching in j
-//   kf_sweep_xr_fluids ring-owning (every fluid in one launch): VxMed,
-//                  residual, van Leer and PPA X sweeps, integer shift and
-//                  NewVelocity_x, cell state in registers, stencils in LDS
-//   kf_sweep_x_tile the same X sweep on tiles with halos, for long rings
+//   kf_sweep_z     3-D: momenta + Z sweep, a thread holding up to 4 planes of
+//                  a column and their halo in registers; VxMed of Vx_temp in
+//                  workgroups of their own (kf_sweep_y2v: the same in 2-D)
+//   kf_sweep_y2/y3 momenta (2-D) + Y sweep, the same over rows
+//   kf_sweep_x     residual, van Leer and PPA X sweeps, integer shift and
+//                  NewVelocity_x on one-wave tiles of the rings, one to four
+//                  cells per lane, neighbours by wave rotation
 //   kf_finish      NewVelocity_y/z and Stockholm damping
 //   (boundaries)   end-of-step ghost fill
 //
@@ -507,7 +507,11 @@ __global__ void __launch_bounds__(WG) kf_src_a(dmesh m, const real* __restrict__
 // active cells, in the order the reference applies them.  MODE fixes the
 // flags of a viscous gas with a potential at compile time (1 isothermal, 2
 // adiabatic; 0: the flags as passed), so that no branch separates the
-// stencil's loads.
+// stencil's loads.  Memory latency bounds it: in 3-D 118 VGPRs (4 waves per SIMD)
+// for the gathered loads beat the 5 waves of the branching form, 256x96x32 35.4 ->
+// 27.5 us (FP32 23.6 -> 18.0), 500x150x45 180 -> 152 us.  Two rows per thread gave
+// 32.3 and 150, an order of workgroups that keeps three planes of a strip of
+// rows in L2 27.9 and 151.
 template <int G, int DZ, int MODE = 0>
 __device__ __forceinline__ void kd_src_b(const dim3 bid, const dmesh& m, real dt, const real* __restrict__ rho, const real* __restrict__ energy, const real* __restrict__ vx, const real* __restrict__ vy, const real* __restrict__ vz, const double* __restrict__ pot, const real* __restrict__ txx, const real* __restrict__ tyy, const real* __restrict__ tzz, const real* __restrict__ txz, const real* __restrict__ tyx, const real* __restrict__ tzy, real* __restrict__ vxt, real* __restrict__ vyt, real* __restrict__ vzt, real* __restrict__ e2, int visc, int potential, int dust, int iso, real gm1, double omegaframe, real domega) {
   if constexpr (MODE != 0) {
@@ -548,7 +552,7 @@ __device__ __forceinline__ void kd_src_b(const dim3 bid, const dmesh& m, real dt
   if (!iso) e2[l] = e;
 }
 template <int G, int DZ, int MODE>
-__global__ void __launch_bounds__(WG, DZ ? 5 : 8) kf_src_b(dmesh m, real dt, const real* __restrict__ rho, const real* __restrict__ energy,
+__global__ void __launch_bounds__(BXF, DZ ? 4 : 8) kf_src_b(dmesh m, real dt, const real* __restrict__ rho, const real* __restrict__ energy,
                                                const real* __restrict__ vx, const real* __restrict__ vy, const real* __restrict__ vz,
                                                const double* __restrict__ pot, const real* __restrict__ txx, const real* __restrict__ tyy,
                                                const real* __restrict__ tzz, const real* __restrict__ txz, const real* __restrict__ tyx,
@@ -2925,8 +2929,9 @@ int F3D_API(fused_sources)(f3d_hip_ctx* ctx, double dt, double domega) {
   dim3 gb((m.nx + BXF - 1) / BXF, m.ny + ext, m.dimz ? m.nz + ext : 1);
   f3d_stage_begin(ctx, F3D_ST_SRC_B);
   // measured on MI355X: the fixed flags pay in 2-D (adiabatic 4096x1024 step
-  // 0.662 -> 0.645 ms); in 3-D the kernel took longer (34.5 -> 38.8 us)
-  const int mode = (visc && pot && !dust && !m.dimz) ? (iso ? 1 : 2) : 0;
+  // 0.662 -> 0.645 ms) and, with the registers for the loads they let the
+  // compiler gather, in 3-D (kf_src_b)
+  const int mode = (visc && pot && !dust) ? (iso ? 1 : 2) : 0;
 #define SRCB(MODE_) FDISPATCH_T(ctx, kf_src_b, MODE_, gb, dim3(BXF), 0, rdt, f.Density, f.Energy, f.Vx, f.Vy, f.Vz, \
                                 ctx->f.Pot, f.Mmx, f.Mmy, f.Mmz, f.Mpx, f.Mpy, f.Mpz, f.Vx_temp, f.Vy_temp,        \
                                 f.Vz_temp, S->f[FS_E2], visc, pot, dust, iso, (real)(ctx->ph.gamma - 1.0),        \
