@@ -281,27 +281,24 @@ int f3d_fused_transport_fluids(f3d_hip_ctx *ctx, double dt, int nf, const f3d_fi
  * updates, rounded down to 4, 2 or 1 (automatic until set); a tuning knob that
  * does not change results.  Returns -2 for rows_y below 0 or rows_z below 1. */
 int f3d_fused_set_tiling(int rows_y, int rows_z);
-/* X-sweep kernel: 0 automatic (one wave per ring with the cells in
- * registers for rings of 256 cells from 2048 rings x fluids on, else the
- * ring in LDS when it fits, else tiles of 256 cells with halos, one wave
- * each, the cells in registers), 1 ring in LDS, 2 tiles of 128 cells in LDS,
- * 3 one wave per ring (rings of 256 cells; others as 0), 4 one-wave tiles;
- * results do not depend on it.  Returns -2 for other values. */
+/* X-sweep form: 0 (and 1) automatic (one-wave tiles of 64 to 256 cells by ring
+ * length and count, one wave per ring on many rings of 256 cells), 2 tiles of
+ * the size of f3d_fused_set_xtile, 3 one wave per ring (rings of 256 cells;
+ * others as 0), 4 tiles of 256 cells; results do not depend on it.  Returns
+ * -2 for other values. */
 int f3d_fused_set_xmode(int mode);
-/* Ring X sweep: 1 two workgroups per ring, each carrying the density and
- * half of the transported quantities (about half the LDS, so more
- * workgroups per CU), 0 one workgroup per ring, -1 automatic; results do not
- * depend on it.  Returns -2 for other values. */
+/* X sweep: 1 a tile's quantities dealt to several waves, two each (and the
+ * density in every one), 0 one wave, -1 automatic; results do not depend on
+ * it.  Returns -2 for other values. */
 int f3d_fused_set_xsplit(int split);
-/* Cells per workgroup of the tiled X sweep: 64, 128 (default) or 256;
+/* Cells per tile of X-sweep form 2: 64, 128 (default) or 256;
  * results do not depend on it.  Returns -2 for other values. */
 int f3d_fused_set_xtile(int cells);
-/* Where the ring X sweep takes each ring's VxMed (ComputeVmed of Vx_temp,
- * src/compute_vmed.c:14-30) from: 0 its own sequential sum, 1 a one-wave-
- * per-ring pass on a second stream that overlaps the Z/Y sweeps, 2 that pass
- * on the step's stream just before the X sweep, -1 automatic (1 from 1024
- * rings x fluids on); the tiled sweep always uses the pass.  Results do not
- * depend on it.  Returns -2 for other values. */
+/* Where the X sweep's VxMed pass (ComputeVmed of Vx_temp,
+ * src/compute_vmed.c:14-30, one wave per ring) runs: 2 on the step's stream
+ * just before the X sweep, 0, 1 and -1 (automatic) beside the Z/Y sweeps; a wave
+ * that holds a whole ring sums its own.  Results do not depend on it.  Returns
+ * -2 for other values. */
 int f3d_fused_set_xvmed(int form);
 /* Column (Y and Z) sweeps: 1 one row by two threads, each with the density
  * and half of the quantities, 0 never so (at least two rows per thread), -1
