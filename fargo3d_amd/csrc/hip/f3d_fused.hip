@@ -6,6 +6,7 @@
 
 #include "f3d_internal.h"
 #include "f3d_cell.h"
+#include "f3d_columns.h"
 #include "f3d_ringsum.h"
 
 #define F3D_NS f3d

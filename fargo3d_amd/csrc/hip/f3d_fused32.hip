@@ -9,6 +9,7 @@
 
 #include "f3d_internal.h"
 #include "f3d_cell32.h"
+#include "f3d_columns.h"
 #include "f3d_ringsum.h"
 
 #define F3D_NS f3d32

@@ -570,7 +570,7 @@ __global__ void __launch_bounds__(BXF, DZ ? 4 : 8) kf_src_b(dmesh m, real dt, co
 // rows per segment); the x neighbours' stresses come from the next lanes by
 // wave rotation.  A wave holds 64 stress columns, i0-1 .. i0+62, and updates
 // the 62 cells between (waves overlap by two columns), so every neighbour a
-// cell reads is in the wave.  MODE as kd_src_b (1 isothermal, 2 adiabatic),
+// cell reads is in the wave (f3d_columns.h).  MODE as kd_src_b (1 isothermal, 2 adiabatic),
 // VM as kd_src_a (1 constant nu, 2 alpha isothermal, 3 alpha adiabatic).
 struct StressAt {
   real c, xm, xp, ym, yp;  // at the cell, its x-1, x+1, y-1 and y+1 neighbours
@@ -578,7 +578,6 @@ struct StressAt {
     return di < 0 ? xm : di > 0 ? xp : dj < 0 ? ym : dj > 0 ? yp : c;
   }
 };
-constexpr int kSrcCols = 62;  // cells a wave of kf_src_fused2 updates
 template <int G, int MODE, int VM>
 __device__ __forceinline__ void kd_src_fused2(const dim3 b, const dmesh& m, real dt, const real* __restrict__ rho,
                                               const real* __restrict__ energy, const real* __restrict__ vx,
@@ -590,9 +589,8 @@ __device__ __forceinline__ void kd_src_fused2(const dim3 b, const dmesh& m, real
   vp.model = VM == 1 ? 1 : 2;
   vp.iso = VM != 3;
   const int lane = (int)threadIdx.x;
-  const int is = kSrcCols * (int)b.x - 1 + lane;  // this lane's stress column
-  const int i = is < 0 ? is + m.nx : (is >= m.nx ? is - m.nx : is);
-  const bool upd = lane >= 1 && lane <= kSrcCols && is < m.nx;
+  const int is = src_position((int)b.x, lane), i = src_cell(is, m.nx);  // this lane's stress column
+  const bool upd = src_updates(is, lane, m.nx);
   const int r0 = m.nghy + (int)b.y * rows_per;
   const int r1 = min(r0 + rows_per, jend);
   // visctensor (src/visctensor_cyl.c:140-186, src/visctensor_sph.c:126-206)
