@@ -12,8 +12,9 @@ C1 = "fargo3d_amd/setups/c1_fargo2d.par"
 C3 = "fargo3d_amd/setups/c3_adiabatic2d.par"
 
 
-@pytest.mark.parametrize("ov", ["Nx=12 Ny=9 Nu=1e-5", "Nx=16 Ny=14 Nu=0.0 Alpha=1e-3", "Nx=20 Ny=13 Nu=1e-4",
-                                "Nx=31 Ny=12 Nu=1e-5", "Nx=32 Ny=16 Nu=0.0 Alpha=1e-3"])
+@pytest.mark.parametrize("ov", ["Nx=12 Ny=9 Nu=1e-5", "Nx=16 Ny=14 ViscosityModel=alpha Alpha=1e-3",
+                                "Nx=20 Ny=13 Nu=1e-4", "Nx=31 Ny=12 ViscosityModel=none",
+                                "Nx=32 Ny=16 ViscosityModel=alpha Alpha=1e-3"])
 def test_batched(ov):
     import fargo3d_amd as fa
     print(ov, flush=True)
