@@ -87,14 +87,14 @@ __global__ void __launch_bounds__(64) kb_cfl(const BInst* I, const int* off, int
 // the star's term, each planet's softened term and its indirect term, at the
 // planets' positions at the start of the step (cylindrical 2-D disks).
 // A thread takes kPotCells cells of a row, which share the star's term and the
-// planets' distances; the divisions are rdivd()'s.
+// planets' distances.
 constexpr int kPotCells = 4;
 __device__ __forceinline__ void bp_potential(const BInst& in, const dim3 b) {
   const int i0 = b.x * (kPotCells * BXF) + threadIdx.x, nx = in.m.nx;
   const int j = b.y;
   const BPsys& P = *in.ps;
   const double r = in.ymed64[j], ZC = in.zc;
-  const double star = qdivd(-1.0, sqrt(r * r + ZC * ZC));
+  const double star = Fixed::q64(-1.0, sqrt(r * r + ZC * ZC));
   double pot[kPotCells];
 #pragma unroll
   for (int u = 0; u < kPotCells; u++) pot[u] = star;
@@ -108,7 +108,7 @@ __device__ __forceinline__ void bp_potential(const BInst& in, const dim3 b) {
       const double XC = r * in.cosx64[i], YC = r * in.sinx64[i];
       const double dist = (XC - xp) * (XC - xp) + (YC - yp) * (YC - yp) + (ZC - zp) * (ZC - zp);
       if (P.indirect) pot[u] += rdivd(mp * (XC * xp + YC * yp + ZC * zp), D3);
-      pot[u] += qdivd(-mp, sqrt(dist + s2));
+      pot[u] += Fixed::q64(-mp, sqrt(dist + s2));
     }
   }
 #pragma unroll
@@ -337,7 +337,7 @@ __global__ void __launch_bounds__(64) kb_dt(BInst* I, int n) {
 // the one-pass sources (kd_src_fused2), kBSrcRows rows per lane: 58.5 us for 16
 // disks up to 1536x384, 62.4 with 8 rows, the two passes 68.4
 constexpr int kBSrcRows = 4;
-__global__ void __launch_bounds__(64) kb_src2(const BInst* I, const int* off, int n) {
+__global__ void __launch_bounds__(64, 4) kb_src2(const BInst* I, const int* off, int n) {
   const int ii = find_inst(off, n, blockIdx.x);
   const BInst& in = I[ii];
   const dim3 b = local2(blockIdx.x - off[ii], (in.m.nx + kSrcCols - 1) / kSrcCols);

@@ -77,28 +77,28 @@ __device__ __forceinline__ double lbase(const dmesh& m, int j, int k, double ome
 
 // ---------------------------------------------------------------- SubStep1
 // src/substep1_x.c:112-120
-template <int G, class LR, class LP, class LPOT, class LV>
+template <int G, class D, class LR, class LP, class LPOT, class LV>
 __device__ __forceinline__ real substep1_x(const dmesh& m, int i, int j, int k, real dt, LR rho, LP p,
                                              LPOT pot, LV vx, int dust, int potential) {
   const int im = ixm_of(i, m.nx);
   real dxmed = real(0.5) * (m.sxi[i] + m.sxi[im]);
-  real dtOVERrhom = qdiv(real(2.) * dt, rho(0, 0, 0) * m.sxi[i] + rho(-1, 0, 0) * m.sxi[im]) * dxmed;
+  real dtOVERrhom = D::rho(real(2.) * dt, rho(0, 0, 0) * m.sxi[i] + rho(-1, 0, 0) * m.sxi[im]) * dxmed;
   real v = vx(0, 0, 0);
-  const real izs = inv_zone_size_xmed<G>(m, i, j, k);
+  const real izs = inv_zone_size_xmed<G, D>(m, i, j, k);
   if (!dust) v -= dtOVERrhom * (p(0, 0, 0) - p(-1, 0, 0)) * izs;
   if (potential) v -= (pot(0, 0, 0) - pot(-1, 0, 0)) * dt * izs;
   return v;
 }
 
 // src/substep1_y.c:313-316, 352-355 (CYL), 379-383 (SPH), 408-410
-template <int G, int DZ, class LR, class LP, class LPOT, class LVX, class LVY, class LVZ>
+template <int G, int DZ, class D, class LR, class LP, class LPOT, class LVX, class LVY, class LVZ>
 __device__ __forceinline__ real substep1_y(const dmesh& m, int i, int j, int k, real dt, LR rho, LP p,
                                              LPOT pot, LVX vx, LVY vy, LVZ vz, int dust, int potential,
                                              double omegaframe) {
-  real dtOVERrhom = qdiv(real(2.0) * dt, rho(0, 0, 0) * (m.ymin[j + 1] - m.ymin[j]) + rho(0, -1, 0) * (m.ymin[j] - m.ymin[j - 1])) *
+  real dtOVERrhom = D::rho(real(2.0) * dt, rho(0, 0, 0) * (m.ymin[j + 1] - m.ymin[j]) + rho(0, -1, 0) * (m.ymin[j] - m.ymin[j - 1])) *
                       (m.ymed[j] - m.ymed[j - 1]);
   real v = vy(0, 0, 0);
-  if (!dust) v -= qdiv(dtOVERrhom * (p(0, 0, 0) - p(0, -1, 0)), m.ymed[j] - m.ymed[j - 1]);
+  if (!dust) v -= D::q(dtOVERrhom * (p(0, 0, 0) - p(0, -1, 0)), m.ymed[j] - m.ymed[j - 1]);
   if constexpr (kFix64) {
     double vphi = 0.25 * ((double)vx(0, 0, 0) + (double)vx(1, 0, 0) + (double)vx(0, -1, 0) + (double)vx(1, -1, 0)) +
                   0.5 * (vbase(m, j, k) + vbase(m, j - 1, k));
@@ -108,34 +108,34 @@ __device__ __forceinline__ real substep1_y(const dmesh& m, int i, int j, int k, 
       const double vzz = DZ ? 0.25 * ((double)vz(0, 0, 0) + (double)vz(0, 0, 1) + (double)vz(0, -1, 0) +
                                       (double)vz(0, -1, 1))
                             : 0.0;
-      acc = qdivd(vphi * vphi + vzz * vzz, m.ymin64[j]);
+      acc = D::q64(vphi * vphi + vzz * vzz, m.ymin64[j]);
     } else {
       vphi += m.ymin64[j] * (double)omegaframe;
-      acc = qdivd(vphi * vphi, m.ymin64[j]);
+      acc = D::q64(vphi * vphi, m.ymin64[j]);
     }
-    if (potential) acc -= qdivd((double)pot(0, 0, 0) - (double)pot(0, -1, 0), m.ymed64[j] - m.ymed64[j - 1]);
+    if (potential) acc -= D::q64((double)pot(0, 0, 0) - (double)pot(0, -1, 0), m.ymed64[j] - m.ymed64[j - 1]);
     return v + (real)(acc * (double)dt);
   } else {
     real vphi = real(.25) * (vx(0, 0, 0) + vx(1, 0, 0) + vx(0, -1, 0) + vx(1, -1, 0));
     if (G == SPH) {
       vphi += m.ymin[j] * m.sinzmed[k] * omegaframe;
       real vzz = DZ ? real(.25) * (vz(0, 0, 0) + vz(0, 0, 1) + vz(0, -1, 0) + vz(0, -1, 1)) : real(0.0);
-      v += qdiv(vphi * vphi + vzz * vzz, m.ymin[j]) * dt;
+      v += D::q(vphi * vphi + vzz * vzz, m.ymin[j]) * dt;
     } else {
       vphi += m.ymin[j] * omegaframe;
-      v += qdiv(vphi * vphi, m.ymin[j]) * dt;
+      v += D::q(vphi * vphi, m.ymin[j]) * dt;
     }
-    if (potential) v -= qdiv((pot(0, 0, 0) - pot(0, -1, 0)) * dt, m.ymed[j] - m.ymed[j - 1]);
+    if (potential) v -= D::q((pot(0, 0, 0) - pot(0, -1, 0)) * dt, m.ymed[j] - m.ymed[j - 1]);
     return v;
   }
 }
 
 // src/substep1_z.c:120-183 (CYLINDRICAL and SPHERICAL branches)
-template <int G, class LR, class LP, class LPOT, class LVX, class LVZ>
+template <int G, class D, class LR, class LP, class LPOT, class LVX, class LVZ>
 __device__ __forceinline__ real substep1_z(const dmesh& m, int i, int j, int k, real dt, LR rho, LP p,
                                              LPOT pot, LVX vx, LVZ vz, int dust, int potential,
                                              double omegaframe) {
-  real dtOVERrhom = qdiv(real(2.0) * dt, rho(0, 0, 0) * (m.zmin[k + 1] - m.zmin[k]) + rho(0, 0, -1) * (m.zmin[k] - m.zmin[k - 1])) *
+  real dtOVERrhom = D::rho(real(2.0) * dt, rho(0, 0, 0) * (m.zmin[k + 1] - m.zmin[k]) + rho(0, 0, -1) * (m.zmin[k] - m.zmin[k - 1])) *
                       (m.zmed[k] - m.zmed[k - 1]);
   real v;
   if (G == SPH && kFix64) {
@@ -144,21 +144,21 @@ __device__ __forceinline__ real substep1_z(const dmesh& m, int i, int j, int k, 
     const double smin = m.sinzmin64[k], r = m.ymed64[j];
     vphi += r * smin * (double)omegaframe;
     v = vz(0, 0, 0);
-    if (!dust) v -= qdiv(dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)), m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
-    double acc = qdivd(vphi * vphi * m.coszmin64[k], smin * r);
-    if (potential) acc -= qdivd((double)pot(0, 0, 0) - (double)pot(0, 0, -1), r * (m.zmed64[k] - m.zmed64[k - 1]));
+    if (!dust) v -= D::q(dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)), m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
+    double acc = D::q64(vphi * vphi * m.coszmin64[k], smin * r);
+    if (potential) acc -= D::q64((double)pot(0, 0, 0) - (double)pot(0, 0, -1), r * (m.zmed64[k] - m.zmed64[k - 1]));
     v += (real)(acc * (double)dt);
   } else if (G == SPH) {
     real vphi = real(.25) * (vx(0, 0, 0) + vx(1, 0, 0) + vx(0, 0, -1) + vx(1, 0, -1));
     vphi += m.ymed[j] * m.sinzmin[k] * omegaframe;
     v = vz(0, 0, 0);
-    if (!dust) v -= qdiv(dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)), m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
-    v += qdiv(vphi * vphi * m.coszmin[k], m.sinzmin[k] * m.ymed[j]) * dt;
-    if (potential) v -= qdiv((pot(0, 0, 0) - pot(0, 0, -1)) * dt, m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
+    if (!dust) v -= D::q(dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)), m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
+    v += D::q(vphi * vphi * m.coszmin[k], m.sinzmin[k] * m.ymed[j]) * dt;
+    if (potential) v -= D::q((pot(0, 0, 0) - pot(0, 0, -1)) * dt, m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
   } else {
     v = vz(0, 0, 0);
-    if (!dust) v -= qdiv(dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)), m.zmed[k] - m.zmed[k - 1]);
-    if (potential) v -= qdiv((pot(0, 0, 0) - pot(0, 0, -1)) * dt, m.zmed[k] - m.zmed[k - 1]);
+    if (!dust) v -= D::q(dtOVERrhom * (p(0, 0, 0) - p(0, 0, -1)), m.zmed[k] - m.zmed[k - 1]);
+    if (potential) v -= D::q((pot(0, 0, 0) - pot(0, 0, -1)) * dt, m.zmed[k] - m.zmed[k - 1]);
   }
   return v;
 }
@@ -171,7 +171,7 @@ __device__ __forceinline__ real art_q(real rho, real dv) {
 }
 
 // src/substep2_b.c:145-190; inputs are the current v_temp (and e) values
-template <int G, int DZ, class LR, class LVX, class LVY, class LVZ, class LQX, class LQY, class LQZ>
+template <int G, int DZ, class D, class LR, class LVX, class LVY, class LVZ, class LQX, class LQY, class LQZ>
 __device__ __forceinline__ void substep2_b(const dmesh& m, int i, int j, int k, real dt, LR rho, LVX vx, LVY vy,
                                            LVZ vz, LQX px, LQY py, LQZ pz, int adiabatic, real vxt, real vyt,
                                            real vzt, real e, real& oxt, real& oyt, real& ozt,
@@ -180,23 +180,23 @@ __device__ __forceinline__ void substep2_b(const dmesh& m, int i, int j, int k, 
   real dxrho1 = m.sxi[i];
   real dxrho2 = m.sxi[im];
   real dxmed = real(0.5) * (m.sxi[i] + m.sxi[im]);
-  vxt += qdiv(-real(2.0) * dt * dxmed * (px(0, 0, 0) - px(-1, 0, 0)), rho(0, 0, 0) * dxrho1 + rho(-1, 0, 0) * dxrho2) *
-         inv_zone_size_xmed<G>(m, i, j, k);
-  if (adiabatic) e += -dt * qdiv(px(0, 0, 0) * (vx(1, 0, 0) - vx(0, 0, 0)), zone_size_x<G>(m, i, j, k));
+  vxt += D::rho(-real(2.0) * dt * dxmed * (px(0, 0, 0) - px(-1, 0, 0)), rho(0, 0, 0) * dxrho1 + rho(-1, 0, 0) * dxrho2) *
+         inv_zone_size_xmed<G, D>(m, i, j, k);
+  if (adiabatic) e += -dt * D::q(px(0, 0, 0) * (vx(1, 0, 0) - vx(0, 0, 0)), zone_size_x<G>(m, i, j, k));
   real dyrho1 = m.ymin[j + 1] - m.ymin[j];
   real dyrho2 = m.ymin[j] - m.ymin[j - 1];
-  vyt += qdiv(-real(2.0) * (py(0, 0, 0) - py(0, -1, 0)), rho(0, 0, 0) * dyrho1 + rho(0, -1, 0) * dyrho2) * dt;
-  if (adiabatic) e += -dt * qdiv(py(0, 0, 0) * (vy(0, 1, 0) - vy(0, 0, 0)), zone_size_y(m, j));
+  vyt += D::rho(-real(2.0) * (py(0, 0, 0) - py(0, -1, 0)), rho(0, 0, 0) * dyrho1 + rho(0, -1, 0) * dyrho2) * dt;
+  if (adiabatic) e += -dt * D::q(py(0, 0, 0) * (vy(0, 1, 0) - vy(0, 0, 0)), zone_size_y(m, j));
   if (DZ) {
     real dzmed = m.zmed[k] - m.zmed[k - 1];
     real dzrho1 = m.zmin[k + 1] - m.zmin[k];
     real dzrho2 = m.zmin[k] - m.zmin[k - 1];
     if (G == SPH)
-      vzt += qdiv(qdiv(-real(2.0) * dzmed * (pz(0, 0, 0) - pz(0, 0, -1)), rho(0, 0, 0) * dzrho1 + rho(0, 0, -1) * dzrho2) * dt,
+      vzt += D::q(D::rho(-real(2.0) * dzmed * (pz(0, 0, 0) - pz(0, 0, -1)), rho(0, 0, 0) * dzrho1 + rho(0, 0, -1) * dzrho2) * dt,
                   m.ymed[j] * (m.zmed[k] - m.zmed[k - 1]));
     else
-      vzt += qdiv(-real(2.0) * (pz(0, 0, 0) - pz(0, 0, -1)), rho(0, 0, 0) * dzrho1 + rho(0, 0, -1) * dzrho2) * dt;
-    if (adiabatic) e += -dt * qdiv(pz(0, 0, 0) * (vz(0, 0, 1) - vz(0, 0, 0)), zone_size_z<G>(m, j, k));
+      vzt += D::rho(-real(2.0) * (pz(0, 0, 0) - pz(0, 0, -1)), rho(0, 0, 0) * dzrho1 + rho(0, 0, -1) * dzrho2) * dt;
+    if (adiabatic) e += -dt * D::q(pz(0, 0, 0) * (vz(0, 0, 1) - vz(0, 0, 0)), zone_size_z<G>(m, j, k));
   }
   oxt = vxt;
   oyt = vyt;
@@ -215,20 +215,20 @@ __device__ __forceinline__ real div_v(const dmesh& m, int i, int j, int k, LVX v
 }
 
 // src/substep3.c:106-110
-template <int DZ, class LVX, class LVY, class LVZ>
+template <int DZ, class D, class LVX, class LVY, class LVZ>
 __device__ __forceinline__ real substep3(const dmesh& m, int i, int j, int k, real dt, real e, LVX vx,
                                            LVY vy, LVZ vz, real gamma) {
   real dv = div_v<DZ>(m, i, j, k, vx, vy, vz);
-  real term = mul_invvol(m, real(0.5) * dt * (gamma - real(1.)) * dv, i, j, k);
+  real term = mul_invvol<D>(m, real(0.5) * dt * (gamma - real(1.)) * dv, i, j, k);
   if constexpr (kFix64) {
     // e (1 - t)/(1 + t) = e - e 2t/(1 + t): the change of e formed directly.
     // In FP32 the rounding of 1 - t is the same for every cell of a ring
     // with the same t and would heat or cool the ring by a fixed amount
     // each step; here it is relative to the change only.
-    e -= e * qdiv(real(2.0) * term, real(1.0) + term);
+    e -= e * D::q(real(2.0) * term, real(1.0) + term);
     return e;
   }
-  e *= qdiv(real(1.0) - term, real(1.0) + term);
+  e *= D::q(real(1.0) - term, real(1.0) + term);
   return e;
 }
 
@@ -244,7 +244,7 @@ struct Taus {
 };
 
 // src/visctensor_cyl.c:140-198 and src/visctensor_sph.c:126-206
-template <int G, int DZ, class LR, class LE, class LVX, class LVY, class LVZ>
+template <int G, int DZ, class D, class LR, class LE, class LVX, class LVY, class LVZ>
 __device__ __forceinline__ Taus visctensor(const dmesh& m, int i, int j, int k, LR rho, LE energy, LVX vx, LVY vy,
                                            LVZ vz, const ViscPar& vp) {
   real visc, viscm, visczm = real(0.0), visczmym = real(0.0);
@@ -264,13 +264,13 @@ __device__ __forceinline__ Taus visctensor(const dmesh& m, int i, int j, int k, 
       }
     } else {
       const real gg = vp.alpha * vp.gamma * (vp.gamma - real(1.0));
-      visc = qdiv(gg * energy(0, 0, 0), rho(0, 0, 0)) * sq_med;
-      viscm = qdiv(gg * (energy(0, 0, 0) + energy(-1, 0, 0) + energy(0, -1, 0) + energy(-1, -1, 0)),
+      visc = D::rho(gg * energy(0, 0, 0), rho(0, 0, 0)) * sq_med;
+      viscm = D::rho(gg * (energy(0, 0, 0) + energy(-1, 0, 0) + energy(0, -1, 0) + energy(-1, -1, 0)),
                    rho(0, 0, 0) + rho(-1, 0, 0) + rho(0, -1, 0) + rho(-1, -1, 0)) * sq_min;
       if (DZ) {
-        visczm = qdiv(gg * (energy(0, 0, 0) + energy(0, 0, -1) + energy(-1, 0, 0) + energy(-1, 0, -1)),
+        visczm = D::rho(gg * (energy(0, 0, 0) + energy(0, 0, -1) + energy(-1, 0, 0) + energy(-1, 0, -1)),
                       rho(0, 0, 0) + rho(0, 0, -1) + rho(-1, 0, 0) + rho(-1, 0, -1)) * sq_med;
-        visczmym = qdiv(gg * (energy(0, 0, 0) + energy(0, -1, 0) + energy(0, 0, -1) + energy(0, -1, -1)),
+        visczmym = D::rho(gg * (energy(0, 0, 0) + energy(0, -1, 0) + energy(0, 0, -1) + energy(0, -1, -1)),
                         rho(0, 0, 0) + rho(0, -1, 0) + rho(0, 0, -1) + rho(0, -1, -1)) * sq_min;
       }
     }
@@ -278,92 +278,92 @@ __device__ __forceinline__ Taus visctensor(const dmesh& m, int i, int j, int k, 
     visc = viscm = visczm = visczmym = vp.nu;
   }
   real dv = div_v<DZ>(m, i, j, k, vx, vy, vz);
-  dv *= mul_invvol(m, real(2.0) / real(3.0), i, j, k);
+  dv *= D::mesh(real(2.0) / real(3.0) * m.invvj[j], m.syk[k] * m.sxi[i]);
   const real r0 = rho(0, 0, 0);
   Taus t;
-  t.xx = visc * r0 * (qdiv(real(2.0) * (vx(1, 0, 0) - vx(0, 0, 0)), zone_size_x<G>(m, i, j, k)) - dv);
-  t.xx += qdiv(visc * r0 * (vy(0, 1, 0) + vy(0, 0, 0)), m.ymed[j]);
-  if (G == SPH && DZ) t.xx += qdiv(visc * r0 * (vz(0, 0, 1) + vz(0, 0, 0)) * m.coszmed[k], m.sinzmed[k] * m.ymed[j]);
-  t.yy = visc * r0 * (qdiv(real(2.0) * (vy(0, 1, 0) - vy(0, 0, 0)), m.ymin[j + 1] - m.ymin[j]) - dv);
+  t.xx = visc * r0 * (D::q(real(2.0) * (vx(1, 0, 0) - vx(0, 0, 0)), zone_size_x<G>(m, i, j, k)) - dv);
+  t.xx += D::q(visc * r0 * (vy(0, 1, 0) + vy(0, 0, 0)), m.ymed[j]);
+  if (G == SPH && DZ) t.xx += D::q(visc * r0 * (vz(0, 0, 1) + vz(0, 0, 0)) * m.coszmed[k], m.sinzmed[k] * m.ymed[j]);
+  t.yy = visc * r0 * (D::q(real(2.0) * (vy(0, 1, 0) - vy(0, 0, 0)), m.ymin[j + 1] - m.ymin[j]) - dv);
   t.zz = t.xz = t.zy = real(0.0);
   if (DZ) {
     if (G == SPH) {
-      t.zz = visc * r0 * (qdiv(real(2.0) * (vz(0, 0, 1) - vz(0, 0, 0)), m.ymed[j] * (m.zmin[k + 1] - m.zmin[k])) - dv);
-      t.zz += qdiv(visc * r0 * (vy(0, 0, 0) + vy(0, 1, 0)), m.ymed[j]);
+      t.zz = visc * r0 * (D::q(real(2.0) * (vz(0, 0, 1) - vz(0, 0, 0)), m.ymed[j] * (m.zmin[k + 1] - m.zmin[k])) - dv);
+      t.zz += D::q(visc * r0 * (vy(0, 0, 0) + vy(0, 1, 0)), m.ymed[j]);
       t.xz = visczm * real(.25) * (r0 + rho(0, 0, -1) + rho(-1, 0, 0) + rho(-1, 0, -1)) *
-             (qdiv((qdiv(vx(0, 0, 0), m.sinzmed[k]) - qdiv(vx(0, 0, -1), m.sinzmed[k - 1])) * m.sinzmin[k],
+             (D::q((D::q(vx(0, 0, 0), m.sinzmed[k]) - D::q(vx(0, 0, -1), m.sinzmed[k - 1])) * m.sinzmin[k],
                    m.ymed[j] * (m.zmed[k] - m.zmed[k - 1])) +
-              qdiv((vz(0, 0, 0) - vz(-1, 0, 0)) * m.invdiffxmed[i], m.sinzmin[k] * m.ymed[j]));
+              D::q((vz(0, 0, 0) - vz(-1, 0, 0)) * m.invdiffxmed[i], m.sinzmin[k] * m.ymed[j]));
     } else {
-      t.zz = visc * r0 * (qdiv(real(2.0) * (vz(0, 0, 1) - vz(0, 0, 0)), m.zmin[k + 1] - m.zmin[k]) - dv);
+      t.zz = visc * r0 * (D::q(real(2.0) * (vz(0, 0, 1) - vz(0, 0, 0)), m.zmin[k + 1] - m.zmin[k]) - dv);
       t.xz = visczm * real(.25) * (r0 + rho(0, 0, -1) + rho(-1, 0, 0) + rho(-1, 0, -1)) *
-             (qdiv(vx(0, 0, 0) - vx(0, 0, -1), m.zmed[k] - m.zmed[k - 1]) +
-              qdiv((vz(0, 0, 0) - vz(-1, 0, 0)) * m.invdiffxmed[i], m.ymed[j]));
+             (D::q(vx(0, 0, 0) - vx(0, 0, -1), m.zmed[k] - m.zmed[k - 1]) +
+              D::q((vz(0, 0, 0) - vz(-1, 0, 0)) * m.invdiffxmed[i], m.ymed[j]));
     }
   }
   if (G == SPH)
     t.yx = viscm * real(.25) * (r0 + rho(-1, 0, 0) + rho(0, -1, 0) + rho(-1, -1, 0)) *
-           (qdiv((vy(0, 0, 0) - vy(-1, 0, 0)) * m.invdiffxmed[i], m.ymin[j] * m.sinzmed[k]) +
-            qdiv(vx(0, 0, 0) - vx(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) - qdiv(real(.5) * (vx(0, 0, 0) + vx(0, -1, 0)), m.ymin[j]));
+           (D::q((vy(0, 0, 0) - vy(-1, 0, 0)) * m.invdiffxmed[i], m.ymin[j] * m.sinzmed[k]) +
+            D::q(vx(0, 0, 0) - vx(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) - D::q(real(.5) * (vx(0, 0, 0) + vx(0, -1, 0)), m.ymin[j]));
   else
     t.yx = viscm * real(.25) * (r0 + rho(-1, 0, 0) + rho(0, -1, 0) + rho(-1, -1, 0)) *
-           (qdiv((vy(0, 0, 0) - vy(-1, 0, 0)) * m.invdiffxmed[i], m.ymin[j]) +
-            qdiv(vx(0, 0, 0) - vx(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) - qdiv(real(.5) * (vx(0, 0, 0) + vx(0, -1, 0)), m.ymin[j]));
+           (D::q((vy(0, 0, 0) - vy(-1, 0, 0)) * m.invdiffxmed[i], m.ymin[j]) +
+            D::q(vx(0, 0, 0) - vx(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) - D::q(real(.5) * (vx(0, 0, 0) + vx(0, -1, 0)), m.ymin[j]));
   if (DZ) {
     if (G == SPH)
       t.zy = visczmym * real(.25) * (r0 + rho(0, -1, 0) + rho(0, 0, -1) + rho(0, -1, -1)) *
-             (qdiv(vz(0, 0, 0) - vz(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) - qdiv(real(.5) * (vz(0, 0, 0) + vz(0, -1, 0)), m.ymin[j]) +
-              qdiv(vy(0, 0, 0) - vy(0, 0, -1), m.ymin[j] * (m.zmed[k] - m.zmed[k - 1])));
+             (D::q(vz(0, 0, 0) - vz(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) - D::q(real(.5) * (vz(0, 0, 0) + vz(0, -1, 0)), m.ymin[j]) +
+              D::q(vy(0, 0, 0) - vy(0, 0, -1), m.ymin[j] * (m.zmed[k] - m.zmed[k - 1])));
     else
       t.zy = visczmym * real(.25) * (r0 + rho(0, -1, 0) + rho(0, 0, -1) + rho(0, -1, -1)) *
-             (qdiv(vz(0, 0, 0) - vz(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) +
-              qdiv(vy(0, 0, 0) - vy(0, 0, -1), m.zmed[k] - m.zmed[k - 1]));
+             (D::q(vz(0, 0, 0) - vz(0, -1, 0), m.ymed[j] - m.ymed[j - 1]) +
+              D::q(vy(0, 0, 0) - vy(0, 0, -1), m.zmed[k] - m.zmed[k - 1]));
   }
   return t;
 }
 
 // src/addviscosity_cyl.c:97-131 and src/addviscosity_sph.c:97-143
-template <int G, int DZ, class LR, class LXX, class LYY, class LZZ, class LXZ, class LYX, class LZY>
+template <int G, int DZ, class D, class LR, class LXX, class LYY, class LZZ, class LXZ, class LYX, class LZY>
 __device__ __forceinline__ void addviscosity(const dmesh& m, int i, int j, int k, real dt, LR rho, LXX txx,
                                              LYY tyy, LZZ tzz, LXZ txz, LYX tyx, LZY tzy, real vx, real vy,
                                              real vz, real& ox, real& oy, real& oz) {
   const real r0 = rho(0, 0, 0), rxm = rho(-1, 0, 0), rym = rho(0, -1, 0);
   const real ymn = m.ymin[j], ymp = m.ymin[j + 1], yd = m.ymed[j], ydm = m.ymed[j - 1];
-  vx += qdiv(real(2.0) * (txx(0, 0, 0) - txx(-1, 0, 0)) * inv_zone_size_xmed<G>(m, i, j, k), r0 + rxm) * dt;
-  vx += qdiv(real(2.0) * (ymp * ymp * tyx(0, 1, 0) - ymn * ymn * tyx(0, 0, 0)), (ymp - ymn) * yd * yd * (rxm + r0)) * dt;
+  vx += D::rho(real(2.0) * (txx(0, 0, 0) - txx(-1, 0, 0)) * inv_zone_size_xmed<G, D>(m, i, j, k), r0 + rxm) * dt;
+  vx += D::rho(real(2.0) * (ymp * ymp * tyx(0, 1, 0) - ymn * ymn * tyx(0, 0, 0)), (ymp - ymn) * yd * yd * (rxm + r0)) * dt;
   if (G == SPH) {
-    vx += qdiv(tyx(0, 1, 0) + tyx(0, 0, 0), (rxm + r0) * yd) * dt;
+    vx += D::rho(tyx(0, 1, 0) + tyx(0, 0, 0), (rxm + r0) * yd) * dt;
     if (DZ) {
-      vx += qdiv(real(2.0) * (txz(0, 0, 1) - txz(0, 0, 0)), zone_size_z<G>(m, j, k) * (rxm + r0)) * dt;
-      vx += qdiv(real(2.0) * (txz(0, 0, 1) + txz(0, 0, 0)) * m.coszmed[k], m.sinzmed[k] * yd * (rxm + r0)) * dt;
+      vx += D::rho(real(2.0) * (txz(0, 0, 1) - txz(0, 0, 0)), zone_size_z<G>(m, j, k) * (rxm + r0)) * dt;
+      vx += D::rho(real(2.0) * (txz(0, 0, 1) + txz(0, 0, 0)) * m.coszmed[k], m.sinzmed[k] * yd * (rxm + r0)) * dt;
     }
-    vy += qdiv(real(2.0) * (yd * yd * tyy(0, 0, 0) - ydm * ydm * tyy(0, -1, 0)), (yd - ydm) * (r0 + rym) * ymn * ymn) * dt;
-    vy += qdiv(real(2.0) * (tyx(1, 0, 0) - tyx(0, 0, 0)),
+    vy += D::rho(real(2.0) * (yd * yd * tyy(0, 0, 0) - ydm * ydm * tyy(0, -1, 0)), (yd - ydm) * (r0 + rym) * ymn * ymn) * dt;
+    vy += D::rho(real(2.0) * (tyx(1, 0, 0) - tyx(0, 0, 0)),
                (m.xmin[i + 1] - m.xmin[i]) * ymn * m.sinzmed[k] * (r0 + rym)) * dt;
-    vy -= qdiv(txx(0, 0, 0) + txx(0, -1, 0), ymn * (r0 + rym)) * dt;
+    vy -= D::rho(txx(0, 0, 0) + txx(0, -1, 0), ymn * (r0 + rym)) * dt;
     if (DZ) {
       const real rzm = rho(0, 0, -1);
-      vy -= qdiv(tzz(0, 0, 0) + tzz(0, -1, 0), ymn * (r0 + rym)) * dt;
-      vy += qdiv(real(2.0) * (tzy(0, 0, 1) * m.sinzmin[k + 1] - tzy(0, 0, 0) * m.sinzmin[k]),
+      vy -= D::rho(tzz(0, 0, 0) + tzz(0, -1, 0), ymn * (r0 + rym)) * dt;
+      vy += D::rho(real(2.0) * (tzy(0, 0, 1) * m.sinzmin[k + 1] - tzy(0, 0, 0) * m.sinzmin[k]),
                  (m.zmin[k + 1] - m.zmin[k]) * ymn * m.sinzmed[k] * (r0 + rym)) * dt;
-      vz += qdiv(real(2.0) * (tzz(0, 0, 0) * m.sinzmed[k] - tzz(0, 0, -1) * m.sinzmed[k - 1]),
+      vz += D::rho(real(2.0) * (tzz(0, 0, 0) * m.sinzmed[k] - tzz(0, 0, -1) * m.sinzmed[k - 1]),
                  (m.zmed[k] - m.zmed[k - 1]) * yd * m.sinzmin[k] * (r0 + rzm)) * dt;
-      vz += qdiv(real(2.0) * (txz(1, 0, 0) - txz(0, 0, 0)), (m.sxi[i] * yd * m.sinzmin[k]) * (r0 + rzm)) * dt;
-      vz += qdiv(real(2.0) * (ymp * ymp * ymp * tzy(0, 1, 0) - ymn * ymn * ymn * tzy(0, 0, 0)),
+      vz += D::rho(real(2.0) * (txz(1, 0, 0) - txz(0, 0, 0)), (m.sxi[i] * yd * m.sinzmin[k]) * (r0 + rzm)) * dt;
+      vz += D::rho(real(2.0) * (ymp * ymp * ymp * tzy(0, 1, 0) - ymn * ymn * ymn * tzy(0, 0, 0)),
                  (ymp - ymn) * yd * yd * yd * (r0 + rzm)) * dt;
-      vz -= qdiv((txx(0, 0, 0) + txx(0, 0, -1)) * m.coszmin[k], yd * m.sinzmin[k] * (r0 + rzm)) * dt;
+      vz -= D::rho((txx(0, 0, 0) + txx(0, 0, -1)) * m.coszmin[k], yd * m.sinzmin[k] * (r0 + rzm)) * dt;
     }
   } else {
-    if (DZ) vx += qdiv(real(2.0) * (txz(0, 0, 1) - txz(0, 0, 0)), (m.zmin[k + 1] - m.zmin[k]) * (rxm + r0)) * dt;
-    vy += qdiv(real(2.0) * (yd * tyy(0, 0, 0) - ydm * tyy(0, -1, 0)), (yd - ydm) * (r0 + rym) * ymn) * dt;
-    vy += qdiv(real(2.0) * (tyx(1, 0, 0) - tyx(0, 0, 0)), (m.xmin[i + 1] - m.xmin[i]) * ymn * (r0 + rym)) * dt;
-    vy -= qdiv(txx(0, 0, 0) + txx(0, -1, 0), ymn * (r0 + rym)) * dt;
+    if (DZ) vx += D::rho(real(2.0) * (txz(0, 0, 1) - txz(0, 0, 0)), (m.zmin[k + 1] - m.zmin[k]) * (rxm + r0)) * dt;
+    vy += D::rho(real(2.0) * (yd * tyy(0, 0, 0) - ydm * tyy(0, -1, 0)), (yd - ydm) * (r0 + rym) * ymn) * dt;
+    vy += D::rho(real(2.0) * (tyx(1, 0, 0) - tyx(0, 0, 0)), (m.xmin[i + 1] - m.xmin[i]) * ymn * (r0 + rym)) * dt;
+    vy -= D::rho(txx(0, 0, 0) + txx(0, -1, 0), ymn * (r0 + rym)) * dt;
     if (DZ) {
       const real rzm = rho(0, 0, -1);
-      vy += qdiv(real(2.0) * (tzy(0, 0, 1) - tzy(0, 0, 0)), (m.zmin[k + 1] - m.zmin[k]) * (r0 + rym)) * dt;
-      vz += qdiv(real(2.0) * (tzz(0, 0, 0) - tzz(0, 0, -1)), (m.zmed[k] - m.zmed[k - 1]) * (r0 + rzm)) * dt;
-      vz += qdiv(real(2.0) * (txz(1, 0, 0) - txz(0, 0, 0)), zone_size_x<G>(m, i, j, k) * (r0 + rzm)) * dt;
-      vz += qdiv(real(2.0) * (ymp * tzy(0, 1, 0) - ymn * tzy(0, 0, 0)), (ymp - ymn) * yd * (r0 + rzm)) * dt;
+      vy += D::rho(real(2.0) * (tzy(0, 0, 1) - tzy(0, 0, 0)), (m.zmin[k + 1] - m.zmin[k]) * (r0 + rym)) * dt;
+      vz += D::rho(real(2.0) * (tzz(0, 0, 0) - tzz(0, 0, -1)), (m.zmed[k] - m.zmed[k - 1]) * (r0 + rzm)) * dt;
+      vz += D::rho(real(2.0) * (txz(1, 0, 0) - txz(0, 0, 0)), zone_size_x<G>(m, i, j, k) * (r0 + rzm)) * dt;
+      vz += D::rho(real(2.0) * (ymp * tzy(0, 1, 0) - ymn * tzy(0, 0, 0)), (ymp - ymn) * yd * (r0 + rzm)) * dt;
     }
   }
   ox = vx;
@@ -461,29 +461,26 @@ __device__ __forceinline__ real momentum_x(const dmesh& m, int j, int k, real rh
   return (v + rcyl * omegaframe) * rcyl * rho;
 }
 
-// src/newvel_x.c:78-86
-template <int G>
-__device__ __forceinline__ real newvel_x(const dmesh& m, int i, int j, int k, real rho, real rhoxm, real mmx,
-                                           real mpxm, real omegaframe) {
-  const int im = ixm_of(i, m.nx);
+// src/newvel_x.c:78-86, from the masses rho Vol of the cell and of its left
+// neighbour, the cell's Mmx Vol and the neighbour's Mpx Vol
+template <int G, class D>
+__device__ __forceinline__ real newvel_x(const dmesh& m, int j, int k, real mass, real massxm, real mmx, real mpxm,
+                                         real omegaframe) {
   if constexpr (kFix64) {
     // from the momenta's deviations: l0/r - Omega_f r = V0 drops out, and the
     // result is the deviation vx'
     const double r = rcyl64<G>(m, j, k);
-    return (real)qdivd((double)mul_vol(m, mmx, i, j, k) + (double)mul_vol(m, mpxm, im, j, k),
-                       ((double)mul_vol(m, rho, i, j, k) + (double)mul_vol(m, rhoxm, im, j, k)) * r);
+    return (real)D::q64((double)mmx + (double)mpxm, ((double)mass + (double)massxm) * r);
   }
   real r = (G == SPH) ? m.ymed[j] * m.sinzmed[k] : m.ymed[j];
-  return qdiv(mul_vol(m, mmx, i, j, k) + mul_vol(m, mpxm, im, j, k),
-              (mul_vol(m, rho, i, j, k) + mul_vol(m, rhoxm, im, j, k)) * r) -
-         omegaframe * r;
+  return D::rho(mmx + mpxm, (mass + massxm) * r) - omegaframe * r;
 }
 
-// src/newvel_y.c:67
-__device__ __forceinline__ real newvel_y(const dmesh& m, int i, int j, int k, real rho, real rhoym, real mmy,
-                                           real mpym) {
-  return qdiv(mul_vol(m, mmy, i, j, k) + mul_vol(m, mpym, i, j - 1, k),
-              mul_vol(m, rho, i, j, k) + mul_vol(m, rhoym, i, j - 1, k));
+// src/newvel_y.c:67, and the quotient of NewVelocity_z, from the same products
+// of the cell and of the one below it
+template <class D>
+__device__ __forceinline__ real newvel_yz(real mass, real massm, real mm, real mpm) {
+  return D::rho(mm + mpm, mass + massm);
 }
 
 // ---------------------------------------------------------------- PPA (src/fargo_ppa_*.c)
@@ -535,14 +532,14 @@ __device__ __forceinline__ real ppa_swept_down(real k, real q, real qL, real qR)
 // parabolic average over the swept zone (src/fargo_ppa_d.c:62-70)
 __device__ __forceinline__ real ppa_flux_value(real v, real dt, real zsx, real qm, real qLm, real qRm,
                                                  real q, real qL, real qR) {
-  const real k = qdiv(fabs(v * dt), zsx);  // v dt / zsx where v > 0, else -v dt / zsx
+  const real k = Full::q(v > real(0.0) ? v * dt : -v * dt, zsx);
   return (v > real(0.0)) ? ppa_swept_up(k, qm, qLm, qRm) : ppa_swept_down(k, q, qL, qR);
 }
 
 // ---------------------------------------------------------------- conservative updates
 // src/update_x.c:69-71: ((a - b)*SurfX*dt*InvVol)
 __device__ __forceinline__ real flux_x(const dmesh& m, int i, int j, int k, real dt, real a, real b) {
-  return mul_invvol(m, mul_surfx(m, a - b, j, k) * dt, i, j, k);
+  return mul_invvol<Full>(m, mul_surfx(m, a - b, j, k) * dt, i, j, k);
 }
 // the same from the difference d of the face flows, with the cell's InvVol
 // divisor shared by its quantities
@@ -551,10 +548,10 @@ __device__ __forceinline__ real flux_x(const dmesh& m, int j, int k, real dt, re
 }
 // src/update_y.c:68-70: (a*SurfY(j) - b*SurfY(j+1))*dt*InvVol
 __device__ __forceinline__ real flux_y(const dmesh& m, int i, int j, int k, real dt, real a, real b) {
-  return mul_invvol(m, (mul_surfy(m, a, i, j, k) - mul_surfy(m, b, i, j + 1, k)) * dt, i, j, k);
+  return mul_invvol<Full>(m, (mul_surfy(m, a, i, j, k) - mul_surfy(m, b, i, j + 1, k)) * dt, i, j, k);
 }
 __device__ __forceinline__ real flux_z(const dmesh& m, int i, int j, int k, real dt, real a, real b) {
-  return mul_invvol(m, (mul_surfz(m, a, i, j, k) - mul_surfz(m, b, i, j, k + 1)) * dt, i, j, k);
+  return mul_invvol<Full>(m, (mul_surfz(m, a, i, j, k) - mul_surfz(m, b, i, j, k + 1)) * dt, i, j, k);
 }
 
 // ---------------------------------------------------------------- cfl (src/cfl.c:174-253)
@@ -596,12 +593,12 @@ __device__ __forceinline__ double cfl_sumsq(const dmesh& m, int i, int j, int k,
   }
   const double c0 = cs[l];
   double soundspeed2 = 0.0, viscosity;
-  if (!cp.iso) soundspeed2 = qdivd(cp.gamma * (cp.gamma - 1) * c0, (double)rho[l]);
+  if (!cp.iso) soundspeed2 = cp.gamma * (cp.gamma - 1) * c0 / (double)rho[l];
   if (cp.alpha_visc) {
     const double y = m.ymed64[j];
     const double sq = sqrt(y * y * y / (1.0 * 1.0));
     if (cp.iso) viscosity = cp.alpha * c0 * c0 * sq;
-    else viscosity = qdivd(cp.alpha * cp.gamma * (cp.gamma - 1.0) * c0, (double)rho[l]) * sq;
+    else viscosity = cp.alpha * cp.gamma * (cp.gamma - 1.0) * c0 / (double)rho[l] * sq;
   } else {
     viscosity = cp.nu;
   }
@@ -683,25 +680,26 @@ __device__ __forceinline__ Ramps stockholm_ramps(const dmesh& m, int j, int k, c
   return Ramps{rampy + rampz, rampy + rampzz, d.ds * sqrt(ym * ym * ym / real(1.0) / real(1.0))};
 }
 // rho, vx, vy of a cell where R.ramp > 0
-template <int G>
+template <int G, class D>
 __device__ __forceinline__ void stockholm_rxy(const dmesh& m, int j, int k, real dt, const Ramps& R, real& rho,
                                               real& vx, real& vy, real rho0, real vx0, real vy0, const DampPar& d) {
   real taud = R.tau / R.ramp;
-  rho = qdiv(rho * taud + rho0 * dt, dt + taud);
+  rho = D::q(rho * taud + rho0 * dt, dt + taud);
   real vx0_target = vx0;
   real radius = m.ymed[j];
   if (G == SPH) radius *= m.sinzmed[k];
   vx0_target -= (real)((d.of - d.of0) * radius);
-  vx = qdiv(vx * taud + vx0_target * dt, dt + taud);
-  vy = qdiv(vy * taud + vy0 * dt, dt + taud);
+  vx = D::q(vx * taud + vx0_target * dt, dt + taud);
+  vy = D::q(vy * taud + vy0 * dt, dt + taud);
 }
 // vz of a cell where R.rampi > 0
+template <class D>
 __device__ __forceinline__ real stockholm_z(real dt, const Ramps& R, real vz, real vz0) {
   real taud = R.tau / R.rampi;
-  return qdiv(vz * taud + vz0 * dt, dt + taud);
+  return D::q(vz * taud + vz0 * dt, dt + taud);
 }
 // the same on the arrays (cell l of ring (j,k))
-template <int G, int DZ>
+template <int G, int DZ, class D>
 __device__ __forceinline__ void stockholm(const dmesh& m, int j, int k, int l, real dt, real* rho, real* vx,
                                           real* vy, real* vz, const real* rho0, const real* vx0,
                                           const real* vy0, const real* vz0, const DampPar& d) {
@@ -709,13 +707,13 @@ __device__ __forceinline__ void stockholm(const dmesh& m, int j, int k, int l, r
   const int l2 = j + k * m.sy;
   if (R.ramp > real(0.0)) {
     real r = rho[l], x = vx[l], y = vy[l];
-    stockholm_rxy<G>(m, j, k, dt, R, r, x, y, rho0[l2], vx0[l2], vy0[l2], d);
+    stockholm_rxy<G, D>(m, j, k, dt, R, r, x, y, rho0[l2], vx0[l2], vy0[l2], d);
     rho[l] = r;
     vx[l] = x;
     vy[l] = y;
   }
   if (DZ) {
-    if (R.rampi > real(0.0)) vz[l] = stockholm_z(dt, R, vz[l], vz0[l2]);
+    if (R.rampi > real(0.0)) vz[l] = stockholm_z<D>(dt, R, vz[l], vz0[l2]);
   }
 }
 

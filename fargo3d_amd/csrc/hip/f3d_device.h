@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #define F3D_NS f3d
 #define F3D_REAL double
 #include "f3d_device_body.h"

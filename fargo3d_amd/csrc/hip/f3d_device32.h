@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #define F3D_NS f3d32
 #define F3D_REAL float
 #include "f3d_device_body.h"

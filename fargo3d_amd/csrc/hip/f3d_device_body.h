@@ -52,23 +52,22 @@ __device__ __forceinline__ int lxm_of(int l, int i, int nx) { return (i > 0) ? l
 __device__ __forceinline__ int ixm_of(int i, int nx) { return i > 0 ? i - 1 : nx - 1; }
 __device__ __forceinline__ int ixp_of(int i, int nx) { return i < nx - 1 ? i + 1 : 0; }
 
-// Division by a divisor d > 0 that several quotients share: r = recip(d), then
-// per quotient q0 = RN(a r), rem = q0 d - a (exact: one FMA) and
-// q = RN(q0 - rem r) (a second FMA).  With r = RN(1/d) that is RN(a/d), the
-// correction step of Markstein's division (round to nearest, d finite and
-// nonzero, no overflow or underflow), checked with exact integer arithmetic for
-// every pair of significands of the binary formats of precision 4 to 16 (1.4e9
-// pairs; q0 alone is wrong in 27% of them) and against IEEE division on 6e8
-// random and near-midpoint binary64 pairs.  The remainder is formed as q0 d - a:
-// where it vanishes it is then +0, and q0 - (+0) r keeps q0, a zero of either
-// sign included, without the comparison and the two selects that the remainder
-// a - q0 d needs.  recip() refines the hardware's estimate of 1/d by two Newton
-// steps r += r (1 - d r), and q is then, operation for operation, what the
-// full division computes for operands that it does not have to scale
-// (magnitudes far from the ends of the exponent range, as every density, zone
-// size and volume here), without its scaling and special-case instructions: 5
-// for the reciprocal and 3 per quotient against 11 per division.  A quotient
-// by 0 is NaN.
+// Division by a divisor d that several quotients share: r = recip(d), then per
+// quotient q0 = RN(a r), rem = q0 d - a (one FMA) and q = RN(q0 - rem r) (a
+// second FMA).  recip() refines the hardware's estimate of 1/d by two Newton
+// steps r += r (1 - d r).  In FP64 these are, operation for operation, the
+// steps of the full division for operands that it does not have to scale, and
+// the quotient is RN(a/d); in FP32 the compiler's sequence is another one, and
+// the quotient agrees with RN(a/d) on every pair tried
+// (tests/division_binary32_check.c).  The remainder is formed as q0 d - a: where
+// it vanishes it is then +0, and q0 - (+0) r keeps q0, a zero of either sign
+// included, without a comparison and two selects.  5 instructions for the
+// reciprocal and 3 per quotient against 11 per full division.
+//   d and 1/d normal numbers, a = 0 or |a| >= 2^-969 (FP32 2^-102): RN(a/d).
+//   a smaller: the remainder loses bits, q is within an ulp of a/d.
+//   a or d infinite or NaN, d = 0, d so small that 1/d overflows (in FP32 any
+//   subnormal d), a quotient that overflows: NaN.
+//   d above 2^1022 (2^126): not covered.
 struct Recip {
   real d, r;
 };
@@ -84,8 +83,6 @@ __device__ __forceinline__ real rdiv(real a, const Recip& R) {
   const real q0 = a * R.r;
   return fma(-fma(q0, R.d, -a), R.r, q0);
 }
-// a / d for one quotient (the compiler shares recip() between equal divisors)
-__device__ __forceinline__ real qdiv(real a, real d) { return rdiv(a, recip(d)); }
 // the same in FP64 in every build (the CFL time step)
 struct RecipD {
   double d, r;
@@ -100,18 +97,58 @@ __device__ __forceinline__ double rdivd(double a, const RecipD& R) {
   const double q0 = a * R.r;
   return fma(-fma(q0, R.d, -a), R.r, q0);
 }
-__device__ __forceinline__ double qdivd(double a, double d) { return rdivd(a, recipd(d)); }
+
+// How a kernel forms the quotients that stand alone, a / d each.  q(): any
+// field over a mesh quantity; rho(): over something that holds a density, which
+// may vanish or be tiny; mesh(): one mesh quantity over another; q64(): FP64 in
+// every build.
+// Full: IEEE division for every operand.  For the entry points that take a
+// host's arrays as they are, one routine per launch, which are bound by their
+// launches.
+struct Full {
+  __device__ __forceinline__ static real q(real a, real d) { return a / d; }
+  __device__ __forceinline__ static real rho(real a, real d) { return a / d; }
+  __device__ __forceinline__ static real mesh(real a, real d) { return a / d; }
+  __device__ __forceinline__ static double q64(double a, double d) { return a / d; }
+};
+// Short: rdiv() with its range.  For kernels that test what comes out: a quotient
+// outside the range is NaN, and a sum or product keeps it (kd_src_fused2).
+struct Short {
+  __device__ __forceinline__ static real q(real a, real d) { return rdiv(a, recip(d)); }
+  __device__ __forceinline__ static real rho(real a, real d) { return rdiv(a, recip(d)); }
+  __device__ __forceinline__ static real mesh(real a, real d) { return rdiv(a, recip(d)); }
+  __device__ __forceinline__ static double q64(double a, double d) { return rdivd(a, recipd(d)); }
+};
+// Fixed: the short quotient with the full division's last step, which puts the
+// IEEE result in for a zero, infinite or NaN operand; densities by the full
+// division.  That step issues at a quarter of the rate of an FMA, so this is for
+// the kernels that wait for memory: 500x150x45 kf_src_a 115.7 us with Short and
+// 117.2 with Fixed, kf_src_b 147.8 and 148.6; kf_src_fused2 is bound by issue,
+// 104.8 us with Short and 115.5 with Fixed on 4096x1024.
+struct Fixed {
+  __device__ __forceinline__ static double fix(double v, double a, double d) {
+    return __builtin_amdgcn_div_fixup(v, d, a);
+  }
+  __device__ __forceinline__ static float fix(float v, float a, float d) {
+    return __builtin_amdgcn_div_fixupf(v, d, a);
+  }
+  __device__ __forceinline__ static real q(real a, real d) { return fix(Short::q(a, d), a, d); }
+  __device__ __forceinline__ static real rho(real a, real d) { return a / d; }
+  __device__ __forceinline__ static real mesh(real a, real d) { return Short::mesh(a, d); }
+  __device__ __forceinline__ static double q64(double a, double d) { return fix(Short::q64(a, d), a, d); }
+};
 
 // x * InvVol(i,j,k)  ->  (x*InvVj[j]) / (Syk[k]*Sxi[i])
+template <class D>
 __device__ __forceinline__ real mul_invvol(const dmesh& m, real x, int i, int j, int k) {
-  return qdiv(x * m.invvj[j], m.syk[k] * m.sxi[i]);
+  return D::q(x * m.invvj[j], m.syk[k] * m.sxi[i]);
 }
 // its divisor, for rdiv(): several quantities of one cell share it
 __device__ __forceinline__ Recip invvol_recip(const dmesh& m, int i, int k) { return recip(m.syk[k] * m.sxi[i]); }
 __device__ __forceinline__ real mul_invvol(const dmesh& m, real x, int j, const Recip& V) { return rdiv(x * m.invvj[j], V); }
 // x * Vol(i,j,k)  ->  ((x*Syk[k])*Sxi[i]) / InvVj[j]
 __device__ __forceinline__ real mul_vol(const dmesh& m, real x, int i, int j, int k) {
-  return qdiv((x * m.syk[k]) * m.sxi[i], m.invvj[j]);
+  return (x * m.syk[k]) * m.sxi[i] / m.invvj[j];
 }
 // the same with the ring's divisor InvVj[j] shared (rdiv())
 __device__ __forceinline__ real mul_vol(const dmesh& m, real x, int i, int k, const Recip& IV) {
@@ -119,7 +156,7 @@ __device__ __forceinline__ real mul_vol(const dmesh& m, real x, int i, int k, co
 }
 // Vol(i,j,k) standing alone  ->  (Syk[k]*Sxi[i]) / InvVj[j]
 __device__ __forceinline__ real vol(const dmesh& m, int i, int j, int k) {
-  return qdiv(m.syk[k] * m.sxi[i], m.invvj[j]);
+  return (m.syk[k] * m.sxi[i]) / m.invvj[j];
 }
 // x * SurfX(j,k)
 __device__ __forceinline__ real mul_surfx(const dmesh& m, real x, int j, int k) {
@@ -138,10 +175,10 @@ __device__ __forceinline__ real zone_size_x(const dmesh& m, int i, int j, int k)
   if (G == SPH) return (m.sxi[i] * m.ymed[j]) * m.sinzmed[k];
   return m.sxi[i] * m.ymed[j];
 }
-template <int G>
+template <int G, class D>
 __device__ __forceinline__ real inv_zone_size_xmed(const dmesh& m, int i, int j, int k) {
-  if (G == SPH) return qdiv(qdiv(m.invdiffxmed[i], m.ymed[j]), m.sinzmed[k]);
-  return qdiv(m.invdiffxmed[i], m.ymed[j]);
+  if (G == SPH) return D::mesh(D::mesh(m.invdiffxmed[i], m.ymed[j]), m.sinzmed[k]);
+  return D::mesh(m.invdiffxmed[i], m.ymed[j]);
 }
 __device__ __forceinline__ real zone_size_y(const dmesh& m, int j) { return m.ymin[j + 1] - m.ymin[j]; }
 template <int G>
@@ -201,10 +238,12 @@ __device__ inline void cfl_min_publish(const double* ringmin, int n, unsigned lo
 // quotient is formed in every lane and the extremum case selected after it
 // (the same value in both cases): a branch around the division would split
 // the sweeps' loops into blocks that the next row's loads cannot be moved
-// across.
+// across.  Short's range holds: p > 0 bounds the divisor away from 0.
+template <class D = Short>
 __device__ __forceinline__ real vanleer_slope(real dqm, real dqp) {
   const real p = dqp * dqm;
-  const real s = qdiv(p + p, dqm + dqp);  // 2 dqp dqm / (dqm + dqp); p > 0 bounds the divisor away from 0
+  // p + p is 2 dqp dqm but where one of them overflows or is subnormal
+  const real s = D::q(std::is_same<D, Full>::value ? real(2.) * dqp * dqm : p + p, dqm + dqp);
   return (p <= real(0.0)) ? real(0.0) : s;
 }
 // upwind interface value (src/vanleer_y_b.c:60-65)

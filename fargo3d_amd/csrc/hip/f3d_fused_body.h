@@ -484,7 +484,7 @@ __device__ __forceinline__ void kd_src_a(const dim3 bid, const dmesh& m, const r
   const cell::GL VZ = cell::gl(DZ ? vz : vy, m, l, i);
   const cell::GL R = cell::gl(rho, m, l, i);
   if (visc) {
-    cell::Taus t = cell::visctensor<G, DZ>(m, i, j, k, R, cell::gl(energy, m, l, i), VX, VY, VZ, vp);
+    cell::Taus t = cell::visctensor<G, DZ, Fixed>(m, i, j, k, R, cell::gl(energy, m, l, i), VX, VY, VZ, vp);
     txx[l] = t.xx;
     tyy[l] = t.yy;
     tyx[l] = t.yx;
@@ -531,13 +531,13 @@ __device__ __forceinline__ void kd_src_b(const dim3 bid, const dmesh& m, real dt
   const auto VX = vxc<G>(vx, m, l, i, j, k, domega);
   const cell::GL VY = cell::gl(vy, m, l, i);
   const cell::GL VZ = cell::gl(DZ ? vz : vy, m, l, i);
-  real ax = cell::substep1_x<G>(m, i, j, k, dt, R, P, PT, VX, dust, potential);
-  real ay = cell::substep1_y<G, DZ>(m, i, j, k, dt, R, P, PT, VX, VY, VZ, dust, potential, omegaframe);
-  real az = DZ ? cell::substep1_z<G>(m, i, j, k, dt, R, P, PT, VX, VZ, dust, potential, omegaframe) : real(0.0);
+  real ax = cell::substep1_x<G, Fixed>(m, i, j, k, dt, R, P, PT, VX, dust, potential);
+  real ay = cell::substep1_y<G, DZ, Fixed>(m, i, j, k, dt, R, P, PT, VX, VY, VZ, dust, potential, omegaframe);
+  real az = DZ ? cell::substep1_z<G, Fixed>(m, i, j, k, dt, R, P, PT, VX, VZ, dust, potential, omegaframe) : real(0.0);
   if (visc) {
     const cell::GL TZZ = cell::gl(DZ ? tzz : txx, m, l, i), TXZ = cell::gl(DZ ? txz : txx, m, l, i),
                    TZY = cell::gl(DZ ? tzy : txx, m, l, i);
-    cell::addviscosity<G, DZ>(m, i, j, k, dt, R, cell::gl(txx, m, l, i), cell::gl(tyy, m, l, i), TZZ, TXZ,
+    cell::addviscosity<G, DZ, Fixed>(m, i, j, k, dt, R, cell::gl(txx, m, l, i), cell::gl(tyy, m, l, i), TZZ, TXZ,
                               cell::gl(tyx, m, l, i), TZY, ax, ay, az, ax, ay, az);
   }
   real e = iso ? real(0.0) : energy[l];
@@ -545,7 +545,7 @@ __device__ __forceinline__ void kd_src_b(const dim3 bid, const dmesh& m, real dt
   const ArtQ<cell::GL, decltype(VX), 0> QX{R, VX};
   const ArtQ<cell::GL, cell::GL, 1> QY{R, VY};
   const ArtQ<cell::GL, cell::GL, 2> QZ{R, VZ};
-  cell::substep2_b<G, DZ>(m, i, j, k, dt, R, VX, VY, VZ, QX, QY, QZ, !iso, ax, ay, az, e, ax, ay, az, e);
+  cell::substep2_b<G, DZ, Fixed>(m, i, j, k, dt, R, VX, VY, VZ, QX, QY, QZ, !iso, ax, ay, az, e, ax, ay, az, e);
   vxt[l] = ax;
   vyt[l] = ay;
   if (DZ) vzt[l] = az;
@@ -595,51 +595,79 @@ __device__ __forceinline__ void kd_src_fused2(const dim3 b, const dmesh& m, real
   const int r1 = min(r0 + rows_per, jend);
   // visctensor (src/visctensor_cyl.c:140-186, src/visctensor_sph.c:126-206)
   // at (i, row): the same loaders as kd_src_a
-  auto stress = [&](int row) -> cell::Taus {
+  auto stress = [&](auto how, int row) -> cell::Taus {
     const int l = i + row * m.pitch;
     const auto VX = vx_stress<G>(vx, m, l, i, row, 0, domega);
     const cell::GL VY = cell::gl(vy, m, l, i);
-    return cell::visctensor<G, 0>(m, i, row, 0, cell::gl(rho, m, l, i), cell::gl(energy, m, l, i), VX, VY, VY, vp);
+    return cell::visctensor<G, 0, decltype(how)>(m, i, row, 0, cell::gl(rho, m, l, i), cell::gl(energy, m, l, i), VX,
+                                                 VY, VY, vp);
   };
-  cell::Taus Tm = stress(r0 - 1), T0 = stress(r0);
+  // kd_src_b at (i, j) with the stresses of its own column and of its x neighbours
+  auto update = [&](auto how, int j, const cell::Taus& Tm, const cell::Taus& T0, const cell::Taus& Tp, real txx_xm,
+                    real tyx_xp, real& ax, real& ay, real& e) {
+    using D = decltype(how);
+    const int l = i + j * m.pitch;
+    const cell::GL R = cell::gl(rho, m, l, i);
+    const PresLoader P{R, cell::gl(energy, m, l, i), gm1, iso};
+    const cell::GLT<double> PT = cell::gld(pot, m, l, i);
+    const auto VX = vxc<G>(vx, m, l, i, j, 0, domega);
+    const cell::GL VY = cell::gl(vy, m, l, i);
+    ax = cell::substep1_x<G, D>(m, i, j, 0, dt, R, P, PT, VX, 0, 1);
+    ay = cell::substep1_y<G, 0, D>(m, i, j, 0, dt, R, P, PT, VX, VY, VY, 0, 1, omegaframe);
+    real az = real(0.0);
+    const StressAt TXX{T0.xx, txx_xm, real(0.0), Tm.xx, real(0.0)};
+    const StressAt TYY{T0.yy, real(0.0), real(0.0), Tm.yy, real(0.0)};
+    const StressAt TYX{T0.yx, real(0.0), tyx_xp, real(0.0), Tp.yx};
+    cell::addviscosity<G, 0, D>(m, i, j, 0, dt, R, TXX, TYY, TXX, TXX, TYX, TXX, ax, ay, az, ax, ay, az);
+    e = iso ? real(0.0) : energy[l];
+    const ArtQ<cell::GL, decltype(VX), 0> QX{R, VX};
+    const ArtQ<cell::GL, cell::GL, 1> QY{R, VY};
+    cell::substep2_b<G, 0, D>(m, i, j, 0, dt, R, VX, VY, VY, QX, QY, QY, !iso, ax, ay, az, e, ax, ay, az, e);
+  };
+  auto store = [&](int j, real ax, real ay, real e) {
+    const int l = i + j * m.pitch;
+    vxt[l] = ax;
+    vyt[l] = ay;
+    if (!iso) e2[l] = e;
+  };
+  unsigned again = 0;  // bit j - r0 (rows_per <= 32): the cell of row j came out NaN
+  cell::Taus Tm = stress(Short{}, r0 - 1), T0 = stress(Short{}, r0);
   for (int j = r0; j < r1; j++) {
-    const cell::Taus Tp = stress(j + 1);
+    const cell::Taus Tp = stress(Short{}, j + 1);
     // the x neighbours' stresses (every lane takes part in the rotations)
     const real txx_xm = from_left(T0.xx), tyx_xp = from_right(T0.yx);
     if (upd) {
-      // kd_src_b at (i, j)
-      const int l = i + j * m.pitch;
-      const cell::GL R = cell::gl(rho, m, l, i);
-      const PresLoader P{R, cell::gl(energy, m, l, i), gm1, iso};
-      const cell::GLT<double> PT = cell::gld(pot, m, l, i);
-      const auto VX = vxc<G>(vx, m, l, i, j, 0, domega);
-      const cell::GL VY = cell::gl(vy, m, l, i);
-      real ax = cell::substep1_x<G>(m, i, j, 0, dt, R, P, PT, VX, 0, 1);
-      real ay = cell::substep1_y<G, 0>(m, i, j, 0, dt, R, P, PT, VX, VY, VY, 0, 1, omegaframe);
-      real az = real(0.0);
-      const StressAt TXX{T0.xx, txx_xm, real(0.0), Tm.xx, real(0.0)};
-      const StressAt TYY{T0.yy, real(0.0), real(0.0), Tm.yy, real(0.0)};
-      const StressAt TYX{T0.yx, real(0.0), tyx_xp, real(0.0), Tp.yx};
-      cell::addviscosity<G, 0>(m, i, j, 0, dt, R, TXX, TYY, TXX, TXX, TYX, TXX, ax, ay, az, ax, ay, az);
-      real e = iso ? real(0.0) : energy[l];
-      const ArtQ<cell::GL, decltype(VX), 0> QX{R, VX};
-      const ArtQ<cell::GL, cell::GL, 1> QY{R, VY};
-      cell::substep2_b<G, 0>(m, i, j, 0, dt, R, VX, VY, VY, QX, QY, QY, !iso, ax, ay, az, e, ax, ay, az, e);
-      vxt[l] = ax;
-      vyt[l] = ay;
-      if (!iso) e2[l] = e;
+      real ax, ay, e;
+      update(Short{}, j, Tm, T0, Tp, txx_xm, tyx_xp, ax, ay, e);
+      if (ax != ax || ay != ay || e != e) again |= 1u << (j - r0);
+      store(j, ax, ay, e);
     }
     Tm = T0;
     T0 = Tp;
   }
+  // A quotient outside the short division's range made these cells NaN: they
+  // are formed again, with the full division, from the same inputs.  (After the
+  // loop, where nothing of it is live: inside it this took 28 registers more and
+  // a wave per SIMD.)
+  if (__builtin_expect(__any(again != 0), 0)) {
+    for (int j = r0; j < r1; j++) {
+      const cell::Taus Um = stress(Full{}, j - 1), U0 = stress(Full{}, j), Up = stress(Full{}, j + 1);
+      const real txx_xm = from_left(U0.xx), tyx_xp = from_right(U0.yx);
+      if ((again >> (j - r0)) & 1) {
+        real ax, ay, e;
+        update(Full{}, j, Um, U0, Up, txx_xm, tyx_xp, ax, ay, e);
+        store(j, ax, ay, e);
+      }
+    }
+  }
 }
 template <int G, int MODE, int VM>
-__global__ void __launch_bounds__(64) kf_src_fused2(dmesh m, real dt, const real* __restrict__ rho,
-                                                    const real* __restrict__ energy, const real* __restrict__ vx,
-                                                    const real* __restrict__ vy, const double* __restrict__ pot,
-                                                    real* __restrict__ vxt, real* __restrict__ vyt,
-                                                    real* __restrict__ e2, cell::ViscPar vp, real gm1,
-                                                    double omegaframe, real domega, int rows_per, int jend) {
+__global__ void __launch_bounds__(64, 4) kf_src_fused2(dmesh m, real dt, const real* __restrict__ rho,
+                                                       const real* __restrict__ energy, const real* __restrict__ vx,
+                                                       const real* __restrict__ vy, const double* __restrict__ pot,
+                                                       real* __restrict__ vxt, real* __restrict__ vyt,
+                                                       real* __restrict__ e2, cell::ViscPar vp, real gm1,
+                                                       double omegaframe, real domega, int rows_per, int jend) {
   kd_src_fused2<G, MODE, VM>(xcd_bid(), m, dt, rho, energy, vx, vy, pot, vxt, vyt, e2, vp, gm1, omegaframe, domega,
                              rows_per, jend);
 }
@@ -683,7 +711,7 @@ __global__ void __launch_bounds__(WG) kf_substep3(dmesh m, real dt, const real* 
   const int j = m.nghy + (int)blockIdx.y;
   const int k = DZ ? m.nghz + (int)blockIdx.z : 0;
   const int l = i + j * m.pitch + k * m.stride;
-  energy[l] = cell::substep3<DZ>(m, i, j, k, dt, e2[l], cell::gl(vxt, m, l, i), cell::gl(vyt, m, l, i),
+  energy[l] = cell::substep3<DZ, Fixed>(m, i, j, k, dt, e2[l], cell::gl(vxt, m, l, i), cell::gl(vyt, m, l, i),
                                  cell::gl(DZ ? vzt : vyt, m, l, i), gamma);
 }
 
@@ -1142,17 +1170,18 @@ __device__ __forceinline__ void xsweep(const dmesh& m, int ring, int tile, int g
     } else {
       vmed = T.vxmed[l2];
     }
+    // (Short: where vmed is not finite, v and w are not either)
 #pragma unroll
     for (int s = 0; s < CPT; s++) {
       const double zs = zone_size_x64<G>(m, ix[s], j, k);
-      const double ntilde = qdivd(vmed * dt64, zs);
+      const double ntilde = Short::q64(vmed * dt64, zs);
       const double nround = floor(ntilde + 0.5);
       if constexpr (cell::kFix64) v[s] = (real)(vt[s] - (vmed - vb));
       else v[s] = (real)(vt[s] - vmed);
-      w[s] = (real)qdivd((ntilde - nround) * zs, dt64);
+      w[s] = (real)Short::q64((ntilde - nround) * zs, dt64);
     }
     // the shift of the ring is that of its cell 0
-    ns = (int)floor(qdivd(vmed * dt64, zone_size_x64<G>(m, 0, j, k)) + 0.5);
+    ns = (int)floor(Short::q64(vmed * dt64, zone_size_x64<G>(m, 0, j, k)) + 0.5);
     if (lane == 0 && tile == 0 && grp == 0) {
       T.nshift[l2] = ns;
       if (RING) T.vxmed[l2] = vmed;
@@ -1331,11 +1360,15 @@ __device__ __forceinline__ void xsweep(const dmesh& m, int ring, int tile, int g
       real rl[CPT], ml[CPT];
       W::left(rho2, rl);
       W::left(mp, ml);
+      const Recip IV = recip(m.invvj[j]);
 #pragma unroll
       for (int s = 0; s < CPT; s++)
         if (mine[s]) {
           T.rho_out[base + to[s]] = rho2[s];
-          T.vx_out[base + to[s]] = cell::newvel_x<G>(m, to[s], j, k, rho2[s], rl[s], st[s], ml[s], omegaframe);
+          const int il = ixm_of(to[s], nx);
+          T.vx_out[base + to[s]] = cell::newvel_x<G, Fixed>(
+              m, j, k, mul_vol(m, rho2[s], to[s], k, IV), mul_vol(m, rl[s], il, k, IV),
+              mul_vol(m, st[s], to[s], k, IV), mul_vol(m, ml[s], il, k, IV), omegaframe);
         }
     } else {
       real* __restrict__ o = T.out[c];
@@ -1436,12 +1469,15 @@ __device__ __forceinline__ void kd_finish(const dim3 bid, const dmesh& m, real d
   // the faces j = nghy and k = nghz lie on the mesh boundary; the ghost fill
   // sets them to zero, so they are not computed here (the damping, which runs
   // on the values in registers, reads the stored ones there)
-  real y = (j > m.nghy) ? cell::newvel_y(m, i, j, k, r, rho_x[l - m.pitch], mmy[l], mpy[l - m.pitch]) : real(0.0);
-  real z = real(0.0);
+  const Recip IV = recip(m.invvj[j]), IVm = recip(m.invvj[j - 1]);
+  real y = real(0.0), z = real(0.0);
+  if (j > m.nghy)
+    y = cell::newvel_yz<Fixed>(mul_vol(m, r, i, k, IV), mul_vol(m, rho_x[l - m.pitch], i, k, IVm),
+                               mul_vol(m, mmy[l], i, k, IV), mul_vol(m, mpy[l - m.pitch], i, k, IVm));
   if (DZ && k > m.nghz) {
-    z = qdiv(mul_vol(m, mmz[l], i, j, k) + mul_vol(m, mpz[l - m.stride], i, j, k - 1),
-             mul_vol(m, r, i, j, k) + mul_vol(m, rho_x[l - m.stride], i, j, k - 1));
-    if (G == SPH) z = qdiv(z, m.ymed[j]);
+    z = cell::newvel_yz<Fixed>(mul_vol(m, r, i, k, IV), mul_vol(m, rho_x[l - m.stride], i, k - 1, IV),
+                               mul_vol(m, mmz[l], i, k, IV), mul_vol(m, mpz[l - m.stride], i, k - 1, IV));
+    if (G == SPH) z = Fixed::q(z, m.ymed[j]);
   }
   if (stockholm) {
     // StockholmBoundary (src/stockholm.c:129-184) after NewVelocity_y/z; the
@@ -1451,13 +1487,13 @@ __device__ __forceinline__ void kd_finish(const dim3 bid, const dmesh& m, real d
     if (R.ramp > real(0.0)) {
       if (j == m.nghy) y = vy[l];
       real x = vx[l];
-      cell::stockholm_rxy<G>(m, j, k, dt, R, r, x, y, rho0[l2], vx0[l2], vy0[l2], dp);
+      cell::stockholm_rxy<G, Fixed>(m, j, k, dt, R, r, x, y, rho0[l2], vx0[l2], vy0[l2], dp);
       vx[l] = x;
       if (j == m.nghy) vy[l] = y;
     }
     if (DZ && R.rampi > real(0.0)) {
       if (k == m.nghz) z = vz[l];
-      z = cell::stockholm_z(dt, R, z, vz0[l2]);
+      z = cell::stockholm_z<Fixed>(dt, R, z, vz0[l2]);
       if (k == m.nghz) vz[l] = z;
     }
   }
@@ -1686,7 +1722,7 @@ __device__ __forceinline__ void drag_solve(const FluidSet& F, real* const* v, in
       const dreal rho_p = dreal(0.5) * ((dreal)F.rho[p][l] + (dreal)F.rho[p][idm]);
       if (p != o) {
         const dreal rho_o = dreal(0.5) * ((dreal)F.rho[o][l] + (dreal)F.rho[o][idm]);
-        if (p > o) m[p + o * NF] = qdivd(-(dreal)dt * (dreal)omega * (dreal)F.alpha[p + o * NF] * rho_p, rho_o);
+        if (p > o) m[p + o * NF] = Fixed::q64(-(dreal)dt * (dreal)omega * (dreal)F.alpha[p + o * NF] * rho_p, rho_o);
         else m[p + o * NF] = -(dreal)dt * (dreal)omega * (dreal)F.alpha[p + o * NF];
       } else {
         dreal sum = dreal(0.0);
@@ -1694,7 +1730,7 @@ __device__ __forceinline__ void drag_solve(const FluidSet& F, real* const* v, in
         for (int q = 0; q < NF; q++) {
           if (q != p) {
             const dreal rho_q = dreal(0.5) * ((dreal)F.rho[q][l] + (dreal)F.rho[q][idm]);
-            if (q > p) sum += qdivd((dreal)F.alpha[q + p * NF] * rho_q, rho_p);
+            if (q > p) sum += Fixed::q64((dreal)F.alpha[q + p * NF] * rho_q, rho_p);
             else sum += (dreal)F.alpha[q + p * NF];
           }
         }
@@ -1732,7 +1768,7 @@ __device__ __forceinline__ void drag_solve(const FluidSet& F, real* const* v, in
     }
 #pragma unroll
     for (int ir2 = ir + 1; ir2 < NF; ir2++) {
-      const dreal factor = qdivd(m[ir + ir2 * NF], m[ir + ir * NF]);
+      const dreal factor = Fixed::q64(m[ir + ir2 * NF], m[ir + ir * NF]);
 #pragma unroll
       for (int ic = 0; ic < NF; ic++) m[ic + ir2 * NF] -= m[ic + ir * NF] * factor;
       b[ir2] -= b[ir] * factor;
@@ -1742,7 +1778,7 @@ __device__ __forceinline__ void drag_solve(const FluidSet& F, real* const* v, in
   for (int ir = NF - 1; ir > -1; ir--) {
 #pragma unroll
     for (int ic = NF - 1; ic > ir; ic--) b[ir] -= m[ic + ir * NF] * b[ic];
-    b[ir] = qdivd(b[ir], m[ir + ir * NF]);
+    b[ir] = Fixed::q64(b[ir], m[ir + ir * NF]);
   }
 #pragma unroll
   for (int o = 0; o < NF; o++) v[o][l] = (real)b[o];
@@ -1803,23 +1839,23 @@ __device__ __forceinline__ void ddiff_core_cell(const dmesh& m, real dt, int bx,
   const int ll = i + j * m.pitch;
   const int llxm = lxm_of(ll, i, m.nx), llxp = lxp_of(ll, i, m.nx), llyp = ll + m.pitch, llym = ll - m.pitch;
   real update = real(0.0);
-  const real c = qdiv(rhod[ll], rhod[ll] + rhog[ll]);
+  const real c = Fixed::rho(rhod[ll], rhod[ll] + rhog[ll]);
   const real dxmin = m.xmin[i + 1] - m.xmin[i];
-  const real dxmedp = qdiv(real(1.0), m.invdiffxmed[ixp_of(i, m.nx)]);
-  const real dxmedm = qdiv(real(1.0), m.invdiffxmed[i]);
+  const real dxmedp = Fixed::mesh(real(1.0), m.invdiffxmed[ixp_of(i, m.nx)]);
+  const real dxmedm = Fixed::mesh(real(1.0), m.invdiffxmed[i]);
   const real d1 = real(0.25) * (rhod[ll] + rhog[ll] + rhod[llxp] + rhog[llxp]) * (yczc[llxp] + yczc[ll]);
   const real d2 = real(0.25) * (rhod[ll] + rhog[ll] + rhod[llxm] + rhog[llxm]) * (yczc[llxm] + yczc[ll]);
-  const real cxp = qdiv(rhod[llxp], rhod[llxp] + rhog[llxp]);
-  const real cxm = qdiv(rhod[llxm], rhod[llxm] + rhog[llxm]);
+  const real cxp = Fixed::rho(rhod[llxp], rhod[llxp] + rhog[llxp]);
+  const real cxm = Fixed::rho(rhod[llxm], rhod[llxm] + rhog[llxm]);
   const real ym = m.ymed[j];
-  update += qdiv(qdiv(qdiv(real(1.0), ym), ym), dxmin) * (qdiv(d1 * (cxp - c), dxmedp) - qdiv(d2 * (c - cxm), dxmedm));
+  update += Fixed::mesh(Fixed::mesh(Fixed::mesh(real(1.0), ym), ym), dxmin) * (Fixed::q(d1 * (cxp - c), dxmedp) - Fixed::q(d2 * (c - cxm), dxmedm));
   const real d3 = real(0.5) * (rhod[ll] + rhog[ll] + rhod[llyp] + rhog[llyp]) * yfzc[llyp];
   const real d4 = real(0.5) * (rhod[ll] + rhog[ll] + rhod[llym] + rhog[llym]) * yfzc[ll];
-  const real cyp = qdiv(rhod[llyp], rhod[llyp] + rhog[llyp]);
-  const real cym = qdiv(rhod[llym], rhod[llym] + rhog[llym]);
-  update += qdiv(qdiv(real(1.0), ym), m.ymin[j + 1] - m.ymin[j]) *
-            (qdiv(m.ymin[j + 1] * d3 * (cyp - c), m.ymed[j + 1] - ym) -
-             qdiv(m.ymin[j] * d4 * (c - cym), ym - m.ymed[j - 1]));
+  const real cyp = Fixed::rho(rhod[llyp], rhod[llyp] + rhog[llyp]);
+  const real cym = Fixed::rho(rhod[llym], rhod[llym] + rhog[llym]);
+  update += Fixed::mesh(Fixed::mesh(real(1.0), ym), m.ymin[j + 1] - m.ymin[j]) *
+            (Fixed::q(m.ymin[j + 1] * d3 * (cyp - c), m.ymed[j + 1] - ym) -
+             Fixed::q(m.ymin[j] * d4 * (c - cym), ym - m.ymed[j - 1]));
   temp[ll] = rhod[ll] + dt * update;
 }
 

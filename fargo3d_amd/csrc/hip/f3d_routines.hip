@@ -100,7 +100,7 @@ template <int G, int DZ>
 __global__ void k_substep1_x(dmesh m, Range r, double dt, const double* p, const double* rho,
                              const double* pot, const double* vx, double* vx_temp, int dust, int potential) {
   CELL_INDEX;
-  vx_temp[l] = cell::substep1_x<G>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(p, m, l, i),
+  vx_temp[l] = cell::substep1_x<G, Full>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(p, m, l, i),
                                    cell::gl(pot, m, l, i), cell::gl(vx, m, l, i), dust, potential);
 }
 
@@ -109,7 +109,7 @@ __global__ void k_substep1_y(dmesh m, Range r, double dt, const double* p, const
                              const double* pot, const double* vx, const double* vy, const double* vz,
                              double* vy_temp, int dust, int potential, double omegaframe) {
   CELL_INDEX;
-  vy_temp[l] = cell::substep1_y<G, DZ>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(p, m, l, i),
+  vy_temp[l] = cell::substep1_y<G, DZ, Full>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(p, m, l, i),
                                        cell::gl(pot, m, l, i), cell::gl(vx, m, l, i), cell::gl(vy, m, l, i),
                                        cell::gl(DZ ? vz : vy, m, l, i), dust, potential, omegaframe);
 }
@@ -119,7 +119,7 @@ __global__ void k_substep1_z(dmesh m, Range r, double dt, const double* p, const
                              const double* pot, const double* vx, const double* vz, double* vz_temp,
                              int dust, int potential, double omegaframe) {
   CELL_INDEX;
-  vz_temp[l] = cell::substep1_z<G>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(p, m, l, i),
+  vz_temp[l] = cell::substep1_z<G, Full>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(p, m, l, i),
                                    cell::gl(pot, m, l, i), cell::gl(vx, m, l, i), cell::gl(vz, m, l, i), dust,
                                    potential, omegaframe);
 }
@@ -142,7 +142,7 @@ __global__ void k_substep2_b(dmesh m, Range r, double dt, const double* rho, con
   double ax, ay, az, de;
   const double* vzs = DZ ? vz : vy;
   const double* pzs = DZ ? pz : py;
-  cell::substep2_b<G, DZ>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(vx, m, l, i), cell::gl(vy, m, l, i),
+  cell::substep2_b<G, DZ, Full>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(vx, m, l, i), cell::gl(vy, m, l, i),
                           cell::gl(vzs, m, l, i), cell::gl(px, m, l, i), cell::gl(py, m, l, i),
                           cell::gl(pzs, m, l, i), adiabatic, vxt[l], vyt[l], DZ ? vzt[l] : 0.0,
                           adiabatic ? e[l] : 0.0, ax, ay, az, de);
@@ -157,7 +157,7 @@ __global__ void k_substep3(dmesh m, Range r, double dt, double* e, const double*
                            const double* vz, double gamma) {
   CELL_INDEX;
   const double* vzs = DZ ? vz : vy;
-  e[l] = cell::substep3<DZ>(m, i, j, k, dt, e[l], cell::gl(vx, m, l, i), cell::gl(vy, m, l, i),
+  e[l] = cell::substep3<DZ, Full>(m, i, j, k, dt, e[l], cell::gl(vx, m, l, i), cell::gl(vy, m, l, i),
                             cell::gl(vzs, m, l, i), gamma);
 }
 
@@ -168,7 +168,7 @@ __global__ void k_visctensor(dmesh m, Range r, const double* rho, const double* 
   CELL_INDEX;
   const double* vzs = DZ ? vz : vy;
   const double* es = energy ? energy : rho;
-  cell::Taus t = cell::visctensor<G, DZ>(m, i, j, k, cell::gl(rho, m, l, i), cell::gl(es, m, l, i),
+  cell::Taus t = cell::visctensor<G, DZ, Full>(m, i, j, k, cell::gl(rho, m, l, i), cell::gl(es, m, l, i),
                                          cell::gl(vx, m, l, i), cell::gl(vy, m, l, i), cell::gl(vzs, m, l, i), vp);
   txx[l] = t.xx;
   tyy[l] = t.yy;
@@ -189,7 +189,7 @@ __global__ void k_addviscosity(dmesh m, Range r, double dt, const double* rho, d
   const double* tzzs = DZ ? tzz : txx;
   const double* txzs = DZ ? txz : txx;
   const double* tzys = DZ ? tzy : txx;
-  cell::addviscosity<G, DZ>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(txx, m, l, i), cell::gl(tyy, m, l, i),
+  cell::addviscosity<G, DZ, Full>(m, i, j, k, dt, cell::gl(rho, m, l, i), cell::gl(txx, m, l, i), cell::gl(tyy, m, l, i),
                             cell::gl(tzzs, m, l, i), cell::gl(txzs, m, l, i), cell::gl(tyx, m, l, i),
                             cell::gl(tzys, m, l, i), vx[l], vy[l], DZ ? vz[l] : 0.0, ax, ay, az);
   vx[l] = ax;
@@ -303,7 +303,7 @@ __global__ void k_vly_a(dmesh m, Range r, const double* q, double* slope) {
   CELL_INDEX;
   double dqm = (q[l] - q[l - m.pitch]) / zone_size_y(m, j);
   double dqp = (q[l + m.pitch] - q[l]) / zone_size_y(m, j + 1);
-  slope[l] = vanleer_slope(dqm, dqp);
+  slope[l] = vanleer_slope<Full>(dqm, dqp);
 }
 
 template <int G, int DZ>
@@ -319,7 +319,7 @@ __global__ void k_vlz_a(dmesh m, Range r, const double* q, double* slope) {
   CELL_INDEX;
   double dqm = (q[l] - q[l - m.stride]) / zone_size_z<G>(m, j, k);
   double dqp = (q[l + m.stride] - q[l]) / zone_size_z<G>(m, j, k + 1);
-  slope[l] = vanleer_slope(dqm, dqp);
+  slope[l] = vanleer_slope<Full>(dqm, dqp);
 }
 
 template <int G, int DZ>
@@ -337,7 +337,7 @@ __global__ void k_vlx_a(dmesh m, Range r, const double* q, double* slope) {
   const int lxm = lxm_of(l, i, m.nx), lxp = lxp_of(l, i, m.nx);
   double dqm = (q[l] - q[lxm]) / zone_size_x<G>(m, i, j, k);
   double dqp = (q[lxp] - q[l]) / zone_size_x<G>(m, ixp_of(i, m.nx), j, k);
-  slope[l] = vanleer_slope(dqm, dqp);
+  slope[l] = vanleer_slope<Full>(dqm, dqp);
 }
 
 template <int G, int DZ>
@@ -431,14 +431,17 @@ __global__ void k_newvel_x(dmesh m, Range r, const double* rho, const double* mm
                            double omegaframe) {
   CELL_INDEX;
   const int lxm = lxm_of(l, i, m.nx);
-  vx[l] = cell::newvel_x<G>(m, i, j, k, rho[l], rho[lxm], mmx[l], mpx[lxm], omegaframe);
+  const int im = ixm_of(i, m.nx);
+  vx[l] = cell::newvel_x<G, Full>(m, j, k, mul_vol(m, rho[l], i, j, k), mul_vol(m, rho[lxm], im, j, k),
+                                  mul_vol(m, mmx[l], i, j, k), mul_vol(m, mpx[lxm], im, j, k), omegaframe);
 }
 
 template <int G, int DZ>
 __global__ void k_newvel_y(dmesh m, Range r, const double* rho, const double* mmy, const double* mpy, double* vy) {
   CELL_INDEX;
   const int lym = l - m.pitch;
-  vy[l] = cell::newvel_y(m, i, j, k, rho[l], rho[lym], mmy[l], mpy[lym]);
+  vy[l] = cell::newvel_yz<Full>(mul_vol(m, rho[l], i, j, k), mul_vol(m, rho[lym], i, j - 1, k),
+                                mul_vol(m, mmy[l], i, j, k), mul_vol(m, mpy[lym], i, j - 1, k));
 }
 
 template <int G, int DZ>
@@ -446,8 +449,8 @@ __global__ void k_newvel_z(dmesh m, Range r, const double* rho, const double* mm
   CELL_INDEX;
   const int lzm = l - m.stride;
   // "mmz*Vol(i,j,k)" associates as ((mmz*Syk)*Sxi)/InvVj (src/define.h:229)
-  double v = (mul_vol(m, mmz[l], i, j, k) + mul_vol(m, mpz[lzm], i, j, k - 1)) /
-      (mul_vol(m, rho[l], i, j, k) + mul_vol(m, rho[lzm], i, j, k - 1));
+  double v = cell::newvel_yz<Full>(mul_vol(m, rho[l], i, j, k), mul_vol(m, rho[lzm], i, j, k - 1),
+                                   mul_vol(m, mmz[l], i, j, k), mul_vol(m, mpz[lzm], i, j, k - 1));
   if (G == SPH) v /= m.ymed[j];
   vz[l] = v;
 }
@@ -485,7 +488,7 @@ __global__ void k_stockholm(dmesh m, Range r, double dt, double* rho, double* vx
                             const double* rho0, const double* vx0, const double* vy0, const double* vz0,
                             cell::DampPar dp) {
   CELL_INDEX;
-  cell::stockholm<G, DZ>(m, j, k, l, dt, rho, vx, vy, vz, rho0, vx0, vy0, vz0, dp);
+  cell::stockholm<G, DZ, Full>(m, j, k, l, dt, rho, vx, vy, vz, rho0, vx0, vy0, vz0, dp);
 }
 
 // cfl per cell (src/cfl.c:174-253) into DensStar
