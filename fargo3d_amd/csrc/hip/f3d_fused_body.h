@@ -2604,7 +2604,7 @@ int F3D_API(fused_set_vmedterms)(int terms) {
 }
 
 int F3D_API(fused_set_tiling)(int rows_y, int rows_z) {
-  if (rows_y < 0 || rows_z < 1) return -2;
+  if (rows_y < 0 || rows_z < 0) return -2;
   g_rows_y = rows_y;
   g_rows_z = rows_z;
   return 0;

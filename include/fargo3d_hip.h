@@ -277,9 +277,9 @@ int f3d_fused_transport(f3d_hip_ctx *ctx, double dt, int end_of_step);
  * from the handle's bound set): every fluid's sweeps, with the X sweep of all
  * fluids in one launch.  VxMed and Nshift end with the last fluid's values. */
 int f3d_fused_transport_fluids(f3d_hip_ctx *ctx, double dt, int nf, const f3d_fields *fl);
-/* Rows (Y sweep; 0: automatic, the default) and planes (Z sweep) one thread
- * updates, rounded down to 4, 2 or 1 (automatic until set); a tuning knob that
- * does not change results.  Returns -2 for rows_y below 0 or rows_z below 1. */
+/* Rows (Y sweep) and planes (Z sweep) one thread updates, rounded down to 4, 2
+ * or 1; 0, the default of both: automatic.  A tuning knob that does not change
+ * results.  Returns -2 for a number below 0. */
 int f3d_fused_set_tiling(int rows_y, int rows_z);
 /* X-sweep form: 0 (and 1) automatic (one-wave tiles of 64 to 256 cells by ring
  * length and count, one wave per ring on many rings of 256 cells), 2 tiles of

@@ -25,3 +25,14 @@ def _oracle_built():
     if (not os.path.exists(lib)) or any(os.path.getmtime(s) > os.path.getmtime(lib) for s in srcs):
         subprocess.run(["make", "-s", "-C", os.path.join(ROOT, "oracle")], check=True)
     yield
+
+
+@pytest.fixture(autouse=True)
+def _automatic_tiling():
+    """A test that sets the column sweeps' rows and planes per thread leaves the
+    next one the automatic choice."""
+    yield
+    fa = sys.modules.get("fargo3d_amd")
+    if fa is not None and fa._lib is not None:
+        fa._lib.f3d_fused_set_tiling(0, 0)
+        fa._lib.f3d32_fused_set_tiling(0, 0)
