@@ -780,7 +780,7 @@ int f3d_batch_tune(f3d_batch* B, int reps, int* best_rows_y, int* best_tile) {
   BCHECK(B, hipEventCreate(&e1));
   float best = 1e30f;
   int br = B->rows_y, bt = B->tile;
-  const int rows[] = {1, 2, 4, 8}, tiles[] = {64, 128, 256};
+  const int rows[] = {1, 2, 4}, tiles[] = {64, 128, 256};  // the forms there are (column_form, kb_sweep_x)
   for (int r : rows)
     for (int t : tiles) {
       if (f3d_batch_set_tiling(B, r, t)) return -1;

@@ -133,9 +133,9 @@ int f3d_batch_clock(f3d_batch *B, int i, double out[3]); /* dt, dtemp, PhysicalT
  * planet: x, y, z, vx, vy, vz, mass, count), at most maxn; *omegaframe gets
  * the frame rate.  Returns the planet count, or -1/-2 on error. */
 int f3d_batch_planets(f3d_batch *B, int i, double *out, int maxn, double *omegaframe);
-/* tuning knobs (rows per thread of the Y sweep; 64/128/256-cell X tiles) and
- * the autotuner that times every combination on the batch itself, restoring
- * the state afterwards */
+/* tuning knobs (rows per thread of the Y sweep, rounded down to 4, 2 or 1;
+ * 64/128/256-cell X tiles) and the autotuner that times every combination on
+ * the batch itself, restoring the state afterwards */
 int f3d_batch_set_tiling(f3d_batch *B, int rows_y, int tile);
 int f3d_batch_tune(f3d_batch *B, int reps, int *best_rows_y, int *best_tile);
 
