@@ -1,7 +1,6 @@
 // f3d_fused.hip -- the FP64 build of the fused step (entry points f3d_fused_*):
 // bit-for-bit the reference's arithmetic.  The kernels are in f3d_fused_body.h.
 #include <cstring>
-#include <algorithm>
 #include <type_traits>
 
 #include "f3d_internal.h"

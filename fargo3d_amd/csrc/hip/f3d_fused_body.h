@@ -1073,9 +1073,12 @@ __device__ __forceinline__ void kd_sweep_z(const dim3 b, const dmesh& m, real dt
 // from its load to its store before the next one is begun (its successor's load
 // in flight): only one quantity is live at a time, whatever their number, and
 // the loop over them is a loop.  Measured against all quantities held through
-// each pass in turn (256 registers, two waves per SIMD, spills in 3-D) or in LDS (13 barriers a ring):
-// 384x128 14.5 -> 8.5 us, 1250x437 31.6 -> 25.6, five fluids 1024x512 111 -> 96,
-// 3-D 500x150x45 275 -> 187, 256x96x32 45.6 -> 40; FP32 4096x1024 97 -> 94.
+// each pass in turn or in LDS (13 barriers a ring), the divisions' share in
+// both: 384x128 16.3 -> 6.5 us, 1250x437 34.8 -> 23.4, adiabatic 4096x1024 204.8 ->
+// 186.1 (FP32 116.0 -> 95.4), five fluids 1024x512 125.9 -> 92.2, 3-D 500x150x45 301
+// -> 186, 256x96x32 51.7 -> 39.2 (FP32 32.7 -> 27.0).  1, 2, 3 and 4 cells per lane
+// take 78, 135, 199 and 256 registers in FP64 (6, 3, 2 and 2 waves per SIMD, the last
+// with 28 bytes of scratch; a whole ring 255) and 42 to 54, 77, 112 and 147 in FP32.
 struct XFluid {
   const real* rho_in;
   const real* vxt;
@@ -1905,8 +1908,7 @@ __global__ void kf_ddiff_store(dmesh m, DdTab T, cell::BcPar bp0, cell::BcPar bp
     F3D_LAUNCH_CHECK(ctx);                                                                              \
   } while (0)
 
-// the same with a third template argument AD (1: adiabatic, the energy is transported)
-// KERN<G, DZ, T_>
+// the same with a third template argument: KERN<G, DZ, T_>
 #define FDISPATCH_T(ctx, KERN, T_, grid, block, shmem, ...)                                            \
   do {                                                                                                  \
     if (m.geom == SPH) {                                                                                \
@@ -1921,53 +1923,6 @@ __global__ void kf_ddiff_store(dmesh m, DdTab T, cell::BcPar bp0, cell::BcPar bp
         hipLaunchKernelGGL((KERN<CYL, 0, T_>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);      \
     }                                                                                                   \
     F3D_LAUNCH_CHECK(ctx);                                                                              \
-  } while (0)
-
-#define FDISPATCH_AD(ctx, KERN, grid, block, shmem, ...)                                                 \
-  do {                                                                                                    \
-    const bool ad_ = ((ctx)->ph.eos == 2);                                                                \
-    if (m.geom == SPH) {                                                                           \
-      if (m.dimz) {                                                                                \
-        if (ad_) hipLaunchKernelGGL((KERN<SPH, 1, 1>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__); \
-        else hipLaunchKernelGGL((KERN<SPH, 1, 0>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);     \
-      } else {                                                                                            \
-        if (ad_) hipLaunchKernelGGL((KERN<SPH, 0, 1>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__); \
-        else hipLaunchKernelGGL((KERN<SPH, 0, 0>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);     \
-      }                                                                                                   \
-    } else {                                                                                              \
-      if (m.dimz) {                                                                                \
-        if (ad_) hipLaunchKernelGGL((KERN<CYL, 1, 1>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__); \
-        else hipLaunchKernelGGL((KERN<CYL, 1, 0>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);     \
-      } else {                                                                                            \
-        if (ad_) hipLaunchKernelGGL((KERN<CYL, 0, 1>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__); \
-        else hipLaunchKernelGGL((KERN<CYL, 0, 0>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);     \
-      }                                                                                                   \
-    }                                                                                                     \
-    F3D_LAUNCH_CHECK(ctx);                                                                                \
-  } while (0)
-
-// FDISPATCH_AD with one more template argument T_ after the AD flag
-#define FDISPATCH_AD_T(ctx, KERN, T_, grid, block, shmem, ...)                                                    \
-  do {                                                                                                            \
-    const bool ad_ = ((ctx)->ph.eos == 2);                                                                        \
-    if (m.geom == SPH) {                                                                                          \
-      if (m.dimz) {                                                                                               \
-        if (ad_) hipLaunchKernelGGL((KERN<SPH, 1, 1, T_>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);   \
-        else hipLaunchKernelGGL((KERN<SPH, 1, 0, T_>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);       \
-      } else {                                                                                                    \
-        if (ad_) hipLaunchKernelGGL((KERN<SPH, 0, 1, T_>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);   \
-        else hipLaunchKernelGGL((KERN<SPH, 0, 0, T_>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);       \
-      }                                                                                                           \
-    } else {                                                                                                      \
-      if (m.dimz) {                                                                                               \
-        if (ad_) hipLaunchKernelGGL((KERN<CYL, 1, 1, T_>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);   \
-        else hipLaunchKernelGGL((KERN<CYL, 1, 0, T_>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);       \
-      } else {                                                                                                    \
-        if (ad_) hipLaunchKernelGGL((KERN<CYL, 0, 1, T_>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);   \
-        else hipLaunchKernelGGL((KERN<CYL, 0, 0, T_>), grid, block, shmem, (ctx)->stream, m, __VA_ARGS__);       \
-      }                                                                                                           \
-    }                                                                                                             \
-    F3D_LAUNCH_CHECK(ctx);                                                                                        \
   } while (0)
 
 static cell::CflPar cfl_par_f(const f3d_hip_ctx* ctx) {
@@ -2116,8 +2071,8 @@ static int g_srcfuse = -1;
 // end-of-step ghost fill inside kf_finish (3-D: the Z sides, 2-D: the Y
 // sides): -1 automatic (on), 0 off (launches of its own)
 static int g_zfill = -1;
-// 2-D: the X sweep's VxMed pass inside the Y sweep's launch where it would
-// run on the second stream: -1 automatic (on), 0 off
+// the X sweep's VxMed pass inside the Y (2-D) or Z (3-D) sweep's launch where it
+// would run on the second stream: -1 automatic (on), 0 off
 static int g_y2v = -1;
 
 // CFL form, bits: 1 ring minima to an array and a second pass (else one
@@ -2141,10 +2096,12 @@ static int cfl_mode(const dmesh& m, int nf) {
   return mode;
 }
 
-// Terms per lane of the one-wave ring sums (wave_ring_sum): 4, 8 or 16; -1
-// automatic: 16 from 2048 cells on (1024 rings of 4096 cells 11.6 us against
-// 13.6 with 8), else 8 (7150 rings of 500 cells 10.3 us against 13.7 with 16
-// and 11.9 with 4).
+// Terms per lane of the one-wave ring sums (wave_ring_sum) in a launch of their
+// own: 4, 8 or 16; -1 automatic: in FP64 16 from 2048 cells on (1024 rings of 4096
+// cells 11.6 us against 13.6 with 8), else 8 (7150 rings of 500 cells 10.3 us
+// against 13.7 with 16 and 11.9 with 4); in FP32, whose conversions lengthen a
+// chunk, 16 from 512 cells on.  The sums inside the Y or Z sweep's launch take 8
+// whatever the length.
 static int g_vmed_terms = -1;
 static int vmed_terms(int nx) {
   return g_vmed_terms > 0 ? g_vmed_terms : nx >= (cell::kFix64 ? 512 : 2048) ? 16 : 8;
@@ -2419,7 +2376,8 @@ static int side_stream(f3d_hip_ctx* ctx) {
 //     filled GPU (FP32: 1.34, 2.55, 4.06, 6.0), so the cheapest cover of a ring
 //     wins: rings of 4096 cells 4 per lane (adiabatic 4096x1024 in us: 196, 193,
 //     196, 189 for 1 .. 4 per lane), of 1024 cells 2 (five fluids 1024x512:
-//     102, 96, 102, 109), of 500 cells 3 (3-D 500x150x45: 187, 196, 186, 225);
+//     102, 96, 102, 109), of 500 cells 1 (3-D 500x150x45: 187, 196, 186, 225, where
+//     3 per lane would do as well; in FP32 3 per lane);
 //   - below 2048 waves of one cell per lane the launch is a chain of latencies:
 //     one cell per lane and two quantities per wave (384x128: 8.5 us, 9.3 with
 //     all quantities in a wave, 13.4 with four cells per lane; 96x48: 7.2, 8.4,

@@ -311,9 +311,10 @@ int f3d_fused_set_colsplit(int split);
  * workgroup.  -1 automatic.  The result is the same value in every form.
  * Returns -2 for other values. */
 int f3d_fused_set_cflmode(int mode);
-/* Terms per lane of the one-wave sequential ring sums of VxMed (the CFL's
- * and the X sweep's passes): 4, 8 or 16, -1 automatic (by ring length); the
- * sums are the same additions in the same order in every form.  Returns -2
+/* Terms per lane of the one-wave ring sums of VxMed (the CFL's and the X
+ * sweep's passes): 4, 8 or 16, -1 automatic (by ring length; 8 in the Y and Z
+ * sweeps' launches, which other values keep the pass out of); every form gives
+ * the sum of the additions in index order, bit for bit.  Returns -2
  * for other values. */
 int f3d_fused_set_vmedterms(int terms);
 /* 2-D sources of a viscous gas with a potential: one pass that computes the
@@ -327,10 +328,10 @@ int f3d_fused_set_srcfuse(int on);
  * launches of their own.  The same values in both.  Returns -2 for other
  * values. */
 int f3d_fused_set_zfill(int on);
-/* 2-D X sweep of long or many rings: the VxMed pass it reads runs in the Y
- * sweep's launch (its own workgroups beside the sweep's), -1 automatic (on),
- * or 0 on the second stream; the same sums in both.  Returns -2 for other
- * values. */
+/* The VxMed pass of an X sweep by tiles runs in the Y sweep's launch (2-D) or
+ * the Z sweep's (3-D), its own workgroups beside the sweep's, -1 automatic
+ * (on), or 0 on the second stream; the same sums in both.  Returns -2 for
+ * other values. */
 int f3d_fused_set_y2v(int on);
 /* Potential, the ghost fill and the damping references on the fused stages'
  * scratch-free kernels (the same formulas as f3d_Potential, f3d_boundaries,
